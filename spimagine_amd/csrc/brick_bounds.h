@@ -6,7 +6,14 @@
 // (uint16/uint8: the value itself; float: the IEEE bits mapped so that unsigned order is
 // numeric order), stored as (min key, ~max key) so that one unsigned min-reduction bounds a
 // box from both sides.  A brick holding a NaN gets the widest keys, which no skip test
-// accepts.  Built on upload (k_brick_bounds in spimrender.hip).
+// accepts.  Built on upload (volume_build.h).
+//
+// A finer grid of windows serves tests of single rays: entry (bx, by, bz) holds the minimum
+// and maximum over the padded voxels [4 bx, 4 bx + 8) x [4 by, ...) x [4 bz, ...), clipped
+// to the volume.  Windows overlap by half, so a run of samples whose corners span at most
+// 4 voxels past the run's least corner index along every axis lies in the one window that
+// this least corner's block (index >> 2) starts.  Float windows are stored widened (below),
+// a window holding a NaN as [-inf, +inf].  Both planes together take 1/32 of the volume.
 //
 // Why the bounds are exact for the renderer: every trilinear sample is a convex
 // combination of the 8 corners it reads, evaluated as three levels of fma lerps.  For
@@ -64,6 +71,13 @@ __device__ __forceinline__ float bound_margin(float lo, float hi) {
         return fmaxf(fabsf(lo), fabsf(hi)) * 0x1p-16f + 1e-30f;
     else
         return 0.0f;
+}
+
+// Windows of a padded volume (see the file comment): g* = entries per axis
+constexpr uint32_t kWinShift = 2;  // a window starts every 4 padded voxels
+constexpr uint32_t kWinStride = 1u << kWinShift;
+__host__ __device__ inline uint32_t win_entries(uint32_t padded) {
+    return (padded + kWinStride - 1u) / kWinStride;
 }
 
 // Per-brick keys of a padded volume: keys[(bz nby + by) nbx + bx] covers padded voxels

@@ -20,6 +20,7 @@
 #include <vector>
 
 #include "spr_internal.h"
+#include "volume_build.h"
 
 using namespace spr;
 
@@ -89,6 +90,11 @@ struct spr_ctx {
     } stage[8];
     int stage_next = 0;
     void* d_scratch = nullptr;  // the device's scratch (spr_render_batch_noalloc)
+    // device staging of host uploads (pad_volume), grown on demand up to kUploadBytes (one
+    // slab of four planes where that is more)
+    std::mutex upload_mu;
+    void* d_upload = nullptr;
+    size_t upload_bytes = 0;
 };
 
 namespace {
@@ -360,59 +366,36 @@ int render_impl(spr_ctx* c, const VolSlot& vs, const spr_params& prm, int method
 }
 
 
-// Bounds of the 8x8x8 bricks of a padded volume (brick_bounds.h): thread bx of block
-// (by, bz) scans brick (bx, by, bz) over the padded voxels [8 b, 8 b + 8) clipped to the
-// padded extent (PX = nx + 2, PY, PZ); total gets the minimum of every brick's keys (the
-// volume's bounds), one atomic per wave.  A NaN voxel gives its brick the widest keys.
+// Padded planes [4 bz0, 4 bz1) of the slot's padded copy, with their block bounds (blocks not
+// nullptr), from source planes sz0 on
 template <typename T>
-__global__ __launch_bounds__(64) void k_brick_bounds(const T* __restrict__ pad, uint32_t pitch,
-                                                     uint32_t PX, uint32_t PY, uint32_t PZ,
-                                                     uint32_t nbx, uint32_t nby,
-                                                     BrickKey* __restrict__ keys,
-                                                     BrickKey* __restrict__ total) {
-    const uint32_t bx = blockIdx.x * 64u + threadIdx.x, by = blockIdx.y, bz = blockIdx.z;
-    uint32_t kmin = 0xFFFFFFFFu, nkmax = 0xFFFFFFFFu;
-    if (bx < nbx) {
-        const uint32_t x0 = bx * kBrick, x1 = min(x0 + kBrick, PX);
-        const uint32_t y1 = min(by * kBrick + kBrick, PY), z1 = min(bz * kBrick + kBrick, PZ);
-        for (uint32_t z = bz * kBrick; z < z1; ++z)
-            for (uint32_t y = by * kBrick; y < y1; ++y) {
-                const T* row = pad + ((size_t)z * PY + y) * pitch;
-                for (uint32_t x = x0; x < x1; ++x) {
-                    const T v = row[x];
-                    if (v != v) {  // NaN (float voxels only)
-                        kmin = nkmax = 0u;
-                    } else {
-                        const uint32_t k = order_key(v);
-                        kmin = min(kmin, k);
-                        nkmax = min(nkmax, ~k);
-                    }
-                }
-            }
-        keys[((size_t)bz * nby + by) * nbx + bx] = BrickKey{kmin, nkmax};
-    }
-    for (int off = 32; off > 0; off >>= 1) {
-        kmin = min(kmin, (uint32_t)__shfl_xor((int)kmin, off));
-        nkmax = min(nkmax, (uint32_t)__shfl_xor((int)nkmax, off));
-    }
-    if (threadIdx.x == 0) {
-        atomicMin(&total->kmin, kmin);
-        atomicMin(&total->nkmax, nkmax);
-    }
+void launch_pad(const VolSlot& vs, const void* src, int sz0, uint32_t bz0, uint32_t bz1,
+                void* blocks, hipStream_t s) {
+    const uint32_t cols = padded_pitch<T>(vs.nx) / VoxelUnit<T>::E * win_entries((uint32_t)vs.ny + 2u);
+    hipLaunchKernelGGL(k_pad_blocks<T>, dim3((cols + 255u) / 256u, bz1 - bz0), dim3(256), 0, s,
+                       (const T*)src, (T*)vs.d_pad, vs.nx, vs.ny, vs.nz, bz0, sz0,
+                       (BlockBounds<T>*)blocks);
 }
 
-template <typename T>
-void launch_bricks(const VolSlot& vs, BrickKey* total, hipStream_t s) {
-    const uint32_t PX = (uint32_t)vs.nx + 2u, PY = (uint32_t)vs.ny + 2u, PZ = (uint32_t)vs.nz + 2u;
-    const dim3 grid((vs.nbx + 63u) / 64u, vs.nby, vs.nbz);
-    hipLaunchKernelGGL(k_brick_bounds<T>, grid, dim3(64), 0, s, (const T*)vs.d_pad,
-                       padded_pitch<T>(vs.nx), PX, PY, PZ, vs.nbx, vs.nby, vs.d_bricks, total);
+hipError_t launch_pad(const VolSlot& vs, const void* src, int sz0, uint32_t bz0, uint32_t bz1,
+                      void* blocks, hipStream_t s) {
+    switch (vs.dtype) {
+        case SPR_DTYPE_F32: launch_pad<float>(vs, src, sz0, bz0, bz1, blocks, s); break;
+        case SPR_DTYPE_U16: launch_pad<uint16_t>(vs, src, sz0, bz0, bz1, blocks, s); break;
+        case SPR_DTYPE_U16X2: launch_pad<U16Pair>(vs, src, sz0, bz0, bz1, nullptr, s); break;
+        default: launch_pad<uint8_t>(vs, src, sz0, bz0, bz1, blocks, s); break;
+    }
+    return hipGetLastError();
 }
 
+// The window grid and the brick keys from the block bounds; *total: the volume's keys
 template <typename T>
-void launch_pad(const void* src, void* dst, int nx, int ny, int nz, hipStream_t s) {
-    dim3 grid((padded_pitch<T>(nx) + 255) / 256, ny + 2, nz + 2);
-    hipLaunchKernelGGL(k_pad_volume<T>, grid, dim3(256), 0, s, (const T*)src, (T*)dst, nx, ny, nz);
+void launch_windows(const VolSlot& vs, const void* blocks, BrickKey* total, hipStream_t s) {
+    const uint32_t gx = vs.win[0], gy = vs.win[1], gz = vs.win[2];
+    const dim3 grid(std::min((gx * gy + 255u) / 256u, 16u), gz);
+    hipLaunchKernelGGL(k_block_windows<T>, grid, dim3(256), 0, s, (const BlockBounds<T>*)blocks,
+                       padded_pitch<T>(vs.nx) / 4u, gx, gy, gz, (T*)vs.win_max(), (T*)vs.win_min(),
+                       vs.nbx, vs.nby, vs.d_bricks, total);
 }
 
 // out(x, y, z) = max of in over [c - r, c + r] along AXIS (0 x, 1 y, 2 z), coordinates
@@ -512,6 +495,44 @@ void launch_max_filter3(const VolSlot& vs, void* t1, void* t2, int r, hipStream_
                        vs.nz, vs.nx, vs.ny, 0, r);
 }
 
+// Bytes of the context's device staging buffer for host uploads: a volume goes to its padded
+// layout a slab of planes at a time, so an upload holds (and allocates) no second copy of
+// the volume.
+constexpr size_t kUploadBytes = (size_t)64 << 20;
+
+// The slot's padded copy and block bounds from the (nz, ny, nx) array src: device memory in
+// one launch, host memory (from_host) a slab at a time through the staging buffer.
+hipError_t pad_volume(spr_ctx* c, const VolSlot& vs, const void* src, bool from_host, void* blocks) {
+    const uint32_t nbz = win_entries((uint32_t)vs.nz + 2u);
+    if (!from_host) return launch_pad(vs, src, 0, 0, nbz, blocks, c->stream);
+    const size_t plane = (size_t)vs.nx * vs.ny * dtype_size(vs.dtype);
+    // block planes per slab: a slab of n block planes needs 4 n source planes
+    const uint32_t step = (uint32_t)std::min<size_t>(
+        nbz, std::max<size_t>(1, kUploadBytes / (kWinStride * plane)));
+    const size_t need = std::min<size_t>((size_t)step * kWinStride, (size_t)vs.nz) * plane;
+    std::lock_guard<std::mutex> lock(c->upload_mu);
+    hipError_t e = hipSuccess;
+    if (c->upload_bytes < need) {
+        if (c->d_upload) (void)hipFree(c->d_upload);
+        c->d_upload = nullptr;
+        c->upload_bytes = 0;
+        e = hipMalloc(&c->d_upload, need);
+        if (e != hipSuccess) return e;
+        c->upload_bytes = need;
+    }
+    for (uint32_t b = 0; b < nbz && e == hipSuccess; b += step) {
+        const uint32_t b1 = std::min(nbz, b + step);
+        // padded plane z holds source plane z - 1 (clamped)
+        const int z0 = std::min(std::max((int)(b * kWinStride) - 1, 0), vs.nz - 1);
+        const int z1 = std::min((int)(b1 * kWinStride) - 1, vs.nz);
+        if (z0 < z1)
+            e = hipMemcpyAsync(c->d_upload, (const char*)src + (size_t)z0 * plane,
+                               (size_t)(z1 - z0) * plane, hipMemcpyHostToDevice, c->stream);
+        if (e == hipSuccess) e = launch_pad(vs, c->d_upload, z0, b, b1, blocks, c->stream);
+    }
+    return e;
+}
+
 // fill one slot from host or device memory in the requested layout
 int fill_slot(spr_ctx* c, VolSlot& vs, const void* src, bool src_on_device, int dtype, int nx,
               int ny, int nz) {
@@ -546,16 +567,24 @@ int fill_slot(spr_ctx* c, VolSlot& vs, const void* src, bool src_on_device, int 
     if (src_on_device) HIPCALL(c, hipDeviceSynchronize());
 
     // what a batch graph captured of this slot (device buffers, shape, type, layout): a
-    // refill that keeps all of it keeps the slot's generation
+    // refill from device memory that keeps all of it keeps the slot's generation (a host
+    // upload to the padded layout always starts a new one)
     const VolSlot before = vs;
-    bool realloc = false;
-    // linear copy: kept as the resident volume (LINEAR), or staged for padding (host source)
-    const bool need_linear = layout == SPR_LAYOUT_LINEAR || !src_on_device;
-    if (vs.d_pad && (!want_pad || vs.pad_bytes != pbytes)) {
+    bool realloc = !src_on_device && layout == SPR_LAYOUT_PADDED;
+    // bounds of the padded copy (one-channel volumes): the window grid behind it in its
+    // allocation, the brick keys in their own
+    const bool want_bounds = want_pad && dtype != SPR_DTYPE_U16X2;
+    const uint32_t px = (uint32_t)nx + 2u, py = (uint32_t)ny + 2u, pz = (uint32_t)nz + 2u;
+    const uint32_t win[3] = {want_bounds ? win_entries(px) : 0u, want_bounds ? win_entries(py) : 0u,
+                             want_bounds ? win_entries(pz) : 0u};
+    const size_t wbytes = (size_t)win[0] * win[1] * win[2] * es;
+    // linear copy: kept as the resident volume (LINEAR layout)
+    const bool need_linear = layout == SPR_LAYOUT_LINEAR;
+    if (vs.d_pad && (!want_pad || vs.pad_bytes != pbytes || vs.win_bytes != wbytes)) {
         realloc = true;
         HIPCALL(c, hipFree(vs.d_pad));
         vs.d_pad = nullptr;
-        vs.pad_bytes = 0;
+        vs.pad_bytes = vs.win_bytes = 0;
     }
     if (vs.d_vol && (!need_linear || vs.vol_bytes != bytes)) {
         realloc = true;
@@ -573,27 +602,10 @@ int fill_slot(spr_ctx* c, VolSlot& vs, const void* src, bool src_on_device, int 
         HIPCALL(c, hipMemcpyAsync(vs.d_vol, src, bytes,
                                   src_on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice,
                                   c->stream));
-    if (want_pad) {
-        if (!vs.d_pad) {
-            realloc = true;
-            HIPCALL(c, hipMalloc(&vs.d_pad, pbytes));
-            vs.pad_bytes = pbytes;
-        }
-        const void* from = need_linear ? vs.d_vol : src;
-        switch (dtype) {
-            case SPR_DTYPE_F32: launch_pad<float>(from, vs.d_pad, nx, ny, nz, c->stream); break;
-            case SPR_DTYPE_U16: launch_pad<uint16_t>(from, vs.d_pad, nx, ny, nz, c->stream); break;
-            case SPR_DTYPE_U16X2: launch_pad<U16Pair>(from, vs.d_pad, nx, ny, nz, c->stream); break;
-            default: launch_pad<uint8_t>(from, vs.d_pad, nx, ny, nz, c->stream); break;
-        }
-        HIPCALL(c, hipGetLastError());
-    }
-    // per-brick bounds of the padded copy (one-channel volumes) and the volume's bounds
-    const uint32_t nbx = want_pad ? ((uint32_t)nx + 2u + kBrick - 1u) / kBrick : 0u;
-    const uint32_t nby = want_pad ? ((uint32_t)ny + 2u + kBrick - 1u) / kBrick : 0u;
-    const uint32_t nbz = want_pad ? ((uint32_t)nz + 2u + kBrick - 1u) / kBrick : 0u;
-    const bool want_bricks = want_pad && dtype != SPR_DTYPE_U16X2;
-    if (vs.d_bricks && (!want_bricks || vs.nbx != nbx || vs.nby != nby || vs.nbz != nbz)) {
+    const uint32_t nbx = want_pad ? (px + kBrick - 1u) / kBrick : 0u;
+    const uint32_t nby = want_pad ? (py + kBrick - 1u) / kBrick : 0u;
+    const uint32_t nbz = want_pad ? (pz + kBrick - 1u) / kBrick : 0u;
+    if (vs.d_bricks && (!want_bounds || vs.nbx != nbx || vs.nby != nby || vs.nbz != nbz)) {
         realloc = true;
         HIPCALL(c, hipFree(vs.d_bricks));
         vs.d_bricks = nullptr;
@@ -601,52 +613,55 @@ int fill_slot(spr_ctx* c, VolSlot& vs, const void* src, bool src_on_device, int 
     vs.nbx = nbx;
     vs.nby = nby;
     vs.nbz = nbz;
-    if (want_bricks) {
-        const size_t nbricks = (size_t)nbx * nby * nbz;
-        if (!vs.d_bricks) {
-            realloc = true;
-            // one more entry: the volume's bounds
-            HIPCALL(c, hipMalloc(&vs.d_bricks, (nbricks + 1) * sizeof(BrickKey)));
-        }
-        BrickKey* total = vs.d_bricks + nbricks;
-        vs.dtype = dtype;
-        vs.nx = nx;
-        vs.ny = ny;
-        vs.nz = nz;
-        HIPCALL(c, hipMemsetAsync(total, 0xFF, sizeof(BrickKey), c->stream));
-        switch (dtype) {
-            case SPR_DTYPE_F32: launch_bricks<float>(vs, total, c->stream); break;
-            case SPR_DTYPE_U16: launch_bricks<uint16_t>(vs, total, c->stream); break;
-            default: launch_bricks<uint8_t>(vs, total, c->stream); break;
-        }
-        HIPCALL(c, hipGetLastError());
-        BrickKey t;
-        HIPCALL(c, hipMemcpyAsync(&t, total, sizeof(t), hipMemcpyDeviceToHost, c->stream));
-        HIPCALL(c, hipStreamSynchronize(c->stream));
-        switch (dtype) {
-            case SPR_DTYPE_F32:
-                vs.vmin = key_value<float>(t.kmin);
-                vs.vmax = key_value<float>(~t.nkmax);
-                break;
-            default:
-                vs.vmin = (float)t.kmin;
-                vs.vmax = (float)~t.nkmax;
-                break;
-        }
-    }
-    HIPCALL(c, hipStreamSynchronize(c->stream));
-    if (layout == SPR_LAYOUT_PADDED && vs.d_vol) {  // staging copy no longer needed
-        HIPCALL(c, hipFree(vs.d_vol));
-        vs.d_vol = nullptr;
-        vs.vol_bytes = 0;
-    }
-    vs.used = true;
-    vs.layout = layout;
-    vs.pad_wide = wide;
+    for (int k = 0; k < 3; ++k) vs.win[k] = win[k];
     vs.dtype = dtype;
     vs.nx = nx;
     vs.ny = ny;
     vs.nz = nz;
+    if (want_pad) {
+        if (!vs.d_pad) {
+            realloc = true;
+            HIPCALL(c, hipMalloc(&vs.d_pad, VolSlot::align256(pbytes) + 2 * VolSlot::align256(wbytes)));
+            vs.pad_bytes = pbytes;
+            vs.win_bytes = wbytes;
+        }
+        const size_t nbricks = (size_t)nbx * nby * nbz;
+        if (want_bounds && !vs.d_bricks) {
+            realloc = true;
+            // one more entry: the volume's bounds
+            HIPCALL(c, hipMalloc(&vs.d_bricks, (nbricks + 1) * sizeof(BrickKey)));
+        }
+        // the 4x4x4 block bounds live from the padding pass to the windows' only
+        void* blocks = nullptr;
+        if (want_bounds)
+            HIPCALL(c, hipMallocAsync(&blocks, pitch / 4 * win[1] * win[2] * 2 * es, c->stream));
+        hipError_t e = pad_volume(c, vs, need_linear ? vs.d_vol : src, !need_linear && !src_on_device,
+                                  blocks);
+        if (want_bounds) {
+            BrickKey* total = vs.d_bricks + nbricks;
+            BrickKey t{};
+            if (e == hipSuccess) e = hipMemsetAsync(total, 0xFF, sizeof(BrickKey), c->stream);
+            if (e == hipSuccess) {
+                switch (dtype) {
+                    case SPR_DTYPE_F32: launch_windows<float>(vs, blocks, total, c->stream); break;
+                    case SPR_DTYPE_U16: launch_windows<uint16_t>(vs, blocks, total, c->stream); break;
+                    default: launch_windows<uint8_t>(vs, blocks, total, c->stream); break;
+                }
+                e = hipGetLastError();
+            }
+            if (blocks) (void)hipFreeAsync(blocks, c->stream);
+            if (e == hipSuccess)
+                e = hipMemcpyAsync(&t, total, sizeof(t), hipMemcpyDeviceToHost, c->stream);
+            if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+            vs.vmin = dtype == SPR_DTYPE_F32 ? key_value<float>(t.kmin) : (float)t.kmin;
+            vs.vmax = dtype == SPR_DTYPE_F32 ? key_value<float>(~t.nkmax) : (float)~t.nkmax;
+        }
+        HIPCALL(c, e);
+    }
+    HIPCALL(c, hipStreamSynchronize(c->stream));
+    vs.used = true;
+    vs.layout = layout;
+    vs.pad_wide = wide;
     if (realloc || !before.used || before.d_pad != vs.d_pad || before.d_vol != vs.d_vol ||
         before.layout != layout || before.dtype != dtype || before.nx != nx || before.ny != ny ||
         before.nz != nz)
@@ -869,6 +884,7 @@ int spr_destroy(spr_ctx* c) {
         for (VolSlot& v : c->vols) free_slot(v);
         if (c->d_count) (void)hipFree(c->d_count);
         if (c->d_partial) (void)hipFree(c->d_partial);
+        if (c->d_upload) (void)hipFree(c->d_upload);
         for (spr_ctx::Stage& st : c->stage) {
             if (st.done) (void)hipEventSynchronize(st.done);
             if (st.done) (void)hipEventDestroy(st.done);

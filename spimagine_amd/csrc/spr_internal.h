@@ -35,6 +35,13 @@ struct VolSlot {
     BrickKey* d_bricks = nullptr;
     uint32_t nbx = 0, nby = 0, nbz = 0;
     float vmin = 0.0f, vmax = 0.0f;
+    // the window grid (brick_bounds.h): entries per axis (0: none) and bytes of each of its
+    // two planes, which follow the padded copy in its allocation
+    uint32_t win[3] = {0, 0, 0};
+    size_t win_bytes = 0;
+    static size_t align256(size_t n) { return (n + 255) / 256 * 256; }
+    void* win_max() const { return (char*)d_pad + align256(pad_bytes); }
+    void* win_min() const { return (char*)win_max() + align256(win_bytes); }
 };
 
 // spr_set_tuning state (include/spimrender.h SPR_TUNE_*) plus the device's CU count

@@ -1,0 +1,159 @@
+// volume_build.h -- a volume's device layout from the uploaded (nz, ny, nx) array: the padded
+// copy (volume_sampler.h), the window grid and the brick keys (brick_bounds.h).
+#pragma once
+#include "volume_sampler.h"
+
+namespace spr {
+
+// 16 bytes of voxels
+template <typename T>
+struct alignas(16) VoxelUnit {
+    static constexpr uint32_t E = 16u / (uint32_t)sizeof(T);
+    T v[E];
+};
+
+// Minimum and maximum of one 4x4x4 block of padded voxels
+template <typename T>
+struct BlockBounds {
+    T lo, hi;
+};
+
+// Padded voxels and their 4x4x4 block bounds in one pass over the source.  A thread takes
+// one 16-byte unit column: 4 rows of 4 planes of the padded copy, written as aligned units
+// and reduced on the way to one block (4 voxels along x) per 4 elements.  Padded planes
+// [4 bz0, 4 (bz0 + gridDim.y)) clipped to nz + 2; src holds source planes from sz0 on.
+// blocks: (bz, by, bx) with pitch / 4 blocks a row, or nullptr (no bounds wanted).
+//
+// Bound by HBM: the source read once and the copy written once.  Before, the copy went
+// voxel by voxel (2-byte loads and stores) and a second pass read the copy back one brick
+// a thread: 0.36 + 0.37 ms for a 512^3 uint16 volume, 268 MB.
+template <typename T>
+__global__ __launch_bounds__(256) void k_pad_blocks(const T* __restrict__ src, T* __restrict__ dst,
+                                                    int nx, int ny, int nz, uint32_t bz0, int sz0,
+                                                    BlockBounds<T>* __restrict__ blocks) {
+    using U = VoxelUnit<T>;
+    constexpr int E = (int)U::E;
+    constexpr bool kBounds = std::is_arithmetic<T>::value;
+    const uint32_t pitch = padded_pitch<T>(nx), PY = (uint32_t)ny + 2u, PZ = (uint32_t)nz + 2u;
+    const uint32_t units = pitch / (uint32_t)E, nby = win_entries(PY);
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    const uint32_t by = i / units, ux = i - by * units, bz = bz0 + blockIdx.y;
+    if (by >= nby) return;
+    const int x0 = (int)(ux * (uint32_t)E) - 1;  // source x of the unit's first voxel
+    const bool whole = x0 >= 0 && x0 + E <= nx;
+    T lo[E], hi[E];
+    bool bad[E / 4];
+#pragma unroll
+    for (int b = 0; b < E / 4; ++b) bad[b] = false;
+    bool first = true;
+    for (uint32_t k = 0; k < kWinStride; ++k) {
+        const uint32_t z = bz * kWinStride + k;
+        if (z >= PZ) break;
+        const int sz = min(max((int)z - 1, 0), nz - 1) - sz0;
+        U u[kWinStride];
+#pragma unroll
+        for (uint32_t r = 0; r < kWinStride; ++r) {
+            const uint32_t y = min(by * kWinStride + r, PY - 1u);
+            const int sy = min(max((int)y - 1, 0), ny - 1);
+            const T* row = src + ((size_t)sz * ny + sy) * nx;
+            if (whole) {
+                __builtin_memcpy(&u[r], row + x0, 16);
+            } else {
+#pragma unroll
+                for (int e = 0; e < E; ++e) u[r].v[e] = row[min(max(x0 + e, 0), nx - 1)];
+            }
+        }
+#pragma unroll
+        for (uint32_t r = 0; r < kWinStride; ++r) {
+            const uint32_t y = by * kWinStride + r;
+            if (y < PY)
+                *reinterpret_cast<U*>(dst + ((size_t)z * PY + y) * pitch + ux * (uint32_t)E) = u[r];
+            if constexpr (kBounds) {  // (a row past the last repeats it: the same bounds)
+#pragma unroll
+                for (int e = 0; e < E; ++e) {
+                    const T v = u[r].v[e];
+                    if constexpr (std::is_same<T, float>::value) bad[e / 4] = bad[e / 4] || v != v;
+                    lo[e] = first || v < lo[e] ? v : lo[e];
+                    hi[e] = first || v > hi[e] ? v : hi[e];
+                }
+                first = false;
+            }
+        }
+    }
+    if constexpr (kBounds) {
+        if (blocks == nullptr) return;
+        BlockBounds<T>* o = blocks + ((size_t)bz * nby + by) * (pitch / 4u) + ux * (uint32_t)(E / 4);
+#pragma unroll
+        for (int b = 0; b < E / 4; ++b) {
+            BlockBounds<T> m{lo[4 * b], hi[4 * b]};
+#pragma unroll
+            for (int e = 4 * b + 1; e < 4 * b + 4; ++e) {
+                m.lo = lo[e] < m.lo ? lo[e] : m.lo;
+                m.hi = hi[e] > m.hi ? hi[e] : m.hi;
+            }
+            if constexpr (std::is_same<T, float>::value)
+                if (bad[b]) m = BlockBounds<T>{-INFINITY, INFINITY};
+            o[b] = m;
+        }
+    }
+}
+
+// The window grid from the 4x4x4 blocks (window (x, y, z) = blocks x, x+1 / y, y+1 / z, z+1
+// that exist), the 8x8x8 brick keys (brick b is window 2b) and the minimum of every brick's
+// keys (total: the volume's bounds).  grid.y = window planes; a few workgroups a plane, so
+// that few atomics meet in total.  Reads 1/16 of the volume's bytes or less.
+template <typename T>
+__global__ __launch_bounds__(256) void k_block_windows(const BlockBounds<T>* __restrict__ blocks,
+                                                       uint32_t bpitch, uint32_t gx, uint32_t gy,
+                                                       uint32_t gz, T* __restrict__ wmax,
+                                                       T* __restrict__ wmin, uint32_t nbx,
+                                                       uint32_t nby, BrickKey* __restrict__ keys,
+                                                       BrickKey* __restrict__ total) {
+    __shared__ BrickKey part[4];
+    const uint32_t z = blockIdx.y;
+    uint32_t kmin = 0xFFFFFFFFu, nkmax = 0xFFFFFFFFu;
+    for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < gx * gy; i += gridDim.x * 256u) {
+        const uint32_t y = i / gx, x = i - y * gx;
+        BlockBounds<T> m = blocks[((size_t)z * gy + y) * bpitch + x];
+#pragma unroll
+        for (uint32_t c = 1; c < 8; ++c) {
+            const uint32_t xx = min(x + (c & 1u), gx - 1u), yy = min(y + ((c >> 1) & 1u), gy - 1u),
+                           zz = min(z + (c >> 2), gz - 1u);
+            const BlockBounds<T> b = blocks[((size_t)zz * gy + yy) * bpitch + xx];
+            m.lo = b.lo < m.lo ? b.lo : m.lo;
+            m.hi = b.hi > m.hi ? b.hi : m.hi;
+        }
+        if (((x | y | z) & 1u) == 0u) {
+            BrickKey k{order_key(m.lo), ~order_key(m.hi)};
+            if constexpr (std::is_same<T, float>::value)
+                if (m.lo == -INFINITY && m.hi == INFINITY) k = BrickKey{0u, 0u};
+            keys[((size_t)(z >> 1) * nby + (y >> 1)) * nbx + (x >> 1)] = k;
+            kmin = min(kmin, k.kmin);
+            nkmax = min(nkmax, k.nkmax);
+        }
+        if constexpr (std::is_same<T, float>::value) {
+            const float g = bound_margin<T>(m.lo, m.hi);
+            m.lo = m.lo - g;
+            m.hi = m.hi + g;
+        }
+        const size_t o = ((size_t)z * gy + y) * gx + x;
+        wmax[o] = m.hi;
+        wmin[o] = m.lo;
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+        kmin = min(kmin, (uint32_t)__shfl_xor((int)kmin, off));
+        nkmax = min(nkmax, (uint32_t)__shfl_xor((int)nkmax, off));
+    }
+    if ((threadIdx.x & 63u) == 0u) part[threadIdx.x >> 6] = BrickKey{kmin, nkmax};
+    __syncthreads();
+    if (threadIdx.x == 0 && (z & 1u) == 0u) {
+        for (int w = 0; w < 4; ++w) {
+            kmin = min(kmin, part[w].kmin);
+            nkmax = min(nkmax, part[w].nkmax);
+        }
+        atomicMin(&total->kmin, kmin);
+        atomicMin(&total->nkmax, nkmax);
+    }
+}
+
+}  // namespace spr

@@ -318,19 +318,4 @@ struct is_padded<PaddedVolume<T, POW2, WIDE>> {
     static constexpr bool value = true;
 };
 
-// padded[z][y][x] = vol[clamp(z-1)][clamp(y-1)][clamp(x-1)] for x < pitch (the columns
-// past nx+1 also replicate the last voxel)
-template <typename T>
-__global__ __launch_bounds__(256) void k_pad_volume(const T* __restrict__ src, T* __restrict__ dst,
-                                                    int nx, int ny, int nz) {
-    const int PXP = (int)padded_pitch<T>(nx), PY = ny + 2;
-    const int x = blockIdx.x * 256 + threadIdx.x;
-    const int y = blockIdx.y, z = blockIdx.z;
-    if (x >= PXP) return;
-    const int sx = min(max(x - 1, 0), nx - 1);
-    const int sy = min(max(y - 1, 0), ny - 1);
-    const int sz = min(max(z - 1, 0), nz - 1);
-    dst[((size_t)z * PY + y) * PXP + x] = src[((size_t)sz * ny + sy) * nx + sx];
-}
-
 }  // namespace spr
