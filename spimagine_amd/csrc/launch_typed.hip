@@ -315,6 +315,19 @@ void launch_pair_ch(const VolSlot& vs, bool one_wave, dim3 grid, hipStream_t s, 
 }  // namespace
 
 #if SPR_PART != 1
+// the max projection gathered group by group where the window grid leaves something to gain
+template <typename T, bool P2, bool WIDE>
+void launch_windows(int gs, const PaddedVolume<T, P2, WIDE>& v, const RayParams& p, float* out,
+                    float* alpha, hipStream_t s) {
+    const dim3 g(4 * tile_grid(kTileMapInterleaved, p.ntx, p.nty)), block(64 * kWinSegments);
+    if (gs == 4)
+        hipLaunchKernelGGL((k_mip_windows<T, P2, 4, WIDE>), g, block, 0, s, v, p, out, alpha);
+    else if (gs == 2)
+        hipLaunchKernelGGL((k_mip_windows<T, P2, 2, WIDE>), g, block, 0, s, v, p, out, alpha);
+    else
+        hipLaunchKernelGGL((k_mip_windows<T, P2, 1, WIDE>), g, block, 0, s, v, p, out, alpha);
+}
+
 template <typename T, bool P2>
 hipError_t TypedLaunch<T, P2>::max_project(const LaunchTuning& t, const VolSlot& vs, RayParams p,
                                            bool nearest, float* out, float* alpha, hipStream_t s) {
@@ -344,6 +357,17 @@ hipError_t TypedLaunch<T, P2>::max_project(const LaunchTuning& t, const VolSlot&
         }
         if (obuf) (void)hipFreeAsync(obuf, s);
         return e;
+    }
+    // with the default tuning, frames that gain by it are gathered group by group
+    const float step = (float)nmax / (16.0f * (float)p.nouter);
+    if (staged && skip && t.slab_kb == 19 && t.chunk == 0 && t.row_pad == 0 && t.wg_waves != 4 &&
+        t.tile_map == (int)kTileMapInterleaved && windows_pay(vs.need, step, 4u * p.ntiles)) {
+        const int gs = windows_group(step);
+        if (vs.pad_wide)
+            launch_windows(gs, padded_volume<T, P2, true>(vs), p, out, alpha, s);
+        else
+            launch_windows(gs, padded_volume<T, P2>(vs), p, out, alpha, s);
+        return hipGetLastError();
     }
     if ((staged || staged_opac) && vs.pad_wide) {
         const bool one_wave = one_wave_for(t, p);

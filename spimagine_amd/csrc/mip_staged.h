@@ -1640,6 +1640,9 @@ __device__ __forceinline__ PaddedVolume<T, POW2> job_volume(const BatchJob& j) {
     v.bricks.keys = nullptr;  // batched frames sample every box
     v.bricks.nbx = v.bricks.nby = 0;
     v.vmin = v.vmax = 0.0f;
+    v.win_max = v.win_min = nullptr;
+    v.win_gx = v.win_gy = 0;
+    v.wnx = v.wny = v.wnz = 0.0f;
     return v;
 }
 

@@ -1,0 +1,257 @@
+// mip_windows.h -- max projection that samples only where a ray's maximum can still rise.
+//
+// Same result, bit for bit, as k_max_project (volume_kernel.cl:20-185, :190-345 with
+// alpha_pow == 0): a maximum does not depend on which samples that cannot change it are
+// left out, and every sample taken sits at the reference's running-sum position.
+//
+// Each ray asks the window grid (brick_bounds.h) for the largest voxel its next GS samples
+// can read -- one lookup, ~4 instructions a sample against ~52 for a trilinear sample -- and
+// samples a group only when that exceeds its running maximum.  Skipping pays once the
+// maxima are high, so a ray first probes the grid along its length and takes the samples
+// where the bound is largest.  On 512^3 blob volumes with camera noise 27% of the rays'
+// groups are then left; asked per 8x8 rays, as a staged box would be, 44%, and by the
+// wave's 32-sample box and 8^3 bricks (mip_staged.h) 94%.
+#pragma once
+#include "mip_staged.h"
+
+namespace spr {
+
+// p after n additions of d, each rounded (p = p + d), in one step: while the sums stay in
+// one binade each addition moves p by the same multiple of its ulp, ties included (a tie
+// rounds to the even neighbour, so the sum after it starts even and rounds the same way
+// from then on: the step is taken from the third addition, whose two predecessors started
+// on the binade's own grid).  Valid only when `same`: the first sum and the result lie in
+// one binade, the result inside it (a sum a little below 2^e would round to 2^e on this
+// binade's grid and not on the finer one below).  n >= 3.
+__device__ __forceinline__ float sum_ahead(float p, float d, float n, bool& same) {
+    const float a = p + d, b = a + d, c = b + d;
+    const float q = fmaf(n - 3.0f, c - b, c);
+    same = (__float_as_uint(a) ^ __float_as_uint(q)) < 0x00800000u &&
+           (__float_as_uint(q) & 0x007FFFFFu) != 0u;
+    return q;
+}
+
+// p after n additions of d, binade by binade
+__device__ __forceinline__ float sum_n(float p, float d, uint32_t n) {
+    while (n >= 6u) {
+        bool same;
+        float q = sum_ahead(p, d, (float)n, same);
+        if (same) return q;
+        // as many additions as surely stay in the first sum's binade, else three by hand
+        const float a = p + d, b = a + d, c = b + d;
+        const float lo = __uint_as_float(__float_as_uint(a) & 0xFF800000u);  // its signed 2^e
+        const float lim = (c > b) == (a > 0.0f) ? 2.0f * lo : lo;
+        const float m = floorf((lim - c) / (c - b)) - 1.0f;
+        q = sum_ahead(p, d, m + 3.0f, same);
+        const bool far = m >= 1.0f && m + 3.0f < (float)n && same;
+        p = far ? q : c;
+        n -= far ? (uint32_t)m + 3u : 3u;
+    }
+    for (; n > 0u; --n) p = p + d;
+    return p;
+}
+
+constexpr int kWinGroups = 8;  // groups asked for together
+
+// One ray's window lookups: the block coordinates of the least corner of group j's samples
+// are (wx + j gx, ...), in windows.
+template <typename V, int GS>
+struct WindowRay {
+    float gx, gy, gz;  // advance of one group
+    bool ok;           // a group's corners always lie in the one window
+
+    __device__ __forceinline__ void begin(const V& vol, float dx, float dy, float dz, float mgx,
+                                          float mgy, float mgz) {
+        const float vx = dx * vol.fnx, vy = dy * vol.fny, vz = dz * vol.fnz;
+        gx = (float)GS * 0.25f * vx;
+        gy = (float)GS * 0.25f * vy;
+        gz = (float)GS * 0.25f * vz;
+        const float span = (float)(GS - 1);
+        ok = fmaf(span, fabsf(vx), 2.0f * mgx) <= 3.0f && fmaf(span, fabsf(vy), 2.0f * mgy) <= 3.0f &&
+             fmaf(span, fabsf(vz), 2.0f * mgz) <= 3.0f;
+    }
+    // block coordinates of the group whose first sample is at (px, py, pz)
+    __device__ __forceinline__ void at(const V& vol, float px, float py, float pz, float mgx,
+                                       float mgy, float mgz, float& wx, float& wy,
+                                       float& wz) const {
+        constexpr float kBack = (float)(GS - 1) / (float)GS;
+        wx = fmaf(0.25f, texel<V::kPow2>(px, vol.fnx) + (1.0f - mgx), fminf(kBack * gx, 0.0f));
+        wy = fmaf(0.25f, texel<V::kPow2>(py, vol.fny) + (1.0f - mgy), fminf(kBack * gy, 0.0f));
+        wz = fmaf(0.25f, texel<V::kPow2>(pz, vol.fnz) + (1.0f - mgz), fminf(kBack * gz, 0.0f));
+    }
+    __device__ __forceinline__ typename V::value_type top(const V& vol, float wx, float wy,
+                                                          float wz) const {
+        return vol.win_max[vol.window(wx, wy, wz)];
+    }
+    // first sample of the two groups most likely to hold the ray's maximum among `count`
+    // samples from (px, py, pz) on: the largest bound among windows two groups apart
+    __device__ __forceinline__ int best(const V& vol, float px, float py, float pz,
+                                        int count) const {
+        constexpr int PS = 2 * GS;
+        const int probes = (count + PS - 1) / PS;
+        // a probed window reaches two voxels either side of the two groups' middle
+        const float sx = 2.0f * gx, sy = 2.0f * gy, sz = 2.0f * gz;
+        const float bx = fmaf(0.25f, texel<V::kPow2>(px, vol.fnx) - 1.0f, gx),
+                    by = fmaf(0.25f, texel<V::kPow2>(py, vol.fny) - 1.0f, gy),
+                    bz = fmaf(0.25f, texel<V::kPow2>(pz, vol.fnz) - 1.0f, gz);
+        float top_u = -1.0f;
+        int at = 0;
+        for (int i = 0; i < probes; i += 16) {
+            typename V::value_type v[16];
+#pragma unroll
+            for (int k = 0; k < 16; ++k) {
+                const float f = (float)min(i + k, probes - 1);
+                v[k] = top(vol, fmaf(f, sx, bx), fmaf(f, sy, by), fmaf(f, sz, bz));
+            }
+#pragma unroll
+            for (int k = 0; k < 16; ++k) {
+                const float u = (float)v[k];
+                at = u > top_u ? min(i + k, probes - 1) : at;
+                top_u = fmaxf(top_u, u);
+            }
+        }
+        return max(0, min(at * PS, count - PS));
+    }
+};
+
+// One 8x8 pixel quarter of a 16x16 tile per workgroup; its kWinSegments waves march a
+// segment each of the rays' samples and share the running maxima.  No boxes are staged: a
+// wave puts the groups its rays still need into a queue in LDS, and whenever 64 are waiting
+// every lane takes one, gathers its samples from global memory and posts the maximum to
+// the ray's word, so no lane idles through groups that other rays need.
+//
+// Bound by the vector-memory path: ~40 of a gather's 64 lanes touch cache lines of their
+// own (1024x1024x512 uint16 -> 1024^2, 1536 steps: 14.0 M gathers, address units busy 80%
+// of the frame, VALU 37%).
+constexpr int kWinSegments = 4;
+
+// Samples per group for a step of at most `step` voxels along an axis: as many as one window
+// surely holds (WindowRay::ok; rays whose group spans more sample everything).
+__host__ inline int windows_group(float step) {
+    return 3.0f * step <= 2.9f ? 4 : step <= 2.9f ? 2 : 1;
+}
+
+// Whether the frame is gathered group by group (k_mip_windows) instead of staged box by box.
+// need: the volume's share of windows to sample (k_window_need); step: voxels a sample;
+// tiles: 8x8 pixel quarters.  Gathered samples cost 3-4 times staged ones at a fine step, so
+// most groups have to fall away there; from 1.5 voxels a step on a staged box holds few
+// samples of many voxels, and a frame of few rays leaves most of the GPU idle unless their
+// segments are marched side by side.  us staged / gathered, 800^2 frames:
+//   512^3 blobs, uint16 (need 0.044): 896 steps 864 / 715, 320 steps 566 / 353, 102 294 / 179
+//   256^3 blobs, uint16 (0.080): 448 steps 392 / 352, 102 steps 179 / 139
+//   256^3 blobs, float (0.106): 448 steps 353 / 394, 102 steps 183 / 145
+//   512^3 white noise (1.0): 896 steps 956 / 2377, 204 steps 513 / 687
+//   200^2 frame of 128^3 float blobs (0.35), 200 steps: 76 / 55
+__host__ inline bool windows_pay(float need, float step, uint32_t tiles) {
+    if (step >= 1.5f || tiles < 2048u) return need < 0.6f;
+    return need < 0.09f;
+}
+
+template <typename T, bool POW2, int GS, bool WIDE>
+__global__ __launch_bounds__(64 * kWinSegments) void k_mip_windows(
+    PaddedVolume<T, POW2, WIDE> vol, RayParams p, float* __restrict__ out, float* __restrict__ alpha) {
+    using PV = PaddedVolume<T, POW2, WIDE>;
+    constexpr bool kShort = !std::is_same<T, float>::value;
+    constexpr int BS = kWinGroups * GS;
+    __shared__ float4 s_item[kWinSegments][128];  // waiting groups: position, ray (w's bits)
+    __shared__ float s_step[3][64];
+    __shared__ uint32_t s_max[64];  // the rays' running maxima (bits of floats >= 0)
+    const uint32_t lane = threadIdx.x & 63u, seg = threadIdx.x >> 6;
+    if (gate_closed(p)) return;  // uniform over the launch
+    uint32_t x = 0, y = 0;
+    const bool inside = wave_tile_pixel(p, &x, &y);
+    float px = 0.5f, py = 0.5f, pz = 0.5f, dx = 0.0f, dy = 0.0f, dz = 0.0f, tnear = 0.0f;
+    const bool active = inside && staged_ray_pos(p, x, y, px, py, pz, dx, dy, dz, tnear);
+    if (inside && !active && seg == 0) {
+        out[x + p.W * y] = 0.0f;
+        alpha[x + p.W * y] = kShort ? 0.0f : -1.0f;
+    }
+    const uint64_t act = __ballot(active);
+    if (act == 0) return;  // uniform over the workgroup: its waves have the same rays
+    shadow_first_active(act, active, px, py, pz, dx, dy, dz);
+    float4* const item = s_item[seg];
+    if (seg == 0) {
+        s_max[lane] = 0u;
+        s_step[0][lane] = dx;
+        s_step[1][lane] = dy;
+        s_step[2][lane] = dz;
+    }
+    __syncthreads();
+    const int total = (p.nouter + 1) * kLoopUnroll;
+    const int per = ((total + BS - 1) / BS + kWinSegments - 1) / kWinSegments * BS;
+    const int s0 = min((int)seg * per, total);
+    const int count = min(per, total - s0);
+    px = sum_n(px, dx, (uint32_t)s0);
+    py = sum_n(py, dy, (uint32_t)s0);
+    pz = sum_n(pz, dz, (uint32_t)s0);
+    const float mgx = 1e-5f * vol.fnx + 0.01f, mgy = 1e-5f * vol.fny + 0.01f,
+                mgz = 1e-5f * vol.fnz + 0.01f;
+    Opacity op;  // (unused)
+    WindowRay<PV, GS> win;
+    win.begin(vol, dx, dy, dz, mgx, mgy, mgz);
+    if (count > 0) {
+        const int first = win.best(vol, px, py, pz, count);
+        float qx = sum_n(px, dx, (uint32_t)first), qy = sum_n(py, dy, (uint32_t)first),
+              qz = sum_n(pz, dz, (uint32_t)first), c = 0.0f;
+        staged_sample_global<PV, 2 * GS>(vol, qx, qy, qz, dx, dy, dz, c, op);
+        if (c > 0.0f) atomicMax(&s_max[lane], __float_as_uint(c));
+    }
+    __syncthreads();
+    uint32_t waiting = 0;  // items in the queue (uniform)
+    // n items from the queue's end, one a lane
+    auto take = [&](uint32_t n) {
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        waiting -= n;
+        if (lane < n) {
+            const float4 it = item[waiting + lane];
+            const uint32_t ray = __float_as_uint(it.w);
+            float qx = it.x, qy = it.y, qz = it.z, c = 0.0f;
+            staged_sample_global<PV, GS>(vol, qx, qy, qz, s_step[0][ray], s_step[1][ray],
+                                         s_step[2][ray], c, op);
+            if (c > 0.0f) atomicMax(&s_max[ray], __float_as_uint(c));
+        }
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    };
+    T cur[kWinGroups], nxt[kWinGroups];
+    auto ask = [&](float ahead, T (&u)[kWinGroups]) {
+        float wx, wy, wz;
+        win.at(vol, px, py, pz, mgx, mgy, mgz, wx, wy, wz);
+#pragma unroll
+        for (int j = 0; j < kWinGroups; ++j) {
+            const float f = ahead + (float)j;
+            u[j] = win.top(vol, fmaf(f, win.gx, wx), fmaf(f, win.gy, wy), fmaf(f, win.gz, wz));
+        }
+    };
+    if (count > 0) ask(0.0f, cur);
+    for (int s = 0; s < count; s += BS) {
+        if (s + BS < count) ask((float)kWinGroups, nxt);
+        // (other waves may raise it meanwhile: a stale value only asks for more groups)
+        const float col = __uint_as_float(__hip_atomic_load(&s_max[lane], __ATOMIC_RELAXED,
+                                                            __HIP_MEMORY_SCOPE_WORKGROUP));
+#pragma unroll
+        for (int j = 0; j < kWinGroups; ++j) {
+            const bool need = active && s + j * GS < count && (!win.ok || (float)cur[j] > col);
+            const uint64_t m = __ballot(need);
+            if (need)
+                item[waiting + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] =
+                    float4{px, py, pz, __uint_as_float(lane)};
+            waiting += (uint32_t)__popcll(m);
+            if (waiting >= 64u) take(64u);
+#pragma unroll
+            for (int k = 0; k < GS; ++k) {
+                px = px + dx;
+                py = py + dy;
+                pz = pz + dz;
+            }
+            cur[j] = nxt[j];
+        }
+    }
+    if (waiting) take(waiting);
+    __syncthreads();
+    if (active && seg == 0)
+        staged_ray_end<kShort>(p, x + p.W * y, __uint_as_float(s_max[lane]), tnear, out, alpha);
+}
+
+}  // namespace spr

@@ -396,6 +396,10 @@ void launch_windows(const VolSlot& vs, const void* blocks, BrickKey* total, hipS
     hipLaunchKernelGGL(k_block_windows<T>, grid, dim3(256), 0, s, (const BlockBounds<T>*)blocks,
                        padded_pitch<T>(vs.nx) / 4u, gx, gy, gz, (T*)vs.win_max(), (T*)vs.win_min(),
                        vs.nbx, vs.nby, vs.d_bricks, total);
+    const uint32_t cols = std::max(gx * gy, std::max(gy * gz, gx * gz));
+    hipLaunchKernelGGL(k_window_need<T>, dim3(std::min((cols + 255u) / 256u, 256u), 3), dim3(256), 0,
+                       s, (const T*)vs.win_max(), (const T*)vs.win_min(), gx, gy, gz,
+                       (uint32_t*)(total + 1));
 }
 
 // out(x, y, z) = max of in over [c - r, c + r] along AXIS (0 x, 1 y, 2 z), coordinates
@@ -628,8 +632,8 @@ int fill_slot(spr_ctx* c, VolSlot& vs, const void* src, bool src_on_device, int 
         const size_t nbricks = (size_t)nbx * nby * nbz;
         if (want_bounds && !vs.d_bricks) {
             realloc = true;
-            // one more entry: the volume's bounds
-            HIPCALL(c, hipMalloc(&vs.d_bricks, (nbricks + 1) * sizeof(BrickKey)));
+            // two more entries: the volume's bounds, the count of k_window_need
+            HIPCALL(c, hipMalloc(&vs.d_bricks, (nbricks + 2) * sizeof(BrickKey)));
         }
         // the 4x4x4 block bounds live from the padding pass to the windows' only
         void* blocks = nullptr;
@@ -639,8 +643,12 @@ int fill_slot(spr_ctx* c, VolSlot& vs, const void* src, bool src_on_device, int 
                                   blocks);
         if (want_bounds) {
             BrickKey* total = vs.d_bricks + nbricks;
-            BrickKey t{};
+            struct {
+                BrickKey keys;
+                uint32_t needed, pad;
+            } t{};
             if (e == hipSuccess) e = hipMemsetAsync(total, 0xFF, sizeof(BrickKey), c->stream);
+            if (e == hipSuccess) e = hipMemsetAsync(total + 1, 0, sizeof(BrickKey), c->stream);
             if (e == hipSuccess) {
                 switch (dtype) {
                     case SPR_DTYPE_F32: launch_windows<float>(vs, blocks, total, c->stream); break;
@@ -653,8 +661,10 @@ int fill_slot(spr_ctx* c, VolSlot& vs, const void* src, bool src_on_device, int 
             if (e == hipSuccess)
                 e = hipMemcpyAsync(&t, total, sizeof(t), hipMemcpyDeviceToHost, c->stream);
             if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-            vs.vmin = dtype == SPR_DTYPE_F32 ? key_value<float>(t.kmin) : (float)t.kmin;
-            vs.vmax = dtype == SPR_DTYPE_F32 ? key_value<float>(~t.nkmax) : (float)~t.nkmax;
+            const BrickKey k = t.keys;
+            vs.vmin = dtype == SPR_DTYPE_F32 ? key_value<float>(k.kmin) : (float)k.kmin;
+            vs.vmax = dtype == SPR_DTYPE_F32 ? key_value<float>(~k.nkmax) : (float)~k.nkmax;
+            vs.need = (float)t.needed / (3.0f * (float)win[0] * (float)win[1] * (float)win[2]);
         }
         HIPCALL(c, e);
     }

@@ -13,6 +13,7 @@
 #include <cstdint>
 
 #include "mip_staged.h"
+#include "mip_windows.h"
 #include "render_kernels.h"
 #include "split_rays.h"
 #include "spimrender.h"
@@ -39,6 +40,7 @@ struct VolSlot {
     // two planes, which follow the padded copy in its allocation
     uint32_t win[3] = {0, 0, 0};
     size_t win_bytes = 0;
+    float need = 1.0f;  // share of the windows a max projection has to sample (k_window_need)
     static size_t align256(size_t n) { return (n + 255) / 256 * 256; }
     void* win_max() const { return (char*)d_pad + align256(pad_bytes); }
     void* win_min() const { return (char*)win_max() + align256(win_bytes); }
@@ -98,6 +100,13 @@ PaddedVolume<T, POW2, WIDE> padded_volume(const VolSlot& s) {
     v.bricks.nby = s.nby;
     v.vmin = s.vmin;
     v.vmax = s.vmax;
+    v.win_max = s.win_bytes ? (const T*)s.win_max() : nullptr;
+    v.win_min = s.win_bytes ? (const T*)s.win_min() : nullptr;
+    v.win_gx = s.win[0];
+    v.win_gy = s.win[1];
+    v.wnx = 0.25f * v.fnx;
+    v.wny = 0.25f * v.fny;
+    v.wnz = 0.25f * v.fnz;
     return v;
 }
 

@@ -156,4 +156,30 @@ __global__ __launch_bounds__(256) void k_block_windows(const BlockBounds<T>* __r
     }
 }
 
+// Share of the windows that a max projection along the volume's axes would have to sample:
+// *count windows, over the columns of each axis (grid.y: axis), whose maximum exceeds three
+// quarters of the way from the minimum to the maximum of the column's best window.  1 for
+// white noise, 0.04-0.35 for blobs over camera noise.
+template <typename T>
+__global__ __launch_bounds__(256) void k_window_need(const T* __restrict__ wmax,
+                                                     const T* __restrict__ wmin, uint32_t gx,
+                                                     uint32_t gy, uint32_t gz,
+                                                     uint32_t* __restrict__ count) {
+    const uint32_t n[3] = {gx, gy, gz}, stride[3] = {1u, gx, gx * gy};
+    const uint32_t a = blockIdx.y, b = a == 0 ? 1u : 0u, c = a == 2 ? 1u : 2u;
+    uint32_t need = 0;
+    for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < n[b] * n[c]; i += gridDim.x * 256u) {
+        const uint32_t ic = i / n[b], first = (i - ic * n[b]) * stride[b] + ic * stride[c];
+        float level = 0.0f;
+        for (uint32_t k = 0; k < n[a]; ++k) {
+            const uint32_t o = first + k * stride[a];
+            level = fmaxf(level, 0.25f * (float)wmin[o] + 0.75f * (float)wmax[o]);
+        }
+        for (uint32_t k = 0; k < n[a]; ++k)
+            need += (float)wmax[first + k * stride[a]] > level ? 1u : 0u;
+    }
+    for (int off = 32; off > 0; off >>= 1) need += (uint32_t)__shfl_xor((int)need, off);
+    if ((threadIdx.x & 63u) == 0u) atomicAdd(count, need);
+}
+
 }  // namespace spr

@@ -181,6 +181,18 @@ struct PaddedVolume {
     float mx, my, mz;              // N - 1
     BrickGrid bricks;              // per-brick bounds (bricks.keys == nullptr: none)
     float vmin, vmax;              // the volume's minimum and maximum voxel
+    const T* win_max;              // window grid (brick_bounds.h): largest voxel per window,
+    const T* win_min;              // smallest (nullptr: none)
+    uint32_t win_gx, win_gy;       // windows per row, rows per plane
+    float wnx, wny, wnz;           // N / 4: the last window that a sample's corner starts
+
+    // entry of the window at block coordinates (wx, wy, wz), kept inside the grid
+    __device__ __forceinline__ uint32_t window(float wx, float wy, float wz) const {
+        const uint32_t bx = (uint32_t)__builtin_amdgcn_fmed3f(wx, 0.0f, wnx);
+        const uint32_t by = (uint32_t)__builtin_amdgcn_fmed3f(wy, 0.0f, wny);
+        const uint32_t bz = (uint32_t)__builtin_amdgcn_fmed3f(wz, 0.0f, wnz);
+        return __umul24(__umul24(bz, win_gy) + by, win_gx) + bx;
+    }
 
     // raw buffer resource over the padded volume (uniform: lives in SGPRs)
     __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc() const {

@@ -1,0 +1,92 @@
+"""GPU: the max projection gathered group by group by the window grid (the default where it
+pays) against the same frame with every sample taken from global memory (SPR_TUNE_SLAB_KB 0)
+and against the oracle, bit for bit."""
+import numpy as np
+import pytest
+
+import oracle
+from spimagine_amd import _lib, synth
+from spimagine_amd.utils import mat4_perspective, mat4_rotation, mat4_translate
+from spimagine_amd.volumerender.volumerender import render_matrices
+
+pytestmark = pytest.mark.gpu
+
+POSES = [np.dot(mat4_translate(0, 0, -3.4), mat4_rotation(.7, .3, 1, -.2)),
+         np.dot(mat4_translate(.2, -.1, -2.2), mat4_rotation(2.3, 1, .2, .5)),  # enters the volume
+         np.dot(mat4_translate(0, 0, -4.), mat4_rotation(0., 0, 1, 0))]  # along the axes
+BOXES = [(-1, 1, -1, 1, -1, 1), (-.7, .4, -1, .9, -.2, 1), (-1.6, 1.7, -1.2, 1, -1, 2.)]
+
+
+def volume(dtype, shape, seed):
+    amp, bg = {np.uint8: ((60., 200.), 6.), np.uint16: ((500., 3000.), 100.),
+               np.float32: ((.3, 1.), -.1)}[dtype]
+    return synth.blob_volume(shape, n_blobs=14, sigma=(2., 5.), amp=amp, background=bg,
+                             poisson=False, read_noise=.02 * amp[1], dtype=dtype, seed=seed)
+
+
+def render(torch, ctx, slot, p, W, H):
+    o = torch.full((2, H, W), -7., device="cuda")
+    s = torch.cuda.Stream()
+    ctx.render_slot(slot, p, _lib.METHOD_MAX_PROJECT, W, H, o[0].data_ptr(), o[1].data_ptr(),
+                    stream=s.cuda_stream)
+    s.synchronize()
+    return o.cpu().numpy()
+
+
+# steps: 4, 2 and 1 samples a group (0.6, 1.3 and 5 voxels a step), one box, segments without
+# samples (16 steps), long rays
+@pytest.mark.parametrize("dtype", [np.uint16, np.uint8, np.float32])
+@pytest.mark.parametrize("shape,steps", [((64, 64, 64), 112), ((60, 77, 50), 112),
+                                         ((64, 128, 32), 96), ((33, 90, 70), 18),
+                                         ((50, 40, 60), 16), ((30, 31, 29), 1700)])
+def test_windows_equal_every_sample(dtype, shape, steps):
+    import torch
+    ctx = _lib.Context(0)
+    W, H = 117, 75
+    vol = volume(dtype, shape, 5)
+    if dtype == np.float32:
+        vol[shape[0] // 2, shape[1] // 3] = np.nan
+        vol[shape[0] // 4, 2, 3] = np.inf
+    slot = ctx.volume_add(vol)
+    P = mat4_perspective(45, W / float(H), .1, 10)
+    for k, (M, box) in enumerate(zip(POSES, BOXES)):
+        iP, iM = render_matrices(M, P, shape[::-1], (1., 1., 1.5))
+        p = _lib.make_params(iP, iM, box, .02, 900. if dtype == np.uint16 else 150. if
+                             dtype == np.uint8 else .9, gamma=(1., .6, 1.)[k], max_steps=steps)
+        ctx.set_tuning("slab_kb", 19)
+        got = render(torch, ctx, slot, p, W, H)
+        ctx.set_tuning("slab_kb", 0)
+        np.testing.assert_array_equal(got, render(torch, ctx, slot, p, W, H), err_msg=str(k))
+        assert (got[1] > 0).sum() > 100
+
+
+def test_windows_against_the_oracle():
+    import torch
+    ctx = _lib.Context(0)
+    vol = volume(np.uint16, (80, 70, 96), 8)
+    W, H = 90, 66
+    iP, iM = render_matrices(POSES[0], mat4_perspective(45, W / float(H), .1, 10), (96, 70, 80))
+    p = _lib.make_params(iP, iM, (-1, 1, -1, 1, -1, 1), 100., 2500., max_steps=160)
+    got = render(torch, ctx, ctx.volume_add(vol), p, W, H)
+    out, alpha = oracle.max_project(vol, iP, iM, min_val=100., max_val=2500., max_steps=160,
+                                    width=W, height=H)
+    np.testing.assert_array_equal(got[0], out)
+    np.testing.assert_array_equal(got[1], alpha)
+
+
+def test_noise_is_staged():
+    """White noise leaves nothing to skip: the frame stays with the staged kernel, and equals
+    the gathered one's samples."""
+    import torch
+    rng = np.random.default_rng(3)
+    ctx = _lib.Context(0)
+    vol = rng.integers(0, 4000, (64, 60, 70)).astype(np.uint16)
+    W, H = 100, 90
+    iP, iM = render_matrices(POSES[1], mat4_perspective(45, W / float(H), .1, 10), (70, 60, 64))
+    for steps in (112, 24):
+        p = _lib.make_params(iP, iM, (-1, 1, -1, 1, -1, 1), 0., 4000., max_steps=steps)
+        slot = ctx.volume_add(vol)
+        ctx.set_tuning("slab_kb", 19)
+        got = render(torch, ctx, slot, p, W, H)
+        ctx.set_tuning("slab_kb", 0)
+        np.testing.assert_array_equal(got, render(torch, ctx, slot, p, W, H))

@@ -239,3 +239,36 @@ def test_opacity_normalisation_without_division():
     q1 = _fma32(_fma32(-den, q0, x), rcp, q0)
     q2 = _fma32(_fma32(-den, q1, x), rcp, q1)
     np.testing.assert_array_equal(q2.view(np.uint32), (x / den).astype(np.float32).view(np.uint32))
+
+
+def _sum_ahead(p, d, n):
+    """sum_ahead of csrc/mip_windows.h in numpy float32 (the fma exact in float64)."""
+    f = np.float32
+    a = (p + d).astype(f)
+    b = (a + d).astype(f)
+    c = (b + d).astype(f)
+    q = ((n - 3).astype(np.float64) * (c - b).astype(np.float64) + c.astype(np.float64)).astype(f)
+    same = (a.view(np.uint32) ^ q.view(np.uint32)) < 0x800000
+    return q, same & ((q.view(np.uint32) & 0x7FFFFF) != 0)
+
+
+def test_running_sums_in_one_step():
+    """n rounded additions p + d + d ... equal one step of the third increment while the sums
+    stay inside a binade: random and few-bit steps (ties), sums that end at a power of two."""
+    rng = np.random.default_rng(0)
+    m = 400000
+    p = rng.uniform(-.1, 1.1, m).astype(np.float32)
+    p[::3] = (rng.integers(1, 2048, p[::3].size) / 2048.).astype(np.float32)
+    d = (rng.uniform(-1, 1, m) * 2. ** -rng.integers(1, 14, m)).astype(np.float32)
+    u = d.view(np.uint32)
+    u[::2] &= ~((1 << rng.integers(0, 20, u[::2].size)) - 1).astype(np.uint32)
+    for n in (8, 32, 200):
+        q = p.copy()
+        for _ in range(n):
+            q = q + d
+        got, same = _sum_ahead(p, d, np.full(m, n))
+        assert same.mean() > .1
+        np.testing.assert_array_equal(got[same].view(np.uint32), q[same].view(np.uint32))
+    # one that ends a little below 1/4 on the finer grid: not taken in one step
+    p, d = np.float32([float.fromhex("0x1.0a6p-2")]), np.float32([float.fromhex("-0x1.4c028ep-12")])
+    assert not _sum_ahead(p, d, np.full(1, 32))[1][0]
