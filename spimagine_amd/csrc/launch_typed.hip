@@ -329,6 +329,19 @@ void launch_windows(int gs, const PaddedVolume<T, P2, WIDE>& v, const RayParams&
 }
 
 template <typename T, bool P2>
+hipError_t TypedLaunch<T, P2>::windows_batch(int gs, const BatchJob* d_jobs, uint32_t njobs,
+                                             dim3 g, bool mixed, const RayParams& p, hipStream_t s) {
+    const dim3 block(64 * kWinSegments);
+    if (gs == 4)
+        hipLaunchKernelGGL((k_mip_windows_batch<T, P2, 4>), g, block, 0, s, d_jobs, p, njobs, mixed);
+    else if (gs == 2)
+        hipLaunchKernelGGL((k_mip_windows_batch<T, P2, 2>), g, block, 0, s, d_jobs, p, njobs, mixed);
+    else
+        hipLaunchKernelGGL((k_mip_windows_batch<T, P2, 1>), g, block, 0, s, d_jobs, p, njobs, mixed);
+    return hipGetLastError();
+}
+
+template <typename T, bool P2>
 hipError_t TypedLaunch<T, P2>::max_project(const LaunchTuning& t, const VolSlot& vs, RayParams p,
                                            bool nearest, float* out, float* alpha, hipStream_t s) {
     const dim3 grid(tile_grid(p.tile_map, p.ntx, p.nty)), block(256);
@@ -360,8 +373,8 @@ hipError_t TypedLaunch<T, P2>::max_project(const LaunchTuning& t, const VolSlot&
     }
     // with the default tuning, frames that gain by it are gathered group by group
     const float step = (float)nmax / (16.0f * (float)p.nouter);
-    if (staged && skip && t.slab_kb == 19 && t.chunk == 0 && t.row_pad == 0 && t.wg_waves != 4 &&
-        t.tile_map == (int)kTileMapInterleaved && windows_pay(vs.need, step, 4u * p.ntiles)) {
+    if (staged && skip && windows_tuning(t) && windows_pay(vs.need, step, 4u * p.ntiles) &&
+        4u * tile_grid(kTileMapInterleaved, p.ntx, p.nty) <= kWinMaxGroups) {
         const int gs = windows_group(step);
         if (vs.pad_wide)
             launch_windows(gs, padded_volume<T, P2, true>(vs), p, out, alpha, s);

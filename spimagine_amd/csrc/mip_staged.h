@@ -1276,8 +1276,10 @@ static __global__ __launch_bounds__(512) void k_tile_order(const uint32_t* __res
 // Pixel of this thread in a one-wave workgroup: an 8x8 quarter of a 16x16 tile.  Tile
 // rows are dealt to the XCDs as kTileMapInterleaved, the four quarters of a tile to
 // consecutive workgroups of its XCD; kTileMapCostXcd: item p.order[b] = 4 tile + quarter.
-__device__ __forceinline__ bool wave_tile_pixel(const RayParams& p, uint32_t* x, uint32_t* y) {
-    const uint32_t b = blockIdx.x, lane = threadIdx.x & 63u;
+// b: the workgroup's number within the frame.
+__device__ __forceinline__ bool wave_tile_pixel(const RayParams& p, uint32_t b, uint32_t* x,
+                                                uint32_t* y) {
+    const uint32_t lane = threadIdx.x & 63u;
     uint32_t tx, ty, q;
     if (p.tile_map == kTileMapCostXcd) {
         const uint32_t e = p.order[b];  // >= 4 ntiles: a surplus workgroup (ty >= nty)
@@ -1305,7 +1307,7 @@ __global__ __launch_bounds__(64) void k_max_project_wave(PaddedVolume<T, POW2, W
                                                          float* __restrict__ alpha) {
     __shared__ Unit16 lds[SLAB_BYTES / 16 + 1];  // +16 B: lds_pair reads past a pair
     uint32_t x = 0, y = 0;
-    const bool inside = wave_tile_pixel(p, &x, &y);
+    const bool inside = wave_tile_pixel(p, blockIdx.x, &x, &y);
     mip_staged_rays<T, POW2, SLAB_BYTES, CH, false, WIDE, OPAC, true, SKIP, FILT, FASTDIV>(
         vol, p, x, y, inside, reinterpret_cast<uint8_t*>(lds), nullptr, out, alpha);
 }
@@ -1399,7 +1401,7 @@ __global__ __launch_bounds__(WAVE ? 64 : 256) void k_iso_staged(PaddedVolume<T, 
     const uint32_t lane = threadIdx.x & 63u;
     uint8_t* slab = reinterpret_cast<uint8_t*>(lds) + (WAVE ? 0u : (threadIdx.x >> 6) * SLAB_BYTES);
     uint32_t x = 0, y = 0;
-    const bool inside = WAVE ? wave_tile_pixel(p, &x, &y) : tile_pixel(p, &x, &y);
+    const bool inside = WAVE ? wave_tile_pixel(p, blockIdx.x, &x, &y) : tile_pixel(p, &x, &y);
     const uint32_t o = x + p.W * y;
     F4 orig = mk4(0, 0, 0, 0), direc = mk4(0, 0, 0, 0), pos0 = mk4(0.5f, 0.5f, 0.5f, 0.0f),
        delta = mk4(0, 0, 0, 0);
@@ -1640,10 +1642,52 @@ __device__ __forceinline__ PaddedVolume<T, POW2> job_volume(const BatchJob& j) {
     v.bricks.keys = nullptr;  // batched frames sample every box
     v.bricks.nbx = v.bricks.nby = 0;
     v.vmin = v.vmax = 0.0f;
-    v.win_max = v.win_min = nullptr;
-    v.win_gx = v.win_gy = 0;
-    v.wnx = v.wny = v.wnz = 0.0f;
+    // the window grid follows the padded copy in its allocation (VolSlot)
+    v.win_max = reinterpret_cast<const T*>(static_cast<const uint8_t*>(j.base) +
+                                           (((size_t)j.nbytes + 255u) & ~(size_t)255u));
+    v.win_min = nullptr;
+    v.win_gx = win_entries((uint32_t)j.nx + 2u);
+    v.win_gy = win_entries((uint32_t)j.ny + 2u);
+    v.wnx = 0.25f * v.fnx;
+    v.wny = 0.25f * v.fny;
+    v.wnz = 0.25f * v.fnz;
     return v;
+}
+
+// the job whose items in queue q hold `item`: the last one whose first item is at most
+// `item` (jobs without items there share their successor's first)
+__device__ __forceinline__ uint32_t batch_job_of(const BatchJob* __restrict__ jobs, uint32_t njobs,
+                                                 uint32_t q, uint32_t item) {
+    uint32_t lo = 0, hi = njobs;
+    while (hi - lo > 1u) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (jobs[mid].first[q] <= item)
+            lo = mid;
+        else
+            hi = mid;
+    }
+    return lo;
+}
+
+// the launch's parameters with a job's own (mixed: size, box, transfer and steps as well)
+__device__ __forceinline__ void batch_params(RayParams& p, const BatchJob& j, bool mixed) {
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+        p.invP[k] = j.invP[k];
+        p.invM[k] = j.invM[k];
+    }
+    if (!mixed) return;
+    p.W = j.W;
+    p.H = j.H;
+    p.ntx = (j.W + 15u) / 16u;
+    p.nty = (j.H + 15u) / 16u;
+    p.ntiles = p.ntx * p.nty;
+#pragma unroll
+    for (int k = 0; k < 6; ++k) p.box[k] = j.box[k];
+    p.min_val = j.min_val;
+    p.max_val = j.max_val;
+    p.gamma = j.gamma;
+    p.nouter = j.nouter;
 }
 
 // zero the queue counters (a kernel, so the batch can be captured in a HIP graph)
@@ -1680,17 +1724,7 @@ __global__ __launch_bounds__(256) void k_max_project_batch(const BatchJob* __res
         }
         uint32_t jid, t;
         if (qs.mixed) {
-            // the job whose items of queue q hold `item`: the last one whose first item is
-            // at most `item` (jobs without items in queue q share their successor's first)
-            uint32_t lo = 0, hi = qs.njobs;
-            while (hi - lo > 1u) {
-                const uint32_t mid = (lo + hi) >> 1;
-                if (jobs[mid].first[q] <= item)
-                    lo = mid;
-                else
-                    hi = mid;
-            }
-            jid = lo;
+            jid = batch_job_of(jobs, qs.njobs, q, item);
             t = item - jobs[jid].first[q];
         } else {
             const uint32_t per = qs.tiles[q];
@@ -1699,24 +1733,7 @@ __global__ __launch_bounds__(256) void k_max_project_batch(const BatchJob* __res
         }
         const BatchJob& j = jobs[jid];
         RayParams p = shared;
-#pragma unroll
-        for (int k = 0; k < 16; ++k) {
-            p.invP[k] = j.invP[k];
-            p.invM[k] = j.invM[k];
-        }
-        if (qs.mixed) {
-            p.W = j.W;
-            p.H = j.H;
-            p.ntx = (j.W + 15u) / 16u;
-            p.nty = (j.H + 15u) / 16u;
-            p.ntiles = p.ntx * p.nty;
-#pragma unroll
-            for (int k = 0; k < 6; ++k) p.box[k] = j.box[k];
-            p.min_val = j.min_val;
-            p.max_val = j.max_val;
-            p.gamma = j.gamma;
-            p.nouter = j.nouter;
-        }
+        batch_params(p, j, qs.mixed != 0u);
         const uint32_t ty = q + 8u * (t / p.ntx), tx = t % p.ntx;
         uint32_t x, y;
         tile_thread_pixel(tx, ty, &x, &y);

@@ -124,6 +124,8 @@ struct WindowRay {
 // own (1024x1024x512 uint16 -> 1024^2, 1536 steps: 14.0 M gathers, address units busy 80%
 // of the frame, VALU 37%).
 constexpr int kWinSegments = 4;
+// workgroups of one grid dimension: a launch has fewer than 2^32 threads along it
+constexpr uint64_t kWinMaxGroups = (1ull << 32) / (64 * kWinSegments) - 1;
 
 // Samples per group for a step of at most `step` voxels along an axis: as many as one window
 // surely holds (WindowRay::ok; rays whose group spans more sample everything).
@@ -142,24 +144,26 @@ __host__ inline int windows_group(float step) {
 //   256^3 blobs, float (0.106): 448 steps 353 / 394, 102 steps 183 / 145
 //   512^3 white noise (1.0): 896 steps 956 / 2377, 204 steps 513 / 687
 //   200^2 frame of 128^3 float blobs (0.35), 200 steps: 76 / 55
-__host__ inline bool windows_pay(float need, float step, uint32_t tiles) {
+__host__ inline bool windows_pay(float need, float step, uint64_t tiles) {
     if (step >= 1.5f || tiles < 2048u) return need < 0.6f;
     return need < 0.09f;
 }
 
+struct WindowShared {
+    float4 item[kWinSegments][128];  // each wave's waiting groups: position, ray (w's bits)
+    float step[3][64];               // the rays' steps
+    uint32_t top[64];                // the rays' running maxima (bits of floats >= 0)
+};
+
 template <typename T, bool POW2, int GS, bool WIDE>
-__global__ __launch_bounds__(64 * kWinSegments) void k_mip_windows(
-    PaddedVolume<T, POW2, WIDE> vol, RayParams p, float* __restrict__ out, float* __restrict__ alpha) {
+__device__ __forceinline__ void mip_windows_rays(const PaddedVolume<T, POW2, WIDE>& vol,
+                                                 const RayParams& p, uint32_t x, uint32_t y,
+                                                 bool inside, float* __restrict__ out,
+                                                 float* __restrict__ alpha, WindowShared& sh) {
     using PV = PaddedVolume<T, POW2, WIDE>;
     constexpr bool kShort = !std::is_same<T, float>::value;
     constexpr int BS = kWinGroups * GS;
-    __shared__ float4 s_item[kWinSegments][128];  // waiting groups: position, ray (w's bits)
-    __shared__ float s_step[3][64];
-    __shared__ uint32_t s_max[64];  // the rays' running maxima (bits of floats >= 0)
     const uint32_t lane = threadIdx.x & 63u, seg = threadIdx.x >> 6;
-    if (gate_closed(p)) return;  // uniform over the launch
-    uint32_t x = 0, y = 0;
-    const bool inside = wave_tile_pixel(p, &x, &y);
     float px = 0.5f, py = 0.5f, pz = 0.5f, dx = 0.0f, dy = 0.0f, dz = 0.0f, tnear = 0.0f;
     const bool active = inside && staged_ray_pos(p, x, y, px, py, pz, dx, dy, dz, tnear);
     if (inside && !active && seg == 0) {
@@ -169,12 +173,12 @@ __global__ __launch_bounds__(64 * kWinSegments) void k_mip_windows(
     const uint64_t act = __ballot(active);
     if (act == 0) return;  // uniform over the workgroup: its waves have the same rays
     shadow_first_active(act, active, px, py, pz, dx, dy, dz);
-    float4* const item = s_item[seg];
+    float4* const item = sh.item[seg];
     if (seg == 0) {
-        s_max[lane] = 0u;
-        s_step[0][lane] = dx;
-        s_step[1][lane] = dy;
-        s_step[2][lane] = dz;
+        sh.top[lane] = 0u;
+        sh.step[0][lane] = dx;
+        sh.step[1][lane] = dy;
+        sh.step[2][lane] = dz;
     }
     __syncthreads();
     const int total = (p.nouter + 1) * kLoopUnroll;
@@ -194,7 +198,7 @@ __global__ __launch_bounds__(64 * kWinSegments) void k_mip_windows(
         float qx = sum_n(px, dx, (uint32_t)first), qy = sum_n(py, dy, (uint32_t)first),
               qz = sum_n(pz, dz, (uint32_t)first), c = 0.0f;
         staged_sample_global<PV, 2 * GS>(vol, qx, qy, qz, dx, dy, dz, c, op);
-        if (c > 0.0f) atomicMax(&s_max[lane], __float_as_uint(c));
+        if (c > 0.0f) atomicMax(&sh.top[lane], __float_as_uint(c));
     }
     __syncthreads();
     uint32_t waiting = 0;  // items in the queue (uniform)
@@ -207,9 +211,9 @@ __global__ __launch_bounds__(64 * kWinSegments) void k_mip_windows(
             const float4 it = item[waiting + lane];
             const uint32_t ray = __float_as_uint(it.w);
             float qx = it.x, qy = it.y, qz = it.z, c = 0.0f;
-            staged_sample_global<PV, GS>(vol, qx, qy, qz, s_step[0][ray], s_step[1][ray],
-                                         s_step[2][ray], c, op);
-            if (c > 0.0f) atomicMax(&s_max[ray], __float_as_uint(c));
+            staged_sample_global<PV, GS>(vol, qx, qy, qz, sh.step[0][ray], sh.step[1][ray],
+                                         sh.step[2][ray], c, op);
+            if (c > 0.0f) atomicMax(&sh.top[ray], __float_as_uint(c));
         }
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         __builtin_amdgcn_wave_barrier();
@@ -228,7 +232,7 @@ __global__ __launch_bounds__(64 * kWinSegments) void k_mip_windows(
     for (int s = 0; s < count; s += BS) {
         if (s + BS < count) ask((float)kWinGroups, nxt);
         // (other waves may raise it meanwhile: a stale value only asks for more groups)
-        const float col = __uint_as_float(__hip_atomic_load(&s_max[lane], __ATOMIC_RELAXED,
+        const float col = __uint_as_float(__hip_atomic_load(&sh.top[lane], __ATOMIC_RELAXED,
                                                             __HIP_MEMORY_SCOPE_WORKGROUP));
 #pragma unroll
         for (int j = 0; j < kWinGroups; ++j) {
@@ -251,7 +255,38 @@ __global__ __launch_bounds__(64 * kWinSegments) void k_mip_windows(
     if (waiting) take(waiting);
     __syncthreads();
     if (active && seg == 0)
-        staged_ray_end<kShort>(p, x + p.W * y, __uint_as_float(s_max[lane]), tnear, out, alpha);
+        staged_ray_end<kShort>(p, x + p.W * y, __uint_as_float(sh.top[lane]), tnear, out, alpha);
+}
+
+template <typename T, bool POW2, int GS, bool WIDE>
+__global__ __launch_bounds__(64 * kWinSegments) void k_mip_windows(
+    PaddedVolume<T, POW2, WIDE> vol, RayParams p, float* __restrict__ out, float* __restrict__ alpha) {
+    __shared__ WindowShared sh;
+    if (gate_closed(p)) return;  // uniform over the launch
+    uint32_t x = 0, y = 0;
+    const bool inside = wave_tile_pixel(p, blockIdx.x, &x, &y);
+    mip_windows_rays<T, POW2, GS, WIDE>(vol, p, x, y, inside, out, alpha, sh);
+}
+
+// The frames of a batch (many volumes x poses, or frames of their own sizes and settings)
+// the same way, one launch.  Uniform batches: grid.y = job.  Mixed ones: job k's first
+// workgroup in jobs[k].first[0].  A workgroup per quarter instead of persistent ones
+// claiming tiles: the workgroups are short and hold 12 KB of LDS, so the next ones fill in.
+template <typename T, bool POW2, int GS>
+__global__ __launch_bounds__(64 * kWinSegments) void k_mip_windows_batch(
+    const BatchJob* __restrict__ jobs, RayParams shared, uint32_t njobs, bool mixed) {
+    __shared__ WindowShared sh;
+    uint32_t jid = blockIdx.y, b = blockIdx.x;
+    if (mixed) {
+        jid = batch_job_of(jobs, njobs, 0, b);
+        b -= jobs[jid].first[0];
+    }
+    const BatchJob& j = jobs[jid];
+    RayParams p = shared;
+    batch_params(p, j, mixed);
+    uint32_t x = 0, y = 0;
+    const bool inside = wave_tile_pixel(p, b, &x, &y);
+    mip_windows_rays<T, POW2, GS, false>(job_volume<T, POW2>(j), p, x, y, inside, j.out, j.alpha, sh);
 }
 
 }  // namespace spr

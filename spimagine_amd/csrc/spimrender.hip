@@ -72,8 +72,9 @@ struct spr_ctx {
     bool has_params = false;
     // w x h output buffers kept between spr_render calls (VolumeRenderer.buf*, reset_buffer)
     int w = 0, h = 0;
-    float *d_out = nullptr, *d_alpha = nullptr, *d_depth = nullptr, *d_normals = nullptr,
-          *d_occ = nullptr;
+    // (planes of the one allocation d_planes)
+    float *d_planes = nullptr, *d_out = nullptr, *d_alpha = nullptr, *d_depth = nullptr,
+          *d_normals = nullptr, *d_occ = nullptr;
     // iso post-pass scratch (buf_tmp, buf_tmp_vec), grown on demand
     float *d_tmp = nullptr, *d_tmp_vec = nullptr;
     size_t scratch_px = 0;
@@ -147,11 +148,8 @@ struct DeviceGuard {
 };
 
 void free_outputs(spr_ctx* c) {
-    float** bufs[] = {&c->d_out, &c->d_alpha, &c->d_depth, &c->d_normals, &c->d_occ};
-    for (float** b : bufs) {
-        if (*b) (void)hipFree(*b);
-        *b = nullptr;
-    }
+    if (c->d_planes) (void)hipFree(c->d_planes);
+    c->d_planes = c->d_out = c->d_alpha = c->d_depth = c->d_normals = c->d_occ = nullptr;
     c->w = c->h = 0;
 }
 
@@ -190,17 +188,16 @@ int no_volume(spr_ctx* c, int slot) {
 int ensure_outputs(spr_ctx* c, int w, int h) {
     if (c->w == w && c->h == h && c->d_out) return SPR_OK;
     free_outputs(c);
-    const size_t px = (size_t)w * (size_t)h;
-    HIPCALL(c, hipMalloc(&c->d_out, px * 4));
-    HIPCALL(c, hipMalloc(&c->d_alpha, px * 4));
-    HIPCALL(c, hipMalloc(&c->d_depth, px * 4));
-    HIPCALL(c, hipMalloc(&c->d_normals, px * 12));
-    HIPCALL(c, hipMalloc(&c->d_occ, px * 4));
-    HIPCALL(c, hipMemsetAsync(c->d_out, 0, px * 4, c->stream));
-    HIPCALL(c, hipMemsetAsync(c->d_alpha, 0, px * 4, c->stream));
-    HIPCALL(c, hipMemsetAsync(c->d_depth, 0, px * 4, c->stream));
-    HIPCALL(c, hipMemsetAsync(c->d_normals, 0, px * 12, c->stream));
-    HIPCALL(c, hipMemsetAsync(c->d_occ, 0, px * 4, c->stream));
+    // one allocation and one fill for the seven planes (normals hold three): each
+    // allocation is a driver call of 50-100 us, paid by a new size's first frame
+    const size_t plane = VolSlot::align256((size_t)w * (size_t)h * 4) / 4;
+    HIPCALL(c, hipMalloc(&c->d_planes, 7 * plane * 4));
+    c->d_out = c->d_planes;
+    c->d_alpha = c->d_out + plane;
+    c->d_depth = c->d_alpha + plane;
+    c->d_occ = c->d_depth + plane;
+    c->d_normals = c->d_occ + plane;
+    HIPCALL(c, hipMemsetAsync(c->d_planes, 0, 7 * plane * 4, c->stream));
     c->w = w;
     c->h = h;
     return SPR_OK;
@@ -296,12 +293,10 @@ int check_parts(spr_ctx* c, const spr_params& prm, int num_parts) {
     return SPR_OK;
 }
 
-// Calls f(TypedLaunch<T, P2>()) for the slot's voxel type; P2: the padded copy's texel rule
-// (every dimension a power of two; linear-layout slots without a padded copy use false).
+// Calls f(TypedLaunch<T, P2>()) for a voxel type and texel rule
 template <typename F>
-hipError_t visit_launch(const VolSlot& vs, F&& f) {
-    const bool p2 = (vs.layout == SPR_LAYOUT_PADDED || vs.pad_wide) && slot_pow2(vs);
-    switch (vs.dtype) {
+hipError_t visit_launch(int dtype, bool p2, F&& f) {
+    switch (dtype) {
         case SPR_DTYPE_F32:
             return p2 ? f(TypedLaunch<float, true>()) : f(TypedLaunch<float, false>());
         case SPR_DTYPE_U16:
@@ -309,6 +304,14 @@ hipError_t visit_launch(const VolSlot& vs, F&& f) {
         default:
             return p2 ? f(TypedLaunch<uint8_t, true>()) : f(TypedLaunch<uint8_t, false>());
     }
+}
+
+// The same for a slot; the padded copy's texel rule: every dimension a power of two
+// (linear-layout slots without a padded copy use false)
+template <typename F>
+hipError_t visit_launch(const VolSlot& vs, F&& f) {
+    return visit_launch(vs.dtype,
+                        (vs.layout == SPR_LAYOUT_PADDED || vs.pad_wide) && slot_pow2(vs), f);
 }
 
 // render(method, numParts, currentPart) into device buffers; the reference's launch
@@ -686,17 +689,20 @@ void launch_minmax(const void* data, size_t n, float* partial, int blocks, hipSt
 
 // ---------------------------------------------------------------------------------- batch
 
-// Converts the caller's jobs into device job records; checks that every slot is padded and
-// of one voxel type.  *pow2 = every volume's dimensions are powers of two.
+// What decides how a batch is marched: the voxel type and texel rule its jobs share, the
+// largest dimension, and the largest share of windows one of its volumes has to sample.
+struct BatchKind {
+    int dtype = -1;
+    bool pow2 = true;
+    int nmax = 1;
+    float need = 0.0f;
+};
+
 // Converts the caller's jobs into device job records in out[0 .. n-1]; checks that every
-// slot is padded and of one voxel type.  *pow2 = every volume's dimensions are powers of
-// two; *nmax = the largest volume dimension.
-int build_jobs_into(spr_ctx* c, const spr_job* jobs, int n, BatchJob* out, int* dtype, bool* pow2,
-                    int* nmax) {
+// slot is padded and of one voxel type.
+int build_jobs_into(spr_ctx* c, const spr_job* jobs, int n, BatchJob* out, BatchKind* kind) {
     if (!jobs || n <= 0) return fail(c, SPR_ERR_INVALID_ARG, "empty batch");
-    *dtype = -1;
-    *pow2 = true;
-    *nmax = 1;
+    *kind = BatchKind();
     for (int i = 0; i < n; ++i) {
         const VolSlot* vs = slot_of(c, jobs[i].slot);
         if (!vs) {
@@ -707,13 +713,14 @@ int build_jobs_into(spr_ctx* c, const spr_job* jobs, int n, BatchJob* out, int* 
         }
         if (vs->layout != SPR_LAYOUT_PADDED)
             return fail(c, SPR_ERR_INVALID_ARG, "job %d: batched rendering needs the padded layout", i);
-        if (*dtype >= 0 && vs->dtype != *dtype)
+        if (kind->dtype >= 0 && vs->dtype != kind->dtype)
             return fail(c, SPR_ERR_UNSUPPORTED_DTYPE, "job %d: mixed voxel types in one batch", i);
         if (!jobs[i].d_out || !jobs[i].d_alpha)
             return fail(c, SPR_ERR_INVALID_ARG, "job %d: NULL output", i);
-        *dtype = vs->dtype;
-        *pow2 = *pow2 && slot_pow2(*vs);
-        *nmax = std::max(*nmax, std::max(vs->nx, std::max(vs->ny, vs->nz)));
+        kind->dtype = vs->dtype;
+        kind->pow2 = kind->pow2 && slot_pow2(*vs);
+        kind->nmax = std::max(kind->nmax, std::max(vs->nx, std::max(vs->ny, vs->nz)));
+        kind->need = std::max(kind->need, vs->need);
         BatchJob& b = out[i];
         b = BatchJob{};
         b.base = vs->d_pad;
@@ -732,11 +739,10 @@ int build_jobs_into(spr_ctx* c, const spr_job* jobs, int n, BatchJob* out, int* 
     return SPR_OK;
 }
 
-int build_jobs(spr_ctx* c, const spr_job* jobs, int n, std::vector<BatchJob>& out, int* dtype,
-               bool* pow2, int* nmax) {
+int build_jobs(spr_ctx* c, const spr_job* jobs, int n, std::vector<BatchJob>& out, BatchKind* kind) {
     if (!jobs || n <= 0) return fail(c, SPR_ERR_INVALID_ARG, "empty batch");
     out.resize(n);
-    return build_jobs_into(c, jobs, n, out.data(), dtype, pow2, nmax);
+    return build_jobs_into(c, jobs, n, out.data(), kind);
 }
 
 // tile rows of a frame of nty tile rows that fall in queue k (rows k, k + 8, ...)
@@ -753,29 +759,46 @@ BatchQueues make_queues(const RayParams& p, int n) {
     return q;
 }
 
-// ch: samples per staged box (chunk_for of the batch's longest ray step)
-hipError_t dispatch_batch(const spr_ctx* c, const spr_params& prm, int dtype, bool pow2, int ch,
+// Whether a batch is gathered by the window grid: plain max projections with the default
+// tuning whose volumes gain by it (g: the launch, workgroups x frames; step: the longest ray
+// step in voxels)
+bool batch_windows(const spr_ctx* c, const spr_params& prm, const BatchKind& kind, uint64_t gx,
+                   uint64_t gy, float step) {
+    return prm.filter == SPR_FILTER_LINEAR && prm.alpha_pow == 0.0f && windows_tuning(c->tune) &&
+           gx <= kWinMaxGroups && gy <= 65535u && windows_pay(kind.need, step, gx * gy);
+}
+
+// A batch's launch: gathered by the window grid (windows: its grid, mixed: one row of every
+// frame's workgroups) or from the persistent queues (ch: samples per staged box)
+hipError_t dispatch_batch(const spr_ctx* c, const spr_params& prm, const BatchKind& kind, int ch,
                           const BatchJob* d_jobs, const RayParams& p, const BatchQueues& q,
-                          uint32_t* counters, hipStream_t s) {
+                          bool windows, dim3 g, float step, uint32_t* counters, hipStream_t s) {
     const LaunchTuning& t = c->tune;
     const bool nearest = prm.filter == SPR_FILTER_NEAREST;
+    if (windows)
+        return visit_launch(kind.dtype, kind.pow2, [&](auto L) {
+            return L.windows_batch(windows_group(step), d_jobs, q.njobs, g, q.mixed != 0u, p, s);
+        });
     // 0: staged max projection, 3: staged opacity mode (per-wave 19 KiB slabs), 1 / 2: every
     // sample from global memory (linear / nearest)
     const int mode = nearest ? 2
                      : t.slab_kb <= 0 ? 1
                      : prm.alpha_pow == 0.0f ? 0
                      : t.staging == 0 ? 3 : 1;
-    switch (dtype) {
-        case SPR_DTYPE_F32:
-            return pow2 ? TypedLaunch<float, true>::batch(t, mode, ch, d_jobs, p, q, counters, s)
-                        : TypedLaunch<float, false>::batch(t, mode, ch, d_jobs, p, q, counters, s);
-        case SPR_DTYPE_U16:
-            return pow2 ? TypedLaunch<uint16_t, true>::batch(t, mode, ch, d_jobs, p, q, counters, s)
-                        : TypedLaunch<uint16_t, false>::batch(t, mode, ch, d_jobs, p, q, counters, s);
-        default:
-            return pow2 ? TypedLaunch<uint8_t, true>::batch(t, mode, ch, d_jobs, p, q, counters, s)
-                        : TypedLaunch<uint8_t, false>::batch(t, mode, ch, d_jobs, p, q, counters, s);
-    }
+    return visit_launch(kind.dtype, kind.pow2, [&](auto L) {
+        return L.batch(t, mode, ch, d_jobs, p, q, counters, s);
+    });
+}
+
+// The same for a uniform batch (make_queues): frames of p.W x p.H with p.nouter blocks
+hipError_t dispatch_batch(const spr_ctx* c, const spr_params& prm, const BatchKind& kind,
+                          const BatchJob* d_jobs, const RayParams& p, const BatchQueues& q,
+                          uint32_t* counters, hipStream_t s) {
+    const uint32_t per = 4u * tile_grid(kTileMapInterleaved, p.ntx, p.nty);
+    const float step = (float)kind.nmax / (16.0f * (float)p.nouter);
+    return dispatch_batch(c, prm, kind, chunk_for(c->tune, p.nouter, kind.nmax), d_jobs, p, q,
+                          batch_windows(c, prm, kind, per, q.njobs, step), dim3(per, q.njobs), step,
+                          counters, s);
 }
 
 // Enqueues the copy of a batch's job table to d_jobs on stream s from pinned host memory
@@ -1292,9 +1315,8 @@ int spr_render_batch(spr_ctx* c, const spr_params* params, const spr_job* jobs, 
     rc = check_parts(c, prm, num_parts);
     if (rc) return rc;
     std::vector<BatchJob> host;
-    int dtype, nmax;
-    bool pow2;
-    rc = build_jobs(c, jobs, n, host, &dtype, &pow2, &nmax);
+    BatchKind kind;
+    rc = build_jobs(c, jobs, n, host, &kind);
     if (rc) return rc;
     DeviceGuard g(c->device);
     hipStream_t s = stream ? (hipStream_t)stream : c->stream;
@@ -1312,8 +1334,7 @@ int spr_render_batch(spr_ctx* c, const spr_params* params, const spr_job* jobs, 
     p.current_part = current_part;
     const BatchQueues q = make_queues(p, n);
     if (e == hipSuccess)
-        e = dispatch_batch(c, prm, dtype, pow2, chunk_for(c->tune, p.nouter, nmax), d_jobs, p, q,
-                           d_counters, s);
+        e = dispatch_batch(c, prm, kind, d_jobs, p, q, d_counters, s);
     (void)hipFreeAsync(buf, s);
     HIPCALL(c, e);
     return SPR_OK;
@@ -1325,7 +1346,7 @@ namespace {
 
 // The job table of a batch of frames of their own sizes and settings (first[] left 0).
 int frames_to_jobs(spr_ctx* c, const spr_frame* frames, int n, std::vector<BatchJob>& host,
-                   int* dtype, bool* pow2, int* nmax) {
+                   BatchKind* kind) {
     if (!frames || n <= 0) return fail(c, SPR_ERR_INVALID_ARG, "empty batch");
     std::vector<spr_job> jobs((size_t)n);
     for (int i = 0; i < n; ++i) {
@@ -1341,7 +1362,7 @@ int frames_to_jobs(spr_ctx* c, const spr_frame* frames, int n, std::vector<Batch
         jobs[i].d_out = f.d_out;
         jobs[i].d_alpha = f.d_alpha;
     }
-    const int rc = build_jobs(c, jobs.data(), n, host, dtype, pow2, nmax);
+    const int rc = build_jobs(c, jobs.data(), n, host, kind);
     if (rc) return rc;
     for (int i = 0; i < n; ++i) {
         const spr_frame& f = frames[i];
@@ -1367,14 +1388,15 @@ int spr_render_frames(spr_ctx* c, const spr_frame* frames, int n, float alpha_po
     if (filter != SPR_FILTER_LINEAR && filter != SPR_FILTER_NEAREST)
         return fail(c, SPR_ERR_INVALID_ARG, "unknown filter %d", filter);
     std::vector<BatchJob> host;
-    int dtype, nmax;
-    bool pow2;
-    int rc = frames_to_jobs(c, frames, n, host, &dtype, &pow2, &nmax);
+    BatchKind kind;
+    int rc = frames_to_jobs(c, frames, n, host, &kind);
     if (rc) return rc;
     // each frame's first item in each queue; the box length follows the frame with the
     // longest ray step
     BatchQueues q{};
     int ch = kLoopUnroll;
+    uint64_t groups = 0;
+    float step = 0.0f;
     for (int i = 0; i < n; ++i) {
         BatchJob& b = host[i];
         const uint32_t ntx = (b.W + 15u) / 16u, nty = (b.H + 15u) / 16u;
@@ -1382,7 +1404,10 @@ int spr_render_frames(spr_ctx* c, const spr_frame* frames, int n, float alpha_po
             b.first[k] = q.count[k];
             q.count[k] += queue_rows(nty, k) * ntx;
         }
-        ch = std::min(ch, chunk_for(c->tune, b.nouter, std::max(b.nx, std::max(b.ny, b.nz))));
+        const int nmax = std::max(b.nx, std::max(b.ny, b.nz));
+        ch = std::min(ch, chunk_for(c->tune, b.nouter, nmax));
+        groups += 4u * tile_grid(kTileMapInterleaved, ntx, nty);
+        step = std::max(step, (float)nmax / (16.0f * (float)b.nouter));
     }
     q.mixed = 1;
     q.njobs = (uint32_t)n;
@@ -1396,13 +1421,23 @@ int spr_render_frames(spr_ctx* c, const spr_frame* frames, int n, float alpha_po
     staged_tuning(c->tune, p);
     p.nouter = host[0].nouter;
     p.current_part = 0;
+    const bool windows = batch_windows(c, prm, kind, groups, 1, step);
+    if (windows) {  // each frame's first workgroup
+        uint32_t first = 0;
+        for (BatchJob& b : host) {
+            b.first[0] = first;
+            first += 4u * tile_grid(kTileMapInterleaved, (b.W + 15u) / 16u, (b.H + 15u) / 16u);
+        }
+    }
     const size_t jbytes = (size_t)n * sizeof(BatchJob);
     void* buf = nullptr;
     HIPCALL(c, hipMallocAsync(&buf, jbytes + 64, s));
     BatchJob* d_jobs = (BatchJob*)buf;
     uint32_t* d_counters = (uint32_t*)((char*)buf + jbytes);
     hipError_t e = stage_jobs(c, host.data(), jbytes, d_jobs, s);
-    if (e == hipSuccess) e = dispatch_batch(c, prm, dtype, pow2, ch, d_jobs, p, q, d_counters, s);
+    if (e == hipSuccess)
+        e = dispatch_batch(c, prm, kind, ch, d_jobs, p, q, windows, dim3((uint32_t)groups), step,
+                           d_counters, s);
     (void)hipFreeAsync(buf, s);
     HIPCALL(c, e);
     return SPR_OK;
@@ -1415,9 +1450,8 @@ int spr_render_frames_split(spr_ctx* c, const spr_frame* frames, int n, int seg,
     if (seg != 32 && seg != 64 && seg != 128)
         return fail(c, SPR_ERR_INVALID_ARG, "segment length %d (32, 64 or 128)", seg);
     std::vector<BatchJob> host;
-    int dtype, nmax;
-    bool pow2;
-    int rc = frames_to_jobs(c, frames, n, host, &dtype, &pow2, &nmax);
+    BatchKind kind;
+    int rc = frames_to_jobs(c, frames, n, host, &kind);
     if (rc) return rc;
     // job k's first work item (8 x 8 rays x one segment) and first pixel; staged in LDS
     // slabs (tuning slab_kb > 0) when every frame's ray step allows 16-sample boxes
@@ -1449,19 +1483,9 @@ int spr_render_frames_split(spr_ctx* c, const spr_frame* frames, int n, int seg,
     if (e == hipSuccess) {
         const uint32_t nj = (uint32_t)n, ni = (uint32_t)items, np = (uint32_t)pix;
         const uint32_t* gates = reinterpret_cast<const uint32_t*>(d_gates);
-        switch (dtype) {
-            case SPR_DTYPE_F32:
-                e = pow2 ? TypedLaunch<float, true>::split(seg, staged, d_jobs, nj, ni, np, base, gates, s)
-                         : TypedLaunch<float, false>::split(seg, staged, d_jobs, nj, ni, np, base, gates, s);
-                break;
-            case SPR_DTYPE_U16:
-                e = pow2 ? TypedLaunch<uint16_t, true>::split(seg, staged, d_jobs, nj, ni, np, base, gates, s)
-                         : TypedLaunch<uint16_t, false>::split(seg, staged, d_jobs, nj, ni, np, base, gates, s);
-                break;
-            default:
-                e = pow2 ? TypedLaunch<uint8_t, true>::split(seg, staged, d_jobs, nj, ni, np, base, gates, s)
-                         : TypedLaunch<uint8_t, false>::split(seg, staged, d_jobs, nj, ni, np, base, gates, s);
-        }
+        e = visit_launch(kind.dtype, kind.pow2, [&](auto L) {
+            return L.split(seg, staged, d_jobs, nj, ni, np, base, gates, s);
+        });
     }
     (void)hipFreeAsync(d_jobs, s);
     HIPCALL(c, e);
@@ -1486,9 +1510,8 @@ int spr_render_batch_noalloc(spr_ctx* c, const spr_params* params, const spr_job
     if (!c->d_scratch) return fail(c, SPR_ERR_HIP, "no device scratch for this context");
     // one call at a time: the host staging table and each device's scratch are shared
     std::lock_guard<std::mutex> lock(g_noalloc_mu);
-    int dtype, nmax;
-    bool pow2;
-    rc = build_jobs_into(c, jobs, n, g_noalloc_jobs, &dtype, &pow2, &nmax);
+    BatchKind kind;
+    rc = build_jobs_into(c, jobs, n, g_noalloc_jobs, &kind);
     if (rc) return rc;
     DeviceGuard g(c->device);
     hipStream_t s = stream ? (hipStream_t)stream : c->stream;
@@ -1501,7 +1524,7 @@ int spr_render_batch_noalloc(spr_ctx* c, const spr_params* params, const spr_job
     p.nouter = (prm.max_steps / num_parts) / kLoopUnroll;
     p.current_part = current_part;
     const BatchQueues q = make_queues(p, n);
-    HIPCALL(c, dispatch_batch(c, prm, dtype, pow2, chunk_for(c->tune, p.nouter, nmax), d_jobs, p, q, d_counters, s));
+    HIPCALL(c, dispatch_batch(c, prm, kind, d_jobs, p, q, d_counters, s));
     // blocking: the next call may overwrite the staging table and the scratch
     HIPCALL(c, hipStreamSynchronize(s));
     return SPR_OK;
@@ -1588,9 +1611,8 @@ int spr_batch_graph_create(spr_ctx* c, const spr_job* jobs, int n, int w, int h,
     int rc = check_frame(c, w, h);
     if (rc) return rc;
     std::vector<BatchJob> host;
-    int dtype, nmax;
-    bool pow2;
-    rc = build_jobs(c, jobs, n, host, &dtype, &pow2, &nmax);
+    BatchKind kind;
+    rc = build_jobs(c, jobs, n, host, &kind);
     if (rc) return rc;
     DeviceGuard g(c->device);
     spr_batch_graph* bg = new (std::nothrow) spr_batch_graph();
@@ -1598,8 +1620,8 @@ int spr_batch_graph_create(spr_ctx* c, const spr_job* jobs, int n, int w, int h,
     bg->n = n;
     bg->w = w;
     bg->h = h;
-    bg->dtype = dtype;
-    bg->pow2 = pow2;
+    bg->dtype = kind.dtype;
+    bg->pow2 = kind.pow2;
     record_refs(c, jobs, n, bg->refs);
     auto cleanup = [&](int code) {
         spr_batch_graph_destroy(c, bg);
@@ -1625,8 +1647,7 @@ int spr_batch_graph_create(spr_ctx* c, const spr_job* jobs, int n, int w, int h,
     hipError_t e2 = hipSuccess;
     if (e == hipSuccess) {
         // the box length follows the captured jobs' volumes (speed only, never results)
-        e2 = dispatch_batch(c, c->params, dtype, pow2, chunk_for(c->tune, p.nouter, nmax), bg->d_jobs, p, q,
-                            bg->d_counters, cs);
+        e2 = dispatch_batch(c, c->params, kind, bg->d_jobs, p, q, bg->d_counters, cs);
         e = hipStreamEndCapture(cs, &bg->graph);
     }
     (void)hipStreamDestroy(cs);
@@ -1644,19 +1665,18 @@ int spr_batch_graph_update(spr_ctx* c, spr_batch_graph* bg, const spr_job* jobs,
     if (!bg) return fail(c, SPR_ERR_INVALID_ARG, "NULL graph");
     if (n != bg->n) return fail(c, SPR_ERR_INVALID_ARG, "graph holds %d jobs, got %d", bg->n, n);
     std::vector<BatchJob> host;
-    int dtype, nmax;
-    bool pow2;
-    int rc = build_jobs(c, jobs, n, host, &dtype, &pow2, &nmax);
+    BatchKind kind;
+    int rc = build_jobs(c, jobs, n, host, &kind);
     if (rc) return rc;
-    if (dtype != bg->dtype)
+    if (kind.dtype != bg->dtype)
         return fail(c, SPR_ERR_UNSUPPORTED_DTYPE, "voxel type differs from the captured batch");
     // the captured kernel's texel rule (one fma for power-of-two dimensions, two roundings
     // otherwise) must match every new volume, or its samples would differ from single renders
-    if (pow2 != bg->pow2)
+    if (kind.pow2 != bg->pow2)
         return fail(c, SPR_ERR_INVALID_ARG,
                     "the captured batch's volumes %s power-of-two dimensions and the new ones %s "
                     "(capture a new graph)", bg->pow2 ? "all have" : "do not all have",
-                    pow2 ? "do" : "do not");
+                    kind.pow2 ? "do" : "do not");
     DeviceGuard g(c->device);
     if (bg->last_stream) HIPCALL(c, hipStreamSynchronize(bg->last_stream));
     HIPCALL(c, hipMemcpy(bg->d_jobs, host.data(), (size_t)n * sizeof(BatchJob),

@@ -26,20 +26,6 @@ namespace spr {
 // segments x 64 waves.
 constexpr int kSplitSegDefault = 64;
 
-// the job holding item `item` of a job table whose job k starts at jobs[k].first[which]
-__device__ __forceinline__ uint32_t split_job_of(const BatchJob* __restrict__ jobs,
-                                                 uint32_t njobs, uint32_t which, uint32_t item) {
-    uint32_t lo = 0, hi = njobs;
-    while (hi - lo > 1u) {
-        const uint32_t mid = (lo + hi) >> 1;
-        if (jobs[mid].first[which] <= item)
-            lo = mid;
-        else
-            hi = mid;
-    }
-    return lo;
-}
-
 // frame jid is left untouched when its gate is closed (gates == nullptr: every frame runs)
 __device__ __forceinline__ bool split_gated(const uint32_t* __restrict__ gates, uint32_t jid) {
     return gates != nullptr && gates[jid] == 0u;
@@ -74,7 +60,7 @@ static __global__ __launch_bounds__(256) void k_split_clear(const BatchJob* __re
                                                             const uint32_t* __restrict__ gates) {
     const uint32_t i = blockIdx.x * 256u + threadIdx.x;
     if (i >= npix) return;
-    const uint32_t jid = split_job_of(jobs, njobs, 1, i);
+    const uint32_t jid = batch_job_of(jobs, njobs, 1, i);
     if (split_gated(gates, jid)) return;
     const BatchJob& j = jobs[jid];
     j.out[i - j.first[1]] = 0.0f;
@@ -89,7 +75,7 @@ __global__ __launch_bounds__(256) void k_split_march(const BatchJob* __restrict_
                                                      const uint32_t* __restrict__ gates) {
     const uint32_t item = blockIdx.x * 4u + (threadIdx.x >> 6);
     if (item >= nitems) return;  // uniform per wave
-    const uint32_t jid = split_job_of(jobs, njobs, 0, item);
+    const uint32_t jid = batch_job_of(jobs, njobs, 0, item);
     if (split_gated(gates, jid)) return;
     const BatchJob& j = jobs[jid];
     const uint32_t total = (j.nouter + 1u) * (uint32_t)kLoopUnroll;
@@ -139,7 +125,7 @@ __global__ __launch_bounds__(64) void k_split_staged(const BatchJob* __restrict_
     __shared__ Unit16 lds[kSplitSlab / 16 + 1];  // +16 B: lds_pair reads past a pair
     const uint32_t item = blockIdx.x;
     if (item >= nitems) return;
-    const uint32_t jid = split_job_of(jobs, njobs, 0, item);
+    const uint32_t jid = batch_job_of(jobs, njobs, 0, item);
     if (split_gated(gates, jid)) return;  // uniform
     const BatchJob& j = jobs[jid];
     const uint32_t total = (j.nouter + 1u) * (uint32_t)kLoopUnroll;
@@ -182,7 +168,7 @@ __global__ __launch_bounds__(256) void k_split_finish(const BatchJob* __restrict
                                                       const uint32_t* __restrict__ gates) {
     const uint32_t i = blockIdx.x * 256u + threadIdx.x;
     if (i >= npix) return;
-    const uint32_t jid = split_job_of(jobs, njobs, 1, i);
+    const uint32_t jid = batch_job_of(jobs, njobs, 1, i);
     if (split_gated(gates, jid)) return;
     const BatchJob& j = jobs[jid];
     const uint32_t o = i - j.first[1];

@@ -117,6 +117,13 @@ inline int chunk_for(const LaunchTuning& t, int nouter, int nmax, bool mip = fal
                    : mip ? staged_chunk_mip(nouter, nmax) : staged_chunk(nouter, nmax);
 }
 
+// the default launch options: the ones under which a max projection may be gathered by the
+// window grid (windows_pay) instead of staged as they ask
+inline bool windows_tuning(const LaunchTuning& t) {
+    return t.skip != 0 && t.staging == 0 && t.slab_kb == 19 && t.chunk == 0 && t.row_pad == 0 &&
+           t.wg_waves != 4 && t.tile_map == (int)kTileMapInterleaved;
+}
+
 // the staged kernels' launch options carried in RayParams
 inline void staged_tuning(const LaunchTuning& t, RayParams& p) {
     p.row_pad = (uint32_t)t.row_pad;
@@ -148,6 +155,10 @@ struct TypedLaunch {
     static hipError_t batch(const LaunchTuning& t, int mode, int ch, const BatchJob* d_jobs,
                             const RayParams& p, const BatchQueues& q, uint32_t* counters,
                             hipStream_t s);
+    // the frames of a batch gathered by the window grid, gs samples a group (g: workgroups
+    // a frame x frames, or mixed: every frame's workgroups, job k's first in first[0])
+    static hipError_t windows_batch(int gs, const BatchJob* d_jobs, uint32_t njobs, dim3 g,
+                                    bool mixed, const RayParams& p, hipStream_t s);
     // max projections of frames of scattered rays, each ray's samples split into segments
     // of seg (32, 64 or 128) samples (split_rays.h), staged in LDS slabs or gathered from
     // global memory; job k's first item and first pixel in first[0] and first[1]; base: the

@@ -90,3 +90,68 @@ def test_noise_is_staged():
         got = render(torch, ctx, slot, p, W, H)
         ctx.set_tuning("slab_kb", 0)
         np.testing.assert_array_equal(got, render(torch, ctx, slot, p, W, H))
+
+
+def test_batches_gathered_and_staged():
+    """A uniform batch and a mixed one by the window grid (the default for small frames),
+    from the persistent queues (SPR_TUNE_CHUNK 16), without allocation and as a graph: the
+    frames of each rendered alone, bit for bit."""
+    import torch
+    ctx = _lib.Context(0)
+    vols = [volume(np.uint16, s, k) for k, s in enumerate(((40, 50, 60), (33, 64, 41), (70, 30, 52)))]
+    slots = [ctx.volume_add(v) for v in vols]
+    W, H = 75, 93
+    sizes, ps, want = [], [], []
+    for k in range(7):
+        v = k % 3
+        w, h = (W, H) if k < 4 else (16 * k, 131 - 17 * k)
+        iP, iM = render_matrices(POSES[k % 3], mat4_perspective(45, w / float(h), .1, 10),
+                                 vols[v].shape[::-1])
+        p = _lib.make_params(iP, iM, BOXES[0 if k < 4 else k % 3], 50., 2000.,
+                             max_steps=96 if k < 4 else (16, 40, 200)[k % 3])
+        sizes.append((v, w, h))
+        ps.append(p)
+        want.append(render(torch, ctx, slots[v], p, w, h))
+    s = torch.cuda.Stream()
+
+    def check(launch, ks):
+        outs = [torch.full((2, sizes[k][2], sizes[k][1]), -9., device="cuda") for k in ks]
+        launch(outs, ks)
+        s.synchronize()
+        for o, k in zip(outs, ks):
+            np.testing.assert_array_equal(o.cpu().numpy(), want[k], err_msg=str(k))
+
+    def jobs(outs, ks):
+        return [(slots[sizes[k][0]], list(ps[k].inv_p), list(ps[k].inv_m), o[0].data_ptr(),
+                 o[1].data_ptr()) for o, k in zip(outs, ks)]
+
+    def batch(outs, ks):
+        ctx.render_batch(jobs(outs, ks), W, H, params=ps[0], stream=s.cuda_stream)
+
+    def noalloc(outs, ks):
+        ctx.render_batch_noalloc(jobs(outs, ks), W, H, params=ps[0], stream=s.cuda_stream)
+
+    def frames(outs, ks):
+        ctx.render_frames([_lib.make_frame(slots[sizes[k][0]], ps[k], sizes[k][1], sizes[k][2],
+                                           o[0].data_ptr(), o[1].data_ptr())
+                           for o, k in zip(outs, ks)], stream=s.cuda_stream)
+
+    def graph(outs, ks):
+        p = ps[0]
+        ctx.lib.spr_set_params(ctx.handle, p)
+        g = ctx.batch_graph(jobs(outs, ks), W, H)
+        for o in outs:  # replayed after other work on the outputs
+            g.launch(s.cuda_stream)
+            s.synchronize()
+            o.fill_(3.)
+            torch.cuda.synchronize()
+        g.launch(s.cuda_stream)
+        s.synchronize()
+        g.close()
+
+    for chunk in (0, 16):
+        ctx.set_tuning("chunk", chunk)
+        for f in (batch, noalloc, graph):
+            check(f, range(4))
+        check(frames, range(7))
+        check(frames, [6])
