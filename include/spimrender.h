@@ -100,19 +100,21 @@ extern "C" {
                       of a tile: a CU starts new work as soon as any of its waves ends),
                       4 (a 16x16 tile), 0 = default (1: faster at 1024^2 and 2048^2)
    SPR_TUNE_SKIP      1 = empty-space skipping and early ray termination by the volume's
-                      brick bounds (default), 0 = off.  Every padded one-channel volume
-                      keeps the minimum and maximum of each 8x8x8 brick (built on upload,
-                      8 bytes a brick).  With the default per-wave slabs (slab_kb 19) the
-                      max projection skips a 16-sample box
-                      whose bricks' maximum cannot exceed any of the wave's running maxima,
-                      the opacity mode stops a wave once no later sample can raise a ray's
-                      colour (cumsum x the volume's normalised maximum <= colour, with a
-                      transparency factor provably in [0, 1]), and the iso march skips a
-                      box whose bricks lie wholly on each marching ray's starting side of
-                      the iso value (after a skipped box, the next four tested as one
-                      while 63 steps span at most 40 voxels).  Only skipped samples'
-                      positions are still advanced, by the same additions: results are
-                      bit-identical either way. */
+                      bounds (default), 0 = off.  Every padded one-channel volume keeps the
+                      minimum and maximum of each 8x8x8 brick and of overlapping 8x8x8
+                      windows every 4 voxels (built on upload, 1/64 and 1/32 of its bytes
+                      for uint16 voxels).  With the other keys at their defaults, max
+                      projections (linear filter) of volumes whose windows leave enough to
+                      skip are gathered group by group, a group of 4, 2 or 1 samples only
+                      when its window exceeds the ray's running maximum, and the iso march
+                      samples a group only when its window reaches the other side of the
+                      iso value.  Otherwise, with the default per-wave slabs (slab_kb 19),
+                      the max projection skips a box whose bricks' maximum cannot exceed any
+                      of the wave's running maxima and the iso march a box whose bricks lie
+                      wholly on each marching ray's starting side; the opacity mode stops a
+                      wave once no later sample can raise a ray's colour (cumsum x the
+                      volume's normalised maximum <= colour, with a transparency factor
+                      provably in [0, 1]).  Results are bit-identical either way. */
 #define SPR_TUNE_TILE_MAP 0
 #define SPR_TUNE_SLAB_KB 1
 #define SPR_TUNE_STAGING 2

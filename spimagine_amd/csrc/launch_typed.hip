@@ -186,9 +186,7 @@ void launch_iso_wide(const VolSlot& vs, int ch, bool one_wave, dim3 grid, hipStr
                      const RayParams& p, float* out, float* alpha, float* depth, float* normals) {
     const PaddedVolume<T, P2, true> v = padded_volume<T, P2, true>(vs);
     const dim3 g1(4 * tile_grid(kTileMapInterleaved, p.ntx, p.nty));
-    if (one_wave && ch == 16 && SKIP && p.skip16 > 1)
-        hipLaunchKernelGGL((k_iso_staged<T, P2, kWaveSlab19, 16, true, SKIP, 0, true, true>), g1, dim3(64), 0, s, v, p, out, alpha, depth, normals);
-    else if (one_wave && ch == 16)
+    if (one_wave && ch == 16)
         hipLaunchKernelGGL((k_iso_staged<T, P2, kWaveSlab19, 16, true, SKIP, 0, true>), g1, dim3(64), 0, s, v, p, out, alpha, depth, normals);
     else if (one_wave && ch == 8)
         hipLaunchKernelGGL((k_iso_staged<T, P2, kWaveSlab19, 8, true, SKIP, 0, true>), g1, dim3(64), 0, s, v, p, out, alpha, depth, normals);
@@ -237,14 +235,12 @@ void launch_staged_opac(int ch, dim3 grid, hipStream_t s, Args... args) {
 }
 
 // the iso-surface march staged: per-wave slabs; one_wave: one wave per workgroup, grid 4 x
-// the interleaved tile grid (with coarse skip tests when p.skip16 asks for them)
+// the interleaved tile grid
 template <typename T, bool P2, bool SKIP, int FILT = 0, typename... Args>
 void launch_iso_staged(int ch, bool one_wave, dim3 grid, hipStream_t s, const RayParams& p,
                        Args... args) {
     const dim3 g1(4 * tile_grid(kTileMapInterleaved, p.ntx, p.nty));
-    if (one_wave && ch == 16 && SKIP && p.skip16 > 1)
-        hipLaunchKernelGGL((k_iso_staged<T, P2, kWaveSlab19, 16, false, SKIP, FILT, true, true>), g1, dim3(64), 0, s, args...);
-    else if (one_wave && ch == 16)
+    if (one_wave && ch == 16)
         hipLaunchKernelGGL((k_iso_staged<T, P2, kWaveSlab19, 16, false, SKIP, FILT, true>), g1, dim3(64), 0, s, args...);
     else if (one_wave && ch == 8)
         hipLaunchKernelGGL((k_iso_staged<T, P2, kWaveSlab19, 8, false, SKIP, FILT, true>), g1, dim3(64), 0, s, args...);
@@ -426,6 +422,19 @@ hipError_t TypedLaunch<T, P2>::max_project(const LaunchTuning& t, const VolSlot&
     return plain_max_project(vs, p, nearest, out, alpha, s);
 }
 
+// the iso march by the window grid
+template <typename T, bool P2, bool WIDE, int FILT>
+void launch_iso_windows(int gs, const PaddedVolume<T, P2, WIDE>& v, const RayParams& p, float* out,
+                        float* alpha, float* depth, float* normals, hipStream_t s) {
+    const dim3 g(4 * tile_grid(kTileMapInterleaved, p.ntx, p.nty)), block(64 * kWinSegments);
+    if (gs == 4)
+        hipLaunchKernelGGL((k_iso_windows<T, P2, 4, WIDE, FILT>), g, block, 0, s, v, p, out, alpha, depth, normals);
+    else if (gs == 2)
+        hipLaunchKernelGGL((k_iso_windows<T, P2, 2, WIDE, FILT>), g, block, 0, s, v, p, out, alpha, depth, normals);
+    else
+        hipLaunchKernelGGL((k_iso_windows<T, P2, 1, WIDE, FILT>), g, block, 0, s, v, p, out, alpha, depth, normals);
+}
+
 template <typename T, bool P2>
 hipError_t TypedLaunch<T, P2>::iso_march(const LaunchTuning& t, const VolSlot& vs, RayParams p,
                                          bool nearest, float* out, float* alpha, float* depth,
@@ -436,9 +445,22 @@ hipError_t TypedLaunch<T, P2>::iso_march(const LaunchTuning& t, const VolSlot& v
     const int nmax = std::max(vs.nx, std::max(vs.ny, vs.nz));
     const int ch = chunk_for(t, p.max_steps / kLoopUnroll, nmax);
     const bool skip = t.skip != 0 && vs.d_bricks != nullptr;
-    p.skip16 = iso_skip_chunks(ch, p.max_steps, nmax);
     // one wave per workgroup as for the max projection (interleaved tile maps)
     const bool one_wave = one_wave_for(t, p) && p.tile_map == kTileMapInterleaved;
+    // the default tuning: by the window grid
+    if (skip && windows_tuning(t) && p.max_steps <= kIsoWindowMaxSteps &&
+        4u * tile_grid(kTileMapInterleaved, p.ntx, p.nty) <= kWinMaxGroups) {
+        const int gs = windows_group((float)nmax / (float)(p.max_steps - 1));
+        if (vs.pad_wide && !nearest)
+            launch_iso_windows<T, P2, true, 0>(gs, padded_volume<T, P2, true>(vs), p, out, alpha, depth, normals, s);
+        else if (vs.layout == SPR_LAYOUT_PADDED && nearest)
+            launch_iso_windows<T, P2, false, 1>(gs, padded_volume<T, P2>(vs), p, out, alpha, depth, normals, s);
+        else if (vs.layout == SPR_LAYOUT_PADDED)
+            launch_iso_windows<T, P2, false, 0>(gs, padded_volume<T, P2>(vs), p, out, alpha, depth, normals, s);
+        else
+            return plain_iso_march(vs, p, nearest, out, alpha, depth, normals, s);
+        return hipGetLastError();
+    }
     if (staged_iso && vs.pad_wide) {
         skip ? launch_iso_wide<T, P2, true>(vs, ch, one_wave, grid, s, p, out, alpha, depth, normals)
              : launch_iso_wide<T, P2, false>(vs, ch, one_wave, grid, s, p, out, alpha, depth, normals);

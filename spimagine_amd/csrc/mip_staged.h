@@ -1381,11 +1381,10 @@ __device__ __forceinline__ void iso_march_chunk(const V& vol, const uint8_t* sla
 // ray can change side there: bricks' maximum <= iso for rays that start below or at the
 // iso value, bricks' minimum > iso for rays that start above it.
 // WAVE: one wave per workgroup (grid 4 x the interleaved tile grid, as k_max_project_wave),
-// else four waves, one 16x16 tile, per workgroup.  COARSE (SKIP, CH 16): the coarse skip
-// tests of p.skip16 chunks (a kernel of its own: compiled into the kernel and switched off,
-// they made 200-step frames 7% slower).
+// else four waves, one 16x16 tile, per workgroup.  (The default march is k_iso_windows,
+// mip_windows.h; this one runs with other launch options.)
 template <typename T, bool POW2, int SLAB_BYTES, int CH, bool WIDE = false, bool SKIP = false,
-          int FILT = 0, bool WAVE = false, bool COARSE = false>
+          int FILT = 0, bool WAVE = false>
 __global__ __launch_bounds__(WAVE ? 64 : 256) void k_iso_staged(PaddedVolume<T, POW2, WIDE> vol,
                                                                 RayParams p,
                                                                 float* __restrict__ out,
@@ -1426,12 +1425,6 @@ __global__ __launch_bounds__(WAVE ? 64 : 256) void k_iso_staged(PaddedVolume<T, 
     int gt = 0, ihit = 0;
     bool found = false;
     const int nsteps = p.max_steps;
-    // SKIP: after a skipped chunk the next p.skip16 chunks are first tested as one box (one
-    // box reduction and one brick query for all of them); after a failed test the chunks
-    // it covered are tested one by one, and a box over more bricks than one query takes
-    // ends the coarse tests of the wave
-    int coarse_from = 0;
-    bool last_skipped = false;
     for (int k0 = 0; k0 < nsteps; k0 += CH) {
         const bool march = active && !found;
         const uint64_t live = __ballot(march);
@@ -1442,44 +1435,6 @@ __global__ __launch_bounds__(WAVE ? 64 : 256) void k_iso_staged(PaddedVolume<T, 
         const float ex = __shfl(dx, src), ey = __shfl(dy, src), ez = __shfl(dz, src);
         float sx = march ? px : qx, sy_ = march ? py : qy, sz_ = march ? pz : qz;
         const float tx = march ? dx : ex, ty = march ? dy : ey, tz = march ? dz : ez;
-        if constexpr (SKIP && CH == 16 && COARSE) {
-            if (last_skipped && k0 >= coarse_from) {
-                const int NC = (int)p.skip16 * CH;
-                uint32_t c0, c1, c2;
-                staged_box_n<PV>(vol, march, 0.0f, (float)(NC - 1), sx, sy_, sz_, tx, ty, tz,
-                                 mgx, mgy, mgz, c0, c1, c2);
-                wave_min3_u16x2(c0, c1, c2);
-                BrickKey k;
-                bool cskip = false;
-                const bool queried =
-                    brick_load(vol, c0 & 0xFFFFu, c0 >> 16, c1 & 0xFFFFu, 0xFFFFu - (c1 >> 16),
-                               0xFFFFu - (c2 & 0xFFFFu), 0xFFFFu - (c2 >> 16), lane, k);
-                if (queried) {
-                    uint32_t unused = 0;
-                    wave_min3_u32(k.kmin, k.nkmax, unused);
-                    const float bmin = key_value<T>(k.kmin), bmax = key_value<T>(~k.nkmax);
-                    const float m = bound_margin<T>(bmin, bmax);
-                    const bool same_side = gt ? bmin - m > p.iso_val : bmax + m <= p.iso_val;
-                    cskip = __ballot(march && !same_side) == 0;
-                }
-                if (cskip) {
-#pragma unroll 4
-                    for (int j = 0; j < NC; ++j) {
-                        sx = sx + tx;
-                        sy_ = sy_ + ty;
-                        sz_ = sz_ + tz;
-                    }
-                    if (march) {
-                        px = sx;
-                        py = sy_;
-                        pz = sz_;
-                    }
-                    k0 += NC - CH;
-                    continue;
-                }
-                coarse_from = queried ? k0 + NC : nsteps;
-            }
-        }
         uint32_t b0, b1, b2;
         staged_box_n<PV>(vol, march, 0.0f, (float)(CH - 1), sx, sy_, sz_, tx, ty, tz, mgx, mgy,
                          mgz, b0, b1, b2);
@@ -1529,7 +1484,6 @@ __global__ __launch_bounds__(WAVE ? 64 : 256) void k_iso_staged(PaddedVolume<T, 
                                                      tx, ty, tz, k0, nsteps, p.iso_val, march, gt,
                                                      found, ihit);
         }
-        last_skipped = skip;
         if (march) {  // a marching lane's own position moves on
             px = sx;
             py = sy_;
@@ -1573,16 +1527,6 @@ __host__ inline int staged_chunk_mip(int nouter, int nmax) {
 __host__ inline uint32_t staged_groups_mip(int nouter, int nmax) {
     const float step = (float)nmax / (16.0f * (float)(nouter > 0 ? nouter : 1));
     return 31.0f * step <= 40.0f ? 2u : 1u;
-}
-
-// 16-sample chunks per coarse skip test of the staged iso march (RayParams::skip16): four
-// while 63 steps span at most 40 voxels, else none (1024^2 frames of a 512^3 volume: at
-// 896 steps four chunks a test made the iso frames 5% faster, 0.843 against 0.890 ms, and
-// eight 3%; at 200 steps, whose 64-sample boxes mostly cover more bricks than one query
-// takes, the tests cost 6%).
-__host__ inline uint32_t iso_skip_chunks(int ch, int max_steps, int nmax) {
-    const float step = (float)nmax / (float)(max_steps > 0 ? max_steps : 1);
-    return ch == 16 && 63.0f * step <= 40.0f ? 4u : 1u;
 }
 
 // ---------------------------------------------------------------------------------

@@ -41,7 +41,7 @@ __device__ __forceinline__ float sum_n(float p, float d, uint32_t n) {
         const float a = p + d, b = a + d, c = b + d;
         const float lo = __uint_as_float(__float_as_uint(a) & 0xFF800000u);  // its signed 2^e
         const float lim = (c > b) == (a > 0.0f) ? 2.0f * lo : lo;
-        const float m = floorf((lim - c) / (c - b)) - 1.0f;
+        const float m = floorf((lim - c) * __builtin_amdgcn_rcpf(c - b)) - 1.0f;
         q = sum_ahead(p, d, m + 3.0f, same);
         const bool far = m >= 1.0f && m + 3.0f < (float)n && same;
         p = far ? q : c;
@@ -57,6 +57,7 @@ constexpr int kWinGroups = 8;  // groups asked for together
 // are (wx + j gx, ...), in windows.
 template <typename V, int GS>
 struct WindowRay {
+    using T = typename V::value_type;
     float gx, gy, gz;  // advance of one group
     bool ok;           // a group's corners always lie in the one window
 
@@ -79,9 +80,17 @@ struct WindowRay {
         wy = fmaf(0.25f, texel<V::kPow2>(py, vol.fny) + (1.0f - mgy), fminf(kBack * gy, 0.0f));
         wz = fmaf(0.25f, texel<V::kPow2>(pz, vol.fnz) + (1.0f - mgz), fminf(kBack * gz, 0.0f));
     }
-    __device__ __forceinline__ typename V::value_type top(const V& vol, float wx, float wy,
-                                                          float wz) const {
-        return vol.win_max[vol.window(wx, wy, wz)];
+    // entries of the kWinGroups groups that start `ahead` groups past (px, py, pz)
+    __device__ __forceinline__ void ask(const V& vol, float px, float py, float pz, float mgx,
+                                        float mgy, float mgz, float ahead, const T* plane,
+                                        T (&u)[kWinGroups]) const {
+        float wx, wy, wz;
+        at(vol, px, py, pz, mgx, mgy, mgz, wx, wy, wz);
+#pragma unroll
+        for (int j = 0; j < kWinGroups; ++j) {
+            const float f = ahead + (float)j;
+            u[j] = plane[vol.window(fmaf(f, gx, wx), fmaf(f, gy, wy), fmaf(f, gz, wz))];
+        }
     }
     // first sample of the two groups most likely to hold the ray's maximum among `count`
     // samples from (px, py, pz) on: the largest bound among windows two groups apart
@@ -97,11 +106,11 @@ struct WindowRay {
         float top_u = -1.0f;
         int at = 0;
         for (int i = 0; i < probes; i += 16) {
-            typename V::value_type v[16];
+            T v[16];
 #pragma unroll
             for (int k = 0; k < 16; ++k) {
                 const float f = (float)min(i + k, probes - 1);
-                v[k] = top(vol, fmaf(f, sx, bx), fmaf(f, sy, by), fmaf(f, sz, bz));
+                v[k] = vol.win_max[vol.window(fmaf(f, sx, bx), fmaf(f, sy, by), fmaf(f, sz, bz))];
             }
 #pragma unroll
             for (int k = 0; k < 16; ++k) {
@@ -149,9 +158,33 @@ __host__ inline bool windows_pay(float need, float step, uint64_t tiles) {
     return need < 0.09f;
 }
 
+// the rays of a workgroup: which lanes have one, sample 0 and step
+struct SharedRays {
+    float pos[3][64], step[3][64];
+    uint64_t act;
+    __device__ __forceinline__ void put(uint32_t lane, uint64_t a, float px, float py, float pz,
+                                        float dx, float dy, float dz) {
+        pos[0][lane] = px;
+        pos[1][lane] = py;
+        pos[2][lane] = pz;
+        step[0][lane] = dx;
+        step[1][lane] = dy;
+        step[2][lane] = dz;
+        if (lane == 0) act = a;
+    }
+    __device__ __forceinline__ void get(uint32_t lane, float& px, float& py, float& pz, float& dx,
+                                        float& dy, float& dz) const {
+        px = pos[0][lane];
+        py = pos[1][lane];
+        pz = pos[2][lane];
+        dx = step[0][lane];
+        dy = step[1][lane];
+        dz = step[2][lane];
+    }
+};
 struct WindowShared {
     float4 item[kWinSegments][128];  // each wave's waiting groups: position, ray (w's bits)
-    float step[3][64];               // the rays' steps
+    SharedRays rays;
     uint32_t top[64];                // the rays' running maxima (bits of floats >= 0)
 };
 
@@ -164,23 +197,24 @@ __device__ __forceinline__ void mip_windows_rays(const PaddedVolume<T, POW2, WID
     constexpr bool kShort = !std::is_same<T, float>::value;
     constexpr int BS = kWinGroups * GS;
     const uint32_t lane = threadIdx.x & 63u, seg = threadIdx.x >> 6;
+    // one wave sets the rays up (~300 instructions, most of them divisions)
     float px = 0.5f, py = 0.5f, pz = 0.5f, dx = 0.0f, dy = 0.0f, dz = 0.0f, tnear = 0.0f;
-    const bool active = inside && staged_ray_pos(p, x, y, px, py, pz, dx, dy, dz, tnear);
-    if (inside && !active && seg == 0) {
-        out[x + p.W * y] = 0.0f;
-        alpha[x + p.W * y] = kShort ? 0.0f : -1.0f;
-    }
-    const uint64_t act = __ballot(active);
-    if (act == 0) return;  // uniform over the workgroup: its waves have the same rays
-    shadow_first_active(act, active, px, py, pz, dx, dy, dz);
-    float4* const item = sh.item[seg];
     if (seg == 0) {
+        const bool hits = inside && staged_ray_pos(p, x, y, px, py, pz, dx, dy, dz, tnear);
+        if (inside && !hits) {
+            out[x + p.W * y] = 0.0f;
+            alpha[x + p.W * y] = kShort ? 0.0f : -1.0f;
+        }
+        const uint64_t act = __ballot(hits);
+        if (act != 0) shadow_first_active(act, hits, px, py, pz, dx, dy, dz);
+        sh.rays.put(lane, act, px, py, pz, dx, dy, dz);
         sh.top[lane] = 0u;
-        sh.step[0][lane] = dx;
-        sh.step[1][lane] = dy;
-        sh.step[2][lane] = dz;
     }
     __syncthreads();
+    const bool active = (sh.rays.act >> lane & 1u) != 0;
+    if (sh.rays.act == 0) return;  // uniform over the workgroup
+    if (seg != 0) sh.rays.get(lane, px, py, pz, dx, dy, dz);
+    float4* const item = sh.item[seg];
     const int total = (p.nouter + 1) * kLoopUnroll;
     const int per = ((total + BS - 1) / BS + kWinSegments - 1) / kWinSegments * BS;
     const int s0 = min((int)seg * per, total);
@@ -211,26 +245,18 @@ __device__ __forceinline__ void mip_windows_rays(const PaddedVolume<T, POW2, WID
             const float4 it = item[waiting + lane];
             const uint32_t ray = __float_as_uint(it.w);
             float qx = it.x, qy = it.y, qz = it.z, c = 0.0f;
-            staged_sample_global<PV, GS>(vol, qx, qy, qz, sh.step[0][ray], sh.step[1][ray],
-                                         sh.step[2][ray], c, op);
+            staged_sample_global<PV, GS>(vol, qx, qy, qz, sh.rays.step[0][ray], sh.rays.step[1][ray],
+                                         sh.rays.step[2][ray], c, op);
             if (c > 0.0f) atomicMax(&sh.top[ray], __float_as_uint(c));
         }
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         __builtin_amdgcn_wave_barrier();
     };
     T cur[kWinGroups], nxt[kWinGroups];
-    auto ask = [&](float ahead, T (&u)[kWinGroups]) {
-        float wx, wy, wz;
-        win.at(vol, px, py, pz, mgx, mgy, mgz, wx, wy, wz);
-#pragma unroll
-        for (int j = 0; j < kWinGroups; ++j) {
-            const float f = ahead + (float)j;
-            u[j] = win.top(vol, fmaf(f, win.gx, wx), fmaf(f, win.gy, wy), fmaf(f, win.gz, wz));
-        }
-    };
-    if (count > 0) ask(0.0f, cur);
+    if (count > 0) win.ask(vol, px, py, pz, mgx, mgy, mgz, 0.0f, vol.win_max, cur);
     for (int s = 0; s < count; s += BS) {
-        if (s + BS < count) ask((float)kWinGroups, nxt);
+        if (s + BS < count)
+            win.ask(vol, px, py, pz, mgx, mgy, mgz, (float)kWinGroups, vol.win_max, nxt);
         // (other waves may raise it meanwhile: a stale value only asks for more groups)
         const float col = __uint_as_float(__hip_atomic_load(&sh.top[lane], __ATOMIC_RELAXED,
                                                             __HIP_MEMORY_SCOPE_WORKGROUP));
@@ -287,6 +313,181 @@ __global__ __launch_bounds__(64 * kWinSegments) void k_mip_windows_batch(
     uint32_t x = 0, y = 0;
     const bool inside = wave_tile_pixel(p, b, &x, &y);
     mip_windows_rays<T, POW2, GS, false>(job_volume<T, POW2>(j), p, x, y, inside, j.out, j.alpha, sh);
+}
+
+// Iso-surface march by the window grid (iso_kernel.cl:83-131, k_iso_surface): sample 0 sets a
+// ray's side, the first later sample on the other side is the crossing.  A group is sampled
+// only when its window reaches the other side of the iso value.  The four waves of an 8x8
+// quarter take every fourth run of kWinGroups groups, so they move front to back together
+// and stop together; waiting groups are queued and gathered 64 at a time as above, and a
+// crossing is posted as the least sample index.  The refinement, the gradient and the
+// shading then run per ray (iso_finish).
+//
+// Bound by VALU (65% busy; address units 40%): ~5 instructions a sample in windows on one
+// side, the rest in groups near surfaces, their exact positions and the finish.  512^3
+// uint16 -> 1024^2, 896 steps: 412 us; the staged march with 8^3 brick tests of a wave's box
+// 828 us (jumping every run to its exact position 454 us).
+struct IsoWindowShared {
+    float4 item[kWinSegments][128];  // position; w's bits: ray | side << 6 | first sample << 7
+    SharedRays rays;
+    uint64_t above;    // the rays that start above the iso value
+    uint32_t hit[64];  // the rays' least crossing sample (~0: none)
+};
+// Voxels that a window lookup allows for between a position estimated with one fma and the
+// running sum, kIsoAnchor samples from the last exact position: each addition is off by half
+// an ulp of at most 1/2, 3.0e-8 N voxels.
+constexpr float kIsoMargin = 3e-5f;
+constexpr uint32_t kIsoAnchor = 900;
+constexpr int kIsoWindowMaxSteps = 1 << 24;
+
+template <typename T, bool POW2, int GS, bool WIDE, int FILT>
+__global__ __launch_bounds__(64 * kWinSegments) void k_iso_windows(
+    PaddedVolume<T, POW2, WIDE> vol, RayParams p, float* __restrict__ out, float* __restrict__ alpha,
+    float* __restrict__ depth, float* __restrict__ normals) {
+    using PV = PaddedVolume<T, POW2, WIDE>;
+    static_assert(FILT == 0 || !WIDE, "nearest: volumes below 4 GiB");
+    constexpr int BS = kWinGroups * GS, RS = kWinSegments * BS;
+    __shared__ IsoWindowShared sh;
+    const uint32_t lane = threadIdx.x & 63u, seg = threadIdx.x >> 6;
+    uint32_t x = 0, y = 0;
+    const bool inside = wave_tile_pixel(p, blockIdx.x, &x, &y);
+    const uint32_t o = x + p.W * y;
+    F4 orig = mk4(0, 0, 0, 0), direc = mk4(0, 0, 0, 0), pos0 = mk4(0.5f, 0.5f, 0.5f, 0.0f),
+       delta = mk4(0, 0, 0, 0);
+    float tnear = 0.0f, tfar = 0.0f, dt = 0.0f;
+    float px = 0.5f, py = 0.5f, pz = 0.5f, dx = 0.0f, dy = 0.0f, dz = 0.0f;
+    if (seg == 0) {  // one wave sets the rays up and takes sample 0
+        bool hits = false;
+        if (inside) {
+            ray_setup(p.invP, p.invM, x, y, p.W, p.H, &orig, &direc);
+            hits = intersect_box(orig, direc, p.box, &tnear, &tfar);
+            if (hits) {
+                if (tnear < 0.0f) tnear = 0.0f;
+                dt = 1.0f * (tfar - tnear) / ((float)p.max_steps - 1.0f);
+                delta = scl4(0.5f * dt, direc);
+                pos0 = scl4(0.5f, add4(mk4(1.0f + orig.x, 1.0f + orig.y, 1.0f + orig.z,
+                                           1.0f + orig.w),
+                                       scl4(tnear, direc)));
+                px = pos0.x;
+                py = pos0.y;
+                pz = pos0.z;
+                dx = delta.x;
+                dy = delta.y;
+                dz = delta.z;
+            } else {
+                iso_miss(o, out, alpha, depth, normals);
+            }
+        }
+        const uint64_t act = __ballot(hits);
+        if (act != 0) shadow_first_active(act, hits, px, py, pz, dx, dy, dz);
+        sh.rays.put(lane, act, px, py, pz, dx, dy, dz);
+        sh.hit[lane] = 0xFFFFFFFFu;
+        const uint64_t above =
+            act != 0 ? __ballot(vol.template sample<FILT>(px, py, pz) > p.iso_val) : 0;
+        if (lane == 0) sh.above = above;
+    }
+    __syncthreads();
+    if (sh.rays.act == 0) return;  // uniform over the workgroup
+    const bool active = (sh.rays.act >> lane & 1u) != 0;
+    const bool gt = (sh.above >> lane & 1u) != 0;  // the ray's side
+    if (seg != 0) sh.rays.get(lane, px, py, pz, dx, dy, dz);
+    const float mgx = kIsoMargin * vol.fnx + 0.01f, mgy = kIsoMargin * vol.fny + 0.01f,
+                mgz = kIsoMargin * vol.fnz + 0.01f;
+    WindowRay<PV, GS> win;
+    win.begin(vol, dx, dy, dz, mgx, mgy, mgz);
+    const T* const plane = gt ? vol.win_min : vol.win_max;
+    float4* const item = sh.item[seg];
+    uint32_t waiting = 0;  // items in the queue (uniform)
+    auto take = [&](uint32_t n) {
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        waiting -= n;
+        if (lane < n) {
+            const float4 it = item[waiting + lane];
+            const uint32_t w = __float_as_uint(it.w), ray = w & 63u, k = w >> 7;
+            const int side = (int)(w >> 6 & 1u);
+            float qx = it.x, qy = it.y, qz = it.z, v[GS];
+            const float ex = sh.rays.step[0][ray], ey = sh.rays.step[1][ray], ez = sh.rays.step[2][ray];
+#pragma unroll
+            for (int j = 0; j < GS; ++j) {
+                v[j] = vol.template sample<FILT>(qx, qy, qz);
+                qx = qx + ex;
+                qy = qy + ey;
+                qz = qz + ez;
+            }
+            uint32_t first = 0xFFFFFFFFu;
+#pragma unroll
+            for (int j = GS - 1; j >= 0; --j)
+                if ((int)(v[j] > p.iso_val) != side) first = k + (uint32_t)j;
+            if (first < (uint32_t)p.max_steps) atomicMin(&sh.hit[ray], first);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    };
+    const uint32_t nsteps = (uint32_t)p.max_steps;
+    // (px, py, pz): the exact position of sample ka, a whole number of groups from k0 and at
+    // most kIsoAnchor samples before the last one asked for; a run without waiting groups
+    // moves only k0
+    uint32_t k0 = seg * (uint32_t)BS, ka = 0;
+    auto ask = [&](uint32_t k, T (&u)[kWinGroups]) {
+        win.ask(vol, px, py, pz, mgx, mgy, mgz, (float)((int)(k - ka) / GS), plane, u);
+    };
+    auto anchor = [&](uint32_t k) {
+        px = sum_n(px, dx, k - ka);
+        py = sum_n(py, dy, k - ka);
+        pz = sum_n(pz, dz, k - ka);
+        ka = k;
+    };
+    T cur[kWinGroups], nxt[kWinGroups];
+    ask(k0, cur);
+    for (; k0 < nsteps; k0 += (uint32_t)RS) {
+        const uint32_t hit = min(nsteps, __hip_atomic_load(&sh.hit[lane], __ATOMIC_RELAXED,
+                                                           __HIP_MEMORY_SCOPE_WORKGROUP));
+        if (__ballot(active && k0 < hit) == 0) break;  // every ray has crossed before
+        if (k0 + (uint32_t)(RS + BS) > ka + kIsoAnchor) anchor(k0);
+        ask(k0 + (uint32_t)RS, nxt);
+        uint32_t mask = 0, any = 0;  // groups that may cross: this ray's, some ray's (uniform)
+#pragma unroll
+        for (int j = 0; j < kWinGroups; ++j) {
+            const uint32_t k = k0 + (uint32_t)(j * GS);
+            const bool need = active && k < hit && (!win.ok || ((float)cur[j] > p.iso_val) != gt);
+            mask |= need ? 1u << j : 0u;
+            any |= __ballot(need) != 0 ? 1u << j : 0u;
+            cur[j] = nxt[j];
+        }
+        if (any == 0) continue;
+        const uint32_t first = (uint32_t)__builtin_ctz(any);
+        anchor(k0 + first * (uint32_t)GS);
+        float qx = px, qy = py, qz = pz;
+        for (uint32_t j = first; any >> j != 0u; ++j) {
+            if (any >> j & 1u) {
+                const bool need = (mask >> j & 1u) != 0;
+                const uint64_t m = __ballot(need);
+                if (need)
+                    item[waiting + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] =
+                        float4{qx, qy, qz,
+                               __uint_as_float(lane | (gt ? 64u : 0u) | (k0 + j * (uint32_t)GS) << 7)};
+                waiting += (uint32_t)__popcll(m);
+                if (waiting >= 64u) take(64u);
+            }
+#pragma unroll
+            for (int k = 0; k < GS; ++k) {
+                qx = qx + dx;
+                qy = qy + dy;
+                qz = qz + dz;
+            }
+        }
+        if (waiting) take(waiting);  // (a crossing found now saves the groups behind it)
+    }
+    __syncthreads();
+    if (!active || seg != 0) return;
+    const uint32_t hit = sh.hit[lane];
+    if (hit == 0xFFFFFFFFu) {
+        iso_miss(o, out, alpha, depth, normals);
+        return;
+    }
+    iso_finish<FILT>(vol, p, o, tnear, dt, delta, pos0, (int)hit, gt ? 1 : 0, direc, out, alpha,
+                     depth, normals);
 }
 
 }  // namespace spr

@@ -155,3 +155,41 @@ def test_batches_gathered_and_staged():
             check(f, range(4))
         check(frames, range(7))
         check(frames, [6])
+
+
+@pytest.mark.parametrize("dtype,filt", [(np.uint16, 0), (np.uint8, 0), (np.float32, 0),
+                                        (np.uint16, 1), (np.float32, 1)])
+@pytest.mark.parametrize("shape,steps", [((64, 64, 64), 150), ((60, 77, 50), 75), ((33, 90, 70), 17),
+                                         ((40, 41, 50), 2), ((30, 31, 29), 2100)])
+def test_iso_windows_equal_every_sample(dtype, filt, shape, steps):
+    """The iso surface by the window grid against the march with every sample from global
+    memory: all five outputs, from outside and inside the volume, iso values that the first
+    sample lies above and below, a NaN row, one and many runs of groups (4, 2 and 1 samples a
+    group; the least number of steps; more than one anchor along a ray)."""
+    import torch
+    ctx = _lib.Context(0)
+    W, H = 101, 83
+    vol = volume(dtype, shape, 6)
+    if dtype == np.float32:
+        vol[shape[0] // 2, shape[1] // 3] = np.nan
+    slot = ctx.volume_add(vol)
+    P = mat4_perspective(45, W / float(H), .1, 10)
+    top = float(np.nanmax(vol))
+    for k, (M, box) in enumerate(zip(POSES, BOXES)):
+        iP, iM = render_matrices(M, P, shape[::-1], (1., 1., 1.3))
+        for level in (.25, .02 if k else 1.6):
+            p = _lib.make_params(iP, iM, box, 0., top * level * 2, max_steps=steps, occ_radius=5,
+                                 filter=filt)
+            outs = {}
+            for slab in (19, 0):
+                ctx.set_tuning("slab_kb", slab)
+                o = [torch.full((H, W), -7., device="cuda") for _ in range(4)]
+                n = torch.full((H, W, 3), -7., device="cuda")
+                s = torch.cuda.Stream()
+                ctx.render_slot(slot, p, _lib.METHOD_ISO_SURFACE, W, H, o[0].data_ptr(),
+                                o[1].data_ptr(), o[2].data_ptr(), n.data_ptr(), o[3].data_ptr(),
+                                stream=s.cuda_stream)
+                s.synchronize()
+                outs[slab] = [t.cpu().numpy() for t in o + [n]]
+            for a, b in zip(outs[19], outs[0]):
+                np.testing.assert_array_equal(a, b, err_msg="pose %d level %g" % (k, level))
