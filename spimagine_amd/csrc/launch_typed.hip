@@ -326,14 +326,15 @@ void launch_windows(int gs, const PaddedVolume<T, P2, WIDE>& v, const RayParams&
 
 template <typename T, bool P2>
 hipError_t TypedLaunch<T, P2>::windows_batch(int gs, const BatchJob* d_jobs, uint32_t njobs,
-                                             dim3 g, bool mixed, const RayParams& p, hipStream_t s) {
+                                             dim3 g, bool mixed, const RayParams& p,
+                                             const uint32_t* gates, hipStream_t s) {
     const dim3 block(64 * kWinSegments);
     if (gs == 4)
-        hipLaunchKernelGGL((k_mip_windows_batch<T, P2, 4>), g, block, 0, s, d_jobs, p, njobs, mixed);
+        hipLaunchKernelGGL((k_mip_windows_batch<T, P2, 4>), g, block, 0, s, d_jobs, p, njobs, mixed, gates);
     else if (gs == 2)
-        hipLaunchKernelGGL((k_mip_windows_batch<T, P2, 2>), g, block, 0, s, d_jobs, p, njobs, mixed);
+        hipLaunchKernelGGL((k_mip_windows_batch<T, P2, 2>), g, block, 0, s, d_jobs, p, njobs, mixed, gates);
     else
-        hipLaunchKernelGGL((k_mip_windows_batch<T, P2, 1>), g, block, 0, s, d_jobs, p, njobs, mixed);
+        hipLaunchKernelGGL((k_mip_windows_batch<T, P2, 1>), g, block, 0, s, d_jobs, p, njobs, mixed, gates);
     return hipGetLastError();
 }
 

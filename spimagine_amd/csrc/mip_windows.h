@@ -298,15 +298,18 @@ __global__ __launch_bounds__(64 * kWinSegments) void k_mip_windows(
 // the same way, one launch.  Uniform batches: grid.y = job.  Mixed ones: job k's first
 // workgroup in jobs[k].first[0].  A workgroup per quarter instead of persistent ones
 // claiming tiles: the workgroups are short and hold 12 KB of LDS, so the next ones fill in.
+// gates: nullptr, or one device word per frame (0: the frame is left untouched).
 template <typename T, bool POW2, int GS>
 __global__ __launch_bounds__(64 * kWinSegments) void k_mip_windows_batch(
-    const BatchJob* __restrict__ jobs, RayParams shared, uint32_t njobs, bool mixed) {
+    const BatchJob* __restrict__ jobs, RayParams shared, uint32_t njobs, bool mixed,
+    const uint32_t* __restrict__ gates) {
     __shared__ WindowShared sh;
     uint32_t jid = blockIdx.y, b = blockIdx.x;
     if (mixed) {
         jid = batch_job_of(jobs, njobs, 0, b);
         b -= jobs[jid].first[0];
     }
+    if (gates != nullptr && gates[jid] == 0u) return;  // uniform: a closed frame
     const BatchJob& j = jobs[jid];
     RayParams p = shared;
     batch_params(p, j, mixed);

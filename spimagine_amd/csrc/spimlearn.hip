@@ -684,19 +684,24 @@ __global__ __launch_bounds__(256) void k_wgrad_in(const float* __restrict__ x,
     if (tid < C) out[kInW + tid] = gs[1024 + tid];
 }
 
-// out[i] = the sum of the blocks' partial sums: 8 threads a value, each every eighth block in
-// order, then their sums in order (one thread a value read 512 x 37 KB in sequence, 120 us).
-__global__ __launch_bounds__(256) void k_reduce(const float* __restrict__ partial, int nblocks, int nw,
-                                                float* __restrict__ out) {
-    __shared__ float part[8][32];
+// out[i] = the sum of the blocks' partial sums: 32 threads a value, each every 32nd block in
+// order, then their sums in order (one thread a value took 120 us for 512 x 37 KB, eight 20).
+constexpr int kReduceSlices = 32;
+
+__global__ __launch_bounds__(32 * kReduceSlices) void k_reduce(const float* __restrict__ partial,
+                                                               int nblocks, int nw,
+                                                               float* __restrict__ out) {
+    __shared__ float part[kReduceSlices][32];
     const int c = threadIdx.x & 31, k = threadIdx.x >> 5, i = blockIdx.x * 32 + c;
     float s = 0.0f;
-    if (i < nw)
-        for (int b = k; b < nblocks; b += 8) s += partial[(size_t)b * nw + i];
+    if (i < nw) {
+#pragma unroll 16
+        for (int b = k; b < nblocks; b += kReduceSlices) s += partial[(size_t)b * nw + i];
+    }
     part[k][c] = s;
     __syncthreads();
     if (k != 0 || i >= nw) return;
-    for (int j = 1; j < 8; ++j) s += part[j][c];
+    for (int j = 1; j < kReduceSlices; ++j) s += part[j][c];
     out[i] = s;
 }
 
@@ -971,7 +976,8 @@ inline int wgrad_blocks(int n, int h, int w) {
 }
 
 void wgrad_reduce(spl_net* t, int blocks, int nw, float* dst, hipStream_t s) {
-    hipLaunchKernelGGL(k_reduce, dim3((nw + 31) / 32), dim3(256), 0, s, t->wpart, blocks, nw, dst);
+    hipLaunchKernelGGL(k_reduce, dim3((nw + 31) / 32), dim3(32 * kReduceSlices), 0, s, t->wpart,
+                       blocks, nw, dst);
 }
 
 template <int COUT, bool MASK>
