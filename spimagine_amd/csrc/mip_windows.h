@@ -188,6 +188,57 @@ struct WindowShared {
     uint32_t top[64];                // the rays' running maxima (bits of floats >= 0)
 };
 
+// Samples of n >= 1 waiting groups, GS neighbouring lanes a group: batch b's lane takes sample
+// lane % GS of item b 64 / GS + lane / GS, at the position the reference's running sum gives
+// it (the lanes past the last item repeat it).  post(b, value, item's word).
+//
+// The samples of a group lie on one ray within ~3 voxels, so GS lanes mostly share the cache
+// lines that a lane taking the whole group would ask for one after the other.
+template <int FILT, int GS, typename PV, typename F>
+__device__ __forceinline__ void gather_groups(const PV& vol, const float4* item, uint32_t n,
+                                              uint32_t lane, const SharedRays& rays, F&& post) {
+    constexpr uint32_t IPB = 64u / GS;
+    float on[GS];  // on[k]: 1 in the lanes past sample k
+#pragma unroll
+    for (int k = 0; k < GS; ++k) on[k] = (int)(lane % GS) > k ? 1.0f : 0.0f;
+    auto value = [&](uint32_t b, uint32_t& w) {
+        const float4 it = item[min(b * IPB + lane / GS, n - 1u)];
+        w = __float_as_uint(it.w);
+        const uint32_t ray = w & 63u;
+        float qx = it.x, qy = it.y, qz = it.z;
+        const float ex = rays.step[0][ray], ey = rays.step[1][ray], ez = rays.step[2][ray];
+#pragma unroll
+        for (int k = 0; k + 1 < GS; ++k) {  // (fma(e, 1, q) is q + e, rounded once)
+            qx = fmaf(ex, on[k], qx);
+            qy = fmaf(ey, on[k], qy);
+            qz = fmaf(ez, on[k], qz);
+        }
+        return vol.template sample<FILT>(qx, qy, qz);
+    };
+    if (n == 64u) {
+        float v[GS];
+        uint32_t w[GS];
+#pragma unroll
+        for (int b = 0; b < GS; ++b) v[b] = value((uint32_t)b, w[b]);
+#pragma unroll
+        for (int b = 0; b < GS; ++b) post((uint32_t)b, v[b], w[b]);
+    } else {
+#pragma unroll 1
+        for (uint32_t b = 0; b * IPB < n; ++b) {
+            uint32_t w;
+            const float v = value(b, w);
+            post(b, v, w);
+        }
+    }
+}
+
+// the larger of a value and its neighbour's, 1 or 2 lanes away within each four
+template <int AWAY>
+__device__ __forceinline__ float max_quad(float v) {
+    constexpr int perm = AWAY == 1 ? 0xB1 : 0x4E;  // quad_perm [1,0,3,2], [2,3,0,1]
+    return fmaxf(v, __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(v), perm, 0xF, 0xF, true)));
+}
+
 template <typename T, bool POW2, int GS, bool WIDE>
 __device__ __forceinline__ void mip_windows_rays(const PaddedVolume<T, POW2, WIDE>& vol,
                                                  const RayParams& p, uint32_t x, uint32_t y,
@@ -241,14 +292,14 @@ __device__ __forceinline__ void mip_windows_rays(const PaddedVolume<T, POW2, WID
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         waiting -= n;
-        if (lane < n) {
-            const float4 it = item[waiting + lane];
-            const uint32_t ray = __float_as_uint(it.w);
-            float qx = it.x, qy = it.y, qz = it.z, c = 0.0f;
-            staged_sample_global<PV, GS>(vol, qx, qy, qz, sh.rays.step[0][ray], sh.rays.step[1][ray],
-                                         sh.rays.step[2][ray], c, op);
-            if (c > 0.0f) atomicMax(&sh.top[ray], __float_as_uint(c));
-        }
+        gather_groups<0, GS>(vol, item + waiting, n, lane, sh.rays,
+                             [&](uint32_t, float v, uint32_t ray) {
+                                 float c = fmaxf(v, 0.0f);
+                                 if constexpr (GS >= 2) c = max_quad<1>(c);
+                                 if constexpr (GS >= 4) c = max_quad<2>(c);
+                                 if (lane % GS == 0 && c > 0.0f)
+                                     atomicMax(&sh.top[ray], __float_as_uint(c));
+                             });
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         __builtin_amdgcn_wave_barrier();
     };
@@ -405,25 +456,13 @@ __global__ __launch_bounds__(64 * kWinSegments) void k_iso_windows(
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         waiting -= n;
-        if (lane < n) {
-            const float4 it = item[waiting + lane];
-            const uint32_t w = __float_as_uint(it.w), ray = w & 63u, k = w >> 7;
-            const int side = (int)(w >> 6 & 1u);
-            float qx = it.x, qy = it.y, qz = it.z, v[GS];
-            const float ex = sh.rays.step[0][ray], ey = sh.rays.step[1][ray], ez = sh.rays.step[2][ray];
-#pragma unroll
-            for (int j = 0; j < GS; ++j) {
-                v[j] = vol.template sample<FILT>(qx, qy, qz);
-                qx = qx + ex;
-                qy = qy + ey;
-                qz = qz + ez;
-            }
-            uint32_t first = 0xFFFFFFFFu;
-#pragma unroll
-            for (int j = GS - 1; j >= 0; --j)
-                if ((int)(v[j] > p.iso_val) != side) first = k + (uint32_t)j;
-            if (first < (uint32_t)p.max_steps) atomicMin(&sh.hit[ray], first);
-        }
+        gather_groups<FILT, GS>(vol, item + waiting, n, lane, sh.rays,
+                                [&](uint32_t, float v, uint32_t w) {
+                                    const uint32_t k = (w >> 7) + lane % GS;
+                                    if ((v > p.iso_val) != ((w >> 6 & 1u) != 0) &&
+                                        k < (uint32_t)p.max_steps)
+                                        atomicMin(&sh.hit[w & 63u], k);
+                                });
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         __builtin_amdgcn_wave_barrier();
     };
