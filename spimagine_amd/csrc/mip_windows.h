@@ -126,12 +126,13 @@ struct WindowRay {
 // One 8x8 pixel quarter of a 16x16 tile per workgroup; its kWinSegments waves march a
 // segment each of the rays' samples and share the running maxima.  No boxes are staged: a
 // wave puts the groups its rays still need into a queue in LDS, and whenever 64 are waiting
-// every lane takes one, gathers its samples from global memory and posts the maximum to
-// the ray's word, so no lane idles through groups that other rays need.
+// GS neighbouring lanes take one each round, gather its samples from global memory and post
+// the maximum to the ray's word, so no lane idles through groups that other rays need.
 //
-// Bound by the vector-memory path: ~40 of a gather's 64 lanes touch cache lines of their
-// own (1024x1024x512 uint16 -> 1024^2, 1536 steps: 14.0 M gathers, address units busy 80%
-// of the frame, VALU 37%).
+// Bound by the vector-memory path, in cache lines a gather touches: with a lane taking the
+// whole group ~40 of 64 lanes touched lines of their own.  1024x1024x512 uint16 -> 1024^2,
+// 1536 steps: 1144 us a lane a group, 849 us GS lanes a group; 2048x2048x512 -> 2048^2 5561
+// and 4657 us; 64 frames of 1024x1024x256 -> 1024^2 48.0 and 41.6 ms.
 constexpr int kWinSegments = 4;
 // workgroups of one grid dimension: a launch has fewer than 2^32 threads along it
 constexpr uint64_t kWinMaxGroups = (1ull << 32) / (64 * kWinSegments) - 1;
@@ -379,8 +380,8 @@ __global__ __launch_bounds__(64 * kWinSegments) void k_mip_windows_batch(
 //
 // Bound by VALU (65% busy; address units 40%): ~5 instructions a sample in windows on one
 // side, the rest in groups near surfaces, their exact positions and the finish.  512^3
-// uint16 -> 1024^2, 896 steps: 412 us; the staged march with 8^3 brick tests of a wave's box
-// 828 us (jumping every run to its exact position 454 us).
+// uint16 -> 1024^2, 896 steps: frame 477 us (511 us with a lane taking a whole group); march
+// of the frame 412 us before that, 828 us staged with 8^3 brick tests of a wave's box.
 struct IsoWindowShared {
     float4 item[kWinSegments][128];  // position; w's bits: ray | side << 6 | first sample << 7
     SharedRays rays;
