@@ -312,29 +312,35 @@ void launch_pair_ch(const VolSlot& vs, bool one_wave, dim3 grid, hipStream_t s, 
 
 #if SPR_PART != 1
 // the max projection gathered group by group where the window grid leaves something to gain
-template <typename T, bool P2, bool WIDE>
+template <int FILT, typename T, bool P2, bool WIDE>
 void launch_windows(int gs, const PaddedVolume<T, P2, WIDE>& v, const RayParams& p, float* out,
                     float* alpha, hipStream_t s) {
     const dim3 g(4 * tile_grid(kTileMapInterleaved, p.ntx, p.nty)), block(64 * kWinSegments);
     if (gs == 4)
-        hipLaunchKernelGGL((k_mip_windows<T, P2, 4, WIDE>), g, block, 0, s, v, p, out, alpha);
+        hipLaunchKernelGGL((k_mip_windows<T, P2, 4, WIDE, FILT>), g, block, 0, s, v, p, out, alpha);
     else if (gs == 2)
-        hipLaunchKernelGGL((k_mip_windows<T, P2, 2, WIDE>), g, block, 0, s, v, p, out, alpha);
+        hipLaunchKernelGGL((k_mip_windows<T, P2, 2, WIDE, FILT>), g, block, 0, s, v, p, out, alpha);
     else
-        hipLaunchKernelGGL((k_mip_windows<T, P2, 1, WIDE>), g, block, 0, s, v, p, out, alpha);
+        hipLaunchKernelGGL((k_mip_windows<T, P2, 1, WIDE, FILT>), g, block, 0, s, v, p, out, alpha);
+}
+
+template <typename T, bool P2, int FILT, typename... Args>
+void launch_windows_batch(int gs, dim3 g, hipStream_t s, Args... args) {
+    const dim3 block(64 * kWinSegments);
+    if (gs == 4)
+        hipLaunchKernelGGL((k_mip_windows_batch<T, P2, 4, FILT>), g, block, 0, s, args...);
+    else if (gs == 2)
+        hipLaunchKernelGGL((k_mip_windows_batch<T, P2, 2, FILT>), g, block, 0, s, args...);
+    else
+        hipLaunchKernelGGL((k_mip_windows_batch<T, P2, 1, FILT>), g, block, 0, s, args...);
 }
 
 template <typename T, bool P2>
-hipError_t TypedLaunch<T, P2>::windows_batch(int gs, const BatchJob* d_jobs, uint32_t njobs,
-                                             dim3 g, bool mixed, const RayParams& p,
+hipError_t TypedLaunch<T, P2>::windows_batch(int gs, bool nearest, const BatchJob* d_jobs,
+                                             uint32_t njobs, dim3 g, bool mixed, const RayParams& p,
                                              const uint32_t* gates, hipStream_t s) {
-    const dim3 block(64 * kWinSegments);
-    if (gs == 4)
-        hipLaunchKernelGGL((k_mip_windows_batch<T, P2, 4>), g, block, 0, s, d_jobs, p, njobs, mixed, gates);
-    else if (gs == 2)
-        hipLaunchKernelGGL((k_mip_windows_batch<T, P2, 2>), g, block, 0, s, d_jobs, p, njobs, mixed, gates);
-    else
-        hipLaunchKernelGGL((k_mip_windows_batch<T, P2, 1>), g, block, 0, s, d_jobs, p, njobs, mixed, gates);
+    nearest ? launch_windows_batch<T, P2, 1>(gs, g, s, d_jobs, p, njobs, mixed, gates)
+            : launch_windows_batch<T, P2, 0>(gs, g, s, d_jobs, p, njobs, mixed, gates);
     return hipGetLastError();
 }
 
@@ -352,6 +358,21 @@ hipError_t TypedLaunch<T, P2>::max_project(const LaunchTuning& t, const VolSlot&
                       (t.slab_kb == 19 || vs.pad_wide);
     // the plain max projection's box lengths (chunk 0: from the ray step)
     if (t.chunk == 0 && !opac) p.box16 = staged_groups_mip(p.nouter, nmax);
+    // with the default tuning, frames that gain by it are gathered group by group
+    const float step = (float)nmax / (16.0f * (float)p.nouter);
+    if (!opac && skip && windows_tuning(t) &&
+        windows_pay(nearest, vs.need, step, 4u * p.ntiles) &&
+        4u * tile_grid(kTileMapInterleaved, p.ntx, p.nty) <= kWinMaxGroups &&
+        (vs.layout == SPR_LAYOUT_PADDED || (vs.pad_wide && !nearest))) {
+        const int gs = windows_group(step);
+        if (vs.pad_wide && !nearest)
+            launch_windows<0>(gs, padded_volume<T, P2, true>(vs), p, out, alpha, s);
+        else if (nearest)
+            launch_windows<1>(gs, padded_volume<T, P2>(vs), p, out, alpha, s);
+        else
+            launch_windows<0>(gs, padded_volume<T, P2>(vs), p, out, alpha, s);
+        return hipGetLastError();
+    }
     // the nearest filter (plain or opacity mode) staged: padded slots below 4 GiB, per-wave
     // 19 KiB slabs, one wave per workgroup
     if (nearest && t.slab_kb > 0 && t.staging == 0 && vs.layout == SPR_LAYOUT_PADDED) {
@@ -367,17 +388,6 @@ hipError_t TypedLaunch<T, P2>::max_project(const LaunchTuning& t, const VolSlot&
         }
         if (obuf) (void)hipFreeAsync(obuf, s);
         return e;
-    }
-    // with the default tuning, frames that gain by it are gathered group by group
-    const float step = (float)nmax / (16.0f * (float)p.nouter);
-    if (staged && skip && windows_tuning(t) && windows_pay(vs.need, step, 4u * p.ntiles) &&
-        4u * tile_grid(kTileMapInterleaved, p.ntx, p.nty) <= kWinMaxGroups) {
-        const int gs = windows_group(step);
-        if (vs.pad_wide)
-            launch_windows(gs, padded_volume<T, P2, true>(vs), p, out, alpha, s);
-        else
-            launch_windows(gs, padded_volume<T, P2>(vs), p, out, alpha, s);
-        return hipGetLastError();
     }
     if ((staged || staged_opac) && vs.pad_wide) {
         const bool one_wave = one_wave_for(t, p);

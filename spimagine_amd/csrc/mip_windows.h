@@ -134,6 +134,14 @@ struct WindowRay {
 // 1536 steps: 1144 us a lane a group, 849 us GS lanes a group; 2048x2048x512 -> 2048^2 5561
 // and 4657 us; 64 frames of 1024x1024x256 -> 1024^2 48.0 and 41.6 ms.
 constexpr int kWinSegments = 4;
+// Waves per SIMD that the registers are held to (five: 96 of them).  Short marches wait on
+// one load after another and gain by a fifth wave; groups of four trilinear samples (32 loads
+// a lane in flight) and single float ones need the registers.  us with four / five waves,
+// 800^2 frames: nearest, 512^3 uint16 200 steps 146 / 111; linear, 256^3 uint16 200 steps
+// (2 a group) 197 / 178, 512^3 float 896 steps (4) 568 / 616, 200 steps (1) 251 / 257.
+template <typename T, int GS, int FILT>
+constexpr int kWinWaves =
+    FILT == 1 || GS == 2 || (GS == 1 && !std::is_same<T, float>::value) ? 5 : 4;
 // workgroups of one grid dimension: a launch has fewer than 2^32 threads along it
 constexpr uint64_t kWinMaxGroups = (1ull << 32) / (64 * kWinSegments) - 1;
 
@@ -145,18 +153,28 @@ __host__ inline int windows_group(float step) {
 
 // Whether the frame is gathered group by group (k_mip_windows) instead of staged box by box.
 // need: the volume's share of windows to sample (k_window_need); step: voxels a sample;
-// tiles: 8x8 pixel quarters.  Gathered samples cost 3-4 times staged ones at a fine step, so
-// most groups have to fall away there; from 1.5 voxels a step on a staged box holds few
-// samples of many voxels, and a frame of few rays leaves most of the GPU idle unless their
-// segments are marched side by side.  us staged / gathered, 800^2 frames:
-//   512^3 blobs, uint16 (need 0.044): 896 steps 864 / 715, 320 steps 566 / 353, 102 294 / 179
-//   256^3 blobs, uint16 (0.080): 448 steps 392 / 352, 102 steps 179 / 139
-//   256^3 blobs, float (0.106): 448 steps 353 / 394, 102 steps 183 / 145
-//   512^3 white noise (1.0): 896 steps 956 / 2377, 204 steps 513 / 687
-//   200^2 frame of 128^3 float blobs (0.35), 200 steps: 76 / 55
-__host__ inline bool windows_pay(float need, float step, uint64_t tiles) {
+// tiles: 8x8 pixel quarters.  Trilinear samples gathered cost ~1.5 times staged ones at a
+// fine step, so most groups have to fall away there; from 1.5 voxels a step on a staged box
+// holds few samples of many voxels, and a frame of few rays leaves most of the GPU idle
+// unless their segments are marched side by side.  A nearest sample is one load, cheaper
+// than its share of a staged box unless rays are short and leave little to skip.
+// us staged / gathered, 800^2 frames, linear:
+//   512^3 blobs, uint16 (need 0.044): 896 steps 760 / 530, 200 steps 386 / 202
+//   256^3 blobs, uint16 (0.078): 448 steps 357 / 303, 200 steps 226 / 178
+//   256^3 blobs, float (0.097): 448 steps 316 / 303, 200 steps 215 / 185
+//   256x256x128 blobs, uint16 (0.107): 384 steps 259 / 254, 200 steps 188 / 172
+//   256x256x128 blobs, float (0.141): 384 steps 225 / 250
+//   128^3 blobs, uint16 (0.28): 200 steps 189 / 212
+//   256^3 white noise, uint16 (1.0): 448 steps 401 / 534, 200 steps 248 / 300
+//   200^2 frames: 128^3 float blobs (0.42), 200 steps 79 / 43; 96^3 uint16 (0.32) 47 / 48
+// nearest:
+//   512^3 blobs, uint16: 896 steps 502 / 265, 200 steps 325 / 111
+//   256^3 white noise, uint16: 448 steps 247 / 234, 200 steps 176 / 145
+//   128^3 blobs, float (0.42): 224 steps 134 / 131, 200 steps 124 / 132
+__host__ inline bool windows_pay(bool nearest, float need, float step, uint64_t tiles) {
+    if (nearest) return need < 0.2f || step >= 1.25f || tiles < 2048u;
     if (step >= 1.5f || tiles < 2048u) return need < 0.6f;
-    return need < 0.09f;
+    return need < 0.11f;
 }
 
 // the rays of a workgroup: which lanes have one, sample 0 and step
@@ -240,7 +258,7 @@ __device__ __forceinline__ float max_quad(float v) {
     return fmaxf(v, __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(v), perm, 0xF, 0xF, true)));
 }
 
-template <typename T, bool POW2, int GS, bool WIDE>
+template <typename T, bool POW2, int GS, bool WIDE, int FILT>
 __device__ __forceinline__ void mip_windows_rays(const PaddedVolume<T, POW2, WIDE>& vol,
                                                  const RayParams& p, uint32_t x, uint32_t y,
                                                  bool inside, float* __restrict__ out,
@@ -279,11 +297,13 @@ __device__ __forceinline__ void mip_windows_rays(const PaddedVolume<T, POW2, WID
     Opacity op;  // (unused)
     WindowRay<PV, GS> win;
     win.begin(vol, dx, dy, dz, mgx, mgy, mgz);
+    T cur[kWinGroups], nxt[kWinGroups];
     if (count > 0) {
+        win.ask(vol, px, py, pz, mgx, mgy, mgz, 0.0f, vol.win_max, cur);
         const int first = win.best(vol, px, py, pz, count);
         float qx = sum_n(px, dx, (uint32_t)first), qy = sum_n(py, dy, (uint32_t)first),
               qz = sum_n(pz, dz, (uint32_t)first), c = 0.0f;
-        staged_sample_global<PV, 2 * GS>(vol, qx, qy, qz, dx, dy, dz, c, op);
+        staged_sample_global<PV, 2 * GS, false, FILT>(vol, qx, qy, qz, dx, dy, dz, c, op);
         if (c > 0.0f) atomicMax(&sh.top[lane], __float_as_uint(c));
     }
     __syncthreads();
@@ -293,8 +313,8 @@ __device__ __forceinline__ void mip_windows_rays(const PaddedVolume<T, POW2, WID
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         waiting -= n;
-        gather_groups<0, GS>(vol, item + waiting, n, lane, sh.rays,
-                             [&](uint32_t, float v, uint32_t ray) {
+        gather_groups<FILT, GS>(vol, item + waiting, n, lane, sh.rays,
+                                [&](uint32_t, float v, uint32_t ray) {
                                  float c = fmaxf(v, 0.0f);
                                  if constexpr (GS >= 2) c = max_quad<1>(c);
                                  if constexpr (GS >= 4) c = max_quad<2>(c);
@@ -304,8 +324,6 @@ __device__ __forceinline__ void mip_windows_rays(const PaddedVolume<T, POW2, WID
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         __builtin_amdgcn_wave_barrier();
     };
-    T cur[kWinGroups], nxt[kWinGroups];
-    if (count > 0) win.ask(vol, px, py, pz, mgx, mgy, mgz, 0.0f, vol.win_max, cur);
     for (int s = 0; s < count; s += BS) {
         if (s + BS < count)
             win.ask(vol, px, py, pz, mgx, mgy, mgz, (float)kWinGroups, vol.win_max, nxt);
@@ -336,14 +354,15 @@ __device__ __forceinline__ void mip_windows_rays(const PaddedVolume<T, POW2, WID
         staged_ray_end<kShort>(p, x + p.W * y, __uint_as_float(sh.top[lane]), tnear, out, alpha);
 }
 
-template <typename T, bool POW2, int GS, bool WIDE>
-__global__ __launch_bounds__(64 * kWinSegments) void k_mip_windows(
+template <typename T, bool POW2, int GS, bool WIDE, int FILT>
+__global__ __launch_bounds__(64 * kWinSegments, (kWinWaves<T, GS, FILT>)) void k_mip_windows(
     PaddedVolume<T, POW2, WIDE> vol, RayParams p, float* __restrict__ out, float* __restrict__ alpha) {
+    static_assert(FILT == 0 || !WIDE, "nearest: volumes below 4 GiB");
     __shared__ WindowShared sh;
     if (gate_closed(p)) return;  // uniform over the launch
     uint32_t x = 0, y = 0;
     const bool inside = wave_tile_pixel(p, blockIdx.x, &x, &y);
-    mip_windows_rays<T, POW2, GS, WIDE>(vol, p, x, y, inside, out, alpha, sh);
+    mip_windows_rays<T, POW2, GS, WIDE, FILT>(vol, p, x, y, inside, out, alpha, sh);
 }
 
 // The frames of a batch (many volumes x poses, or frames of their own sizes and settings)
@@ -351,8 +370,8 @@ __global__ __launch_bounds__(64 * kWinSegments) void k_mip_windows(
 // workgroup in jobs[k].first[0].  A workgroup per quarter instead of persistent ones
 // claiming tiles: the workgroups are short and hold 12 KB of LDS, so the next ones fill in.
 // gates: nullptr, or one device word per frame (0: the frame is left untouched).
-template <typename T, bool POW2, int GS>
-__global__ __launch_bounds__(64 * kWinSegments) void k_mip_windows_batch(
+template <typename T, bool POW2, int GS, int FILT>
+__global__ __launch_bounds__(64 * kWinSegments, (kWinWaves<T, GS, FILT>)) void k_mip_windows_batch(
     const BatchJob* __restrict__ jobs, RayParams shared, uint32_t njobs, bool mixed,
     const uint32_t* __restrict__ gates) {
     __shared__ WindowShared sh;
@@ -367,7 +386,8 @@ __global__ __launch_bounds__(64 * kWinSegments) void k_mip_windows_batch(
     batch_params(p, j, mixed);
     uint32_t x = 0, y = 0;
     const bool inside = wave_tile_pixel(p, b, &x, &y);
-    mip_windows_rays<T, POW2, GS, false>(job_volume<T, POW2>(j), p, x, y, inside, j.out, j.alpha, sh);
+    mip_windows_rays<T, POW2, GS, false, FILT>(job_volume<T, POW2>(j), p, x, y, inside, j.out, j.alpha,
+                                               sh);
 }
 
 // Iso-surface march by the window grid (iso_kernel.cl:83-131, k_iso_surface): sample 0 sets a

@@ -763,8 +763,9 @@ BatchQueues make_queues(const RayParams& p, int n) {
 // step in voxels)
 bool batch_windows(const spr_ctx* c, const spr_params& prm, const BatchKind& kind, uint64_t gx,
                    uint64_t gy, float step) {
-    return prm.filter == SPR_FILTER_LINEAR && prm.alpha_pow == 0.0f && windows_tuning(c->tune) &&
-           gx <= kWinMaxGroups && gy <= 65535u && windows_pay(kind.need, step, gx * gy);
+    return prm.alpha_pow == 0.0f && windows_tuning(c->tune) && gx <= kWinMaxGroups &&
+           gy <= 65535u &&
+           windows_pay(prm.filter == SPR_FILTER_NEAREST, kind.need, step, gx * gy);
 }
 
 // A batch's launch: gathered by the window grid (windows: its grid, mixed: one row of every
@@ -776,7 +777,8 @@ hipError_t dispatch_batch(const spr_ctx* c, const spr_params& prm, const BatchKi
     const bool nearest = prm.filter == SPR_FILTER_NEAREST;
     if (windows)
         return visit_launch(kind.dtype, kind.pow2, [&](auto L) {
-            return L.windows_batch(windows_group(step), d_jobs, q.njobs, g, q.mixed != 0u, p, nullptr, s);
+            return L.windows_batch(windows_group(step), nearest, d_jobs, q.njobs, g, q.mixed != 0u, p,
+                                   nullptr, s);
         });
     // 0: staged max projection, 3: staged opacity mode (per-wave 19 KiB slabs), 1 / 2: every
     // sample from global memory (linear / nearest)
@@ -1497,7 +1499,7 @@ int spr_render_frames_split(spr_ctx* c, const spr_frame* frames, int n, int seg,
         const uint32_t nj = (uint32_t)n, ni = (uint32_t)items, np = (uint32_t)pix;
         const uint32_t* gates = reinterpret_cast<const uint32_t*>(d_gates);
         e = visit_launch(kind.dtype, kind.pow2, [&](auto L) {
-            return windows ? L.windows_batch(windows_group(step), d_jobs, nj, dim3((uint32_t)groups),
+            return windows ? L.windows_batch(windows_group(step), false, d_jobs, nj, dim3((uint32_t)groups),
                                              true, base, gates, s)
                            : L.split(seg, staged, d_jobs, nj, ni, np, base, gates, s);
         });

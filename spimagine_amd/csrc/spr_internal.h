@@ -158,8 +158,8 @@ struct TypedLaunch {
     // the frames of a batch gathered by the window grid, gs samples a group (g: workgroups
     // a frame x frames, or mixed: every frame's workgroups, job k's first in first[0];
     // gates: nullptr or one device flag per job, 0: skip the job)
-    static hipError_t windows_batch(int gs, const BatchJob* d_jobs, uint32_t njobs, dim3 g,
-                                    bool mixed, const RayParams& p, const uint32_t* gates,
+    static hipError_t windows_batch(int gs, bool nearest, const BatchJob* d_jobs,
+                                    uint32_t njobs, dim3 g, bool mixed, const RayParams& p, const uint32_t* gates,
                                     hipStream_t s);
     // max projections of frames of scattered rays, each ray's samples split into segments
     // of seg (32, 64 or 128) samples (split_rays.h), staged in LDS slabs or gathered from

@@ -193,3 +193,42 @@ def test_iso_windows_equal_every_sample(dtype, filt, shape, steps):
                 outs[slab] = [t.cpu().numpy() for t in o + [n]]
             for a, b in zip(outs[19], outs[0]):
                 np.testing.assert_array_equal(a, b, err_msg="pose %d level %g" % (k, level))
+
+
+@pytest.mark.parametrize("dtype", [np.uint16, np.uint8, np.float32])
+@pytest.mark.parametrize("shape,steps", [((64, 64, 64), 112), ((60, 77, 50), 64),
+                                         ((33, 90, 70), 18), ((30, 31, 29), 1700)])
+def test_nearest_windows_equal_every_sample(dtype, shape, steps):
+    """The nearest filter by the window grid (4, 2 and 1 samples a group, long rays; a frame
+    alone, a uniform and a mixed batch) against every sample from global memory."""
+    import torch
+    ctx = _lib.Context(0)
+    W, H = 117, 75
+    vol = volume(dtype, shape, 7)
+    if dtype == np.float32:
+        vol[shape[0] // 2, shape[1] // 3] = np.nan
+        vol[shape[0] // 4, 2, 3] = np.inf
+    slot = ctx.volume_add(vol)
+    P = mat4_perspective(45, W / float(H), .1, 10)
+    for k, (M, box) in enumerate(zip(POSES, BOXES)):
+        iP, iM = render_matrices(M, P, shape[::-1], (1., 1., 1.5))
+        p = _lib.make_params(iP, iM, box, .02, 900. if dtype == np.uint16 else 150. if
+                             dtype == np.uint8 else .9, gamma=(1., .6, 1.)[k], max_steps=steps,
+                             filter=_lib.FILTER_NEAREST)
+        s = torch.cuda.Stream()
+        outs = []
+        for slab in (19, 0):
+            ctx.set_tuning("slab_kb", slab)
+            o = torch.full((3, 2, H, W), -7., device="cuda")
+            ctx.render_slot(slot, p, _lib.METHOD_MAX_PROJECT, W, H, o[0, 0].data_ptr(),
+                            o[0, 1].data_ptr(), stream=s.cuda_stream)
+            ctx.render_batch([(slot, list(iP), list(iM), o[1, 0].data_ptr(), o[1, 1].data_ptr())],
+                             W, H, params=p, stream=s.cuda_stream)
+            ctx.render_frames([_lib.make_frame(slot, p, W, H, o[2, 0].data_ptr(), o[2, 1].data_ptr())],
+                              stream=s.cuda_stream, filter=_lib.FILTER_NEAREST)
+            s.synchronize()
+            outs.append(o.cpu().numpy())
+        np.testing.assert_array_equal(outs[0], outs[1], err_msg=str(k))
+        assert (outs[0][:, 1] > 0).sum() > 300
+        np.testing.assert_array_equal(outs[0][0], outs[0][1])
+        np.testing.assert_array_equal(outs[0][0], outs[0][2])
