@@ -361,7 +361,7 @@ hipError_t TypedLaunch<T, P2>::max_project(const LaunchTuning& t, const VolSlot&
     // with the default tuning, frames that gain by it are gathered group by group
     const float step = (float)nmax / (16.0f * (float)p.nouter);
     if (!opac && skip && windows_tuning(t) &&
-        windows_pay(nearest, vs.need, step, 4u * p.ntiles) &&
+        windows_pay(nearest, vs.need, nmax, step, 4u * p.ntiles) &&
         4u * tile_grid(kTileMapInterleaved, p.ntx, p.nty) <= kWinMaxGroups &&
         (vs.layout == SPR_LAYOUT_PADDED || (vs.pad_wide && !nearest))) {
         const int gs = windows_group(step);

@@ -157,7 +157,8 @@ __host__ inline int windows_group(float step) {
 // fine step, so most groups have to fall away there; from 1.5 voxels a step on a staged box
 // holds few samples of many voxels, and a frame of few rays leaves most of the GPU idle
 // unless their segments are marched side by side.  A nearest sample is one load, cheaper
-// than its share of a staged box unless rays are short and leave little to skip.
+// than its share of a staged box unless rays are short and leave little to skip.  In volumes
+// of few voxels (nmax, the largest dimension) most of a march is its set-up and first samples.
 // us staged / gathered, 800^2 frames, linear:
 //   512^3 blobs, uint16 (need 0.044): 896 steps 760 / 530, 200 steps 386 / 202
 //   256^3 blobs, uint16 (0.078): 448 steps 357 / 303, 200 steps 226 / 178
@@ -171,7 +172,9 @@ __host__ inline int windows_group(float step) {
 //   512^3 blobs, uint16: 896 steps 502 / 265, 200 steps 325 / 111
 //   256^3 white noise, uint16: 448 steps 247 / 234, 200 steps 176 / 145
 //   128^3 blobs, float (0.42): 224 steps 134 / 131, 200 steps 124 / 132
-__host__ inline bool windows_pay(bool nearest, float need, float step, uint64_t tiles) {
+//   48^3 .. 80^3 blobs, 130^2 .. 600^2 frames: 17-92 / 18-95, 12% slower at the median
+__host__ inline bool windows_pay(bool nearest, float need, int nmax, float step, uint64_t tiles) {
+    if (nmax < 112) return false;
     if (nearest) return need < 0.2f || step >= 1.25f || tiles < 2048u;
     if (step >= 1.5f || tiles < 2048u) return need < 0.6f;
     return need < 0.11f;
@@ -410,7 +413,8 @@ struct IsoWindowShared {
 };
 // Voxels that a window lookup allows for between a position estimated with one fma and the
 // running sum, kIsoAnchor samples from the last exact position: each addition is off by half
-// an ulp of at most 1/2, 3.0e-8 N voxels.
+// an ulp of the position, 3.0e-8 N voxels inside the volume, twice as much for each doubling
+// of how far the box reaches past it.
 constexpr float kIsoMargin = 3e-5f;
 constexpr uint32_t kIsoAnchor = 900;
 constexpr int kIsoWindowMaxSteps = 1 << 24;
@@ -466,8 +470,11 @@ __global__ __launch_bounds__(64 * kWinSegments) void k_iso_windows(
     const bool active = (sh.rays.act >> lane & 1u) != 0;
     const bool gt = (sh.above >> lane & 1u) != 0;  // the ray's side
     if (seg != 0) sh.rays.get(lane, px, py, pz, dx, dy, dz);
-    const float mgx = kIsoMargin * vol.fnx + 0.01f, mgy = kIsoMargin * vol.fny + 0.01f,
-                mgz = kIsoMargin * vol.fnz + 0.01f;
+    float reach = 0.0f;  // uniform
+#pragma unroll
+    for (int k = 0; k < 6; ++k) reach = fmaxf(reach, 0.5f + 0.5f * fabsf(p.box[k]));
+    const float mg = reach <= 1.0f ? kIsoMargin : 2.0f * reach * kIsoMargin;
+    const float mgx = mg * vol.fnx + 0.01f, mgy = mg * vol.fny + 0.01f, mgz = mg * vol.fnz + 0.01f;
     WindowRay<PV, GS> win;
     win.begin(vol, dx, dy, dz, mgx, mgy, mgz);
     const T* const plane = gt ? vol.win_min : vol.win_max;

@@ -765,7 +765,8 @@ bool batch_windows(const spr_ctx* c, const spr_params& prm, const BatchKind& kin
                    uint64_t gy, float step) {
     return prm.alpha_pow == 0.0f && windows_tuning(c->tune) && gx <= kWinMaxGroups &&
            gy <= 65535u &&
-           windows_pay(prm.filter == SPR_FILTER_NEAREST, kind.need, step, gx * gy);
+           windows_pay(prm.filter == SPR_FILTER_NEAREST, kind.need, kind.nmax, step,
+                       gx * gy);
 }
 
 // A batch's launch: gathered by the window grid (windows: its grid, mixed: one row of every

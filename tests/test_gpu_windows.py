@@ -27,6 +27,7 @@ def volume(dtype, shape, seed):
 def render(torch, ctx, slot, p, W, H):
     o = torch.full((2, H, W), -7., device="cuda")
     s = torch.cuda.Stream()
+    torch.cuda.synchronize()
     ctx.render_slot(slot, p, _lib.METHOD_MAX_PROJECT, W, H, o[0].data_ptr(), o[1].data_ptr(),
                     stream=s.cuda_stream)
     s.synchronize()
@@ -36,9 +37,9 @@ def render(torch, ctx, slot, p, W, H):
 # steps: 4, 2 and 1 samples a group (0.6, 1.3 and 5 voxels a step), one box, segments without
 # samples (16 steps), long rays
 @pytest.mark.parametrize("dtype", [np.uint16, np.uint8, np.float32])
-@pytest.mark.parametrize("shape,steps", [((64, 64, 64), 112), ((60, 77, 50), 112),
-                                         ((64, 128, 32), 96), ((33, 90, 70), 18),
-                                         ((50, 40, 60), 16), ((30, 31, 29), 1700)])
+@pytest.mark.parametrize("shape,steps", [((64, 64, 128), 224), ((60, 117, 50), 112),
+                                         ((64, 128, 32), 96), ((33, 90, 130), 18),
+                                         ((50, 40, 112), 16), ((30, 31, 113), 1700)])
 def test_windows_equal_every_sample(dtype, shape, steps):
     import torch
     ctx = _lib.Context(0)
@@ -63,9 +64,9 @@ def test_windows_equal_every_sample(dtype, shape, steps):
 def test_windows_against_the_oracle():
     import torch
     ctx = _lib.Context(0)
-    vol = volume(np.uint16, (80, 70, 96), 8)
+    vol = volume(np.uint16, (80, 70, 116), 8)
     W, H = 90, 66
-    iP, iM = render_matrices(POSES[0], mat4_perspective(45, W / float(H), .1, 10), (96, 70, 80))
+    iP, iM = render_matrices(POSES[0], mat4_perspective(45, W / float(H), .1, 10), (116, 70, 80))
     p = _lib.make_params(iP, iM, (-1, 1, -1, 1, -1, 1), 100., 2500., max_steps=160)
     got = render(torch, ctx, ctx.volume_add(vol), p, W, H)
     out, alpha = oracle.max_project(vol, iP, iM, min_val=100., max_val=2500., max_steps=160,
@@ -80,9 +81,9 @@ def test_noise_is_staged():
     import torch
     rng = np.random.default_rng(3)
     ctx = _lib.Context(0)
-    vol = rng.integers(0, 4000, (64, 60, 70)).astype(np.uint16)
+    vol = rng.integers(0, 4000, (64, 60, 120)).astype(np.uint16)
     W, H = 100, 90
-    iP, iM = render_matrices(POSES[1], mat4_perspective(45, W / float(H), .1, 10), (70, 60, 64))
+    iP, iM = render_matrices(POSES[1], mat4_perspective(45, W / float(H), .1, 10), (120, 60, 64))
     for steps in (112, 24):
         p = _lib.make_params(iP, iM, (-1, 1, -1, 1, -1, 1), 0., 4000., max_steps=steps)
         slot = ctx.volume_add(vol)
@@ -98,7 +99,7 @@ def test_batches_gathered_and_staged():
     frames of each rendered alone, bit for bit."""
     import torch
     ctx = _lib.Context(0)
-    vols = [volume(np.uint16, s, k) for k, s in enumerate(((40, 50, 60), (33, 64, 41), (70, 30, 52)))]
+    vols = [volume(np.uint16, s, k) for k, s in enumerate(((40, 50, 112), (33, 64, 41), (70, 30, 52)))]
     slots = [ctx.volume_add(v) for v in vols]
     W, H = 75, 93
     sizes, ps, want = [], [], []
@@ -196,8 +197,8 @@ def test_iso_windows_equal_every_sample(dtype, filt, shape, steps):
 
 
 @pytest.mark.parametrize("dtype", [np.uint16, np.uint8, np.float32])
-@pytest.mark.parametrize("shape,steps", [((64, 64, 64), 112), ((60, 77, 50), 64),
-                                         ((33, 90, 70), 18), ((30, 31, 29), 1700)])
+@pytest.mark.parametrize("shape,steps", [((64, 64, 128), 224), ((60, 117, 50), 112),
+                                         ((33, 90, 130), 18), ((30, 31, 113), 1700)])
 def test_nearest_windows_equal_every_sample(dtype, shape, steps):
     """The nearest filter by the window grid (4, 2 and 1 samples a group, long rays; a frame
     alone, a uniform and a mixed batch) against every sample from global memory."""
@@ -220,6 +221,7 @@ def test_nearest_windows_equal_every_sample(dtype, shape, steps):
         for slab in (19, 0):
             ctx.set_tuning("slab_kb", slab)
             o = torch.full((3, 2, H, W), -7., device="cuda")
+            torch.cuda.synchronize()
             ctx.render_slot(slot, p, _lib.METHOD_MAX_PROJECT, W, H, o[0, 0].data_ptr(),
                             o[0, 1].data_ptr(), stream=s.cuda_stream)
             ctx.render_batch([(slot, list(iP), list(iM), o[1, 0].data_ptr(), o[1, 1].data_ptr())],
