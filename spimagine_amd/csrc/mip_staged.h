@@ -452,33 +452,149 @@ __host__ inline bool fast_norm_ok(float min_val, float max_val) {
            amn <= 0x1p39f;
 }
 
-// Whether a ray of the opacity mode may stop before its last sample (uniform).  With every
-// sample of the volume in [vmin, vmax] (brick bounds widened for float voxels), normalised
-// as the samples are to [lo, hi]: when every step multiplies cumsum by a factor in [0, 1]
-// -- integer voxels: lo >= 0 and fl(a hi) <= 1; float voxels (v clamped to [0, 1] in the
-// transparency update): a <= 1 -- cumsum never grows and stays >= 0, so a later sample
-// adds fl(cumsum' v) <= fl(cumsum hi) to col (rounding is monotone).  *hi_out = max(hi, 0).
-template <typename T>
-__device__ __forceinline__ bool opacity_can_stop(const Opacity& o, float vmin, float vmax,
-                                                 float& hi_out) {
-    constexpr bool kShort = !std::is_same<T, float>::value;
-    hi_out = 0.0f;
-    if (!(vmin <= vmax)) return false;  // a NaN voxel: never stop
-    const float m = bound_margin<T>(vmin, vmax);
-    float lo = vmin - m, hi = vmax + m;
-    if (o.norm) {
-        if (!(o.den > 0.0f)) return false;
-        lo = (lo - o.mn) / o.den;
-        hi = (hi - o.mn) / o.den;
-    }
-    hi_out = fmaxf(hi, 0.0f);
-    if (kShort) return lo >= 0.0f && o.a * hi_out <= 1.0f;
-    return o.a <= 1.0f;
+// How much the later samples of a wave's rays can still add to their colours, from the window
+// grid (brick_bounds.h).  The n samples are cut into up to 64 epochs of 2^opacity_shift(n), one a
+// lane; lane e returns at least v c / c_e for every sample of value v that any of the rays
+// takes with transparency c in or after epoch e, c_e being the ray's transparency as the epoch
+// starts: the largest window of those samples, times how far transparency can grow on the way
+// (integer voxels below min_val have factors 1 - a v above 1).  So with c_e >= 0 a ray has its
+// colour once c_e bound(e) <= col; rounding is monotone, and growth and result are widened by
+// more than the roundings of the steps.  Infinite where a factor might be negative, where the
+// normalisation isn't increasing, or where the rays run far apart.  A ray that once broke out
+// of a group of 16 lags behind the sample count and is held to bound(0), which covers any run
+// of its samples.  Lanes without a ray have another's (shadow_first_active).
+//
+// A lane asks for its epoch's windows over the box of all 64 rays, ~27 of them: 1-2% of the
+// march.  Asked by each ray for itself along its length the windows stop rays ~3% sooner but
+// cost 9% of the march.  Where opacity_windows says no, the volume's own bounds take the
+// windows' place (they stop few rays where noise reaches below min_val).
+__device__ __forceinline__ uint32_t opacity_shift(uint32_t n) {  // n > 0
+    return n <= 64u ? 0u : 32u - (uint32_t)__builtin_clz((n - 1u) >> 6);
 }
 
-// a ray whose later samples can no longer raise col (opacity_can_stop held)
-__device__ __forceinline__ bool opacity_spent(const Opacity& o, float col, float hi) {
-    return o.cumsum * hi <= col;
+// Whether a frame's rays ask the windows: enough waves that ending some early ends the frame
+// early, rays close together (tiles: 8x8 pixel quarters; a frame of few has them far apart),
+// and a march long enough in voxels (nmax, the largest dimension) and samples.  us volume's
+// bounds / windows, alpha_pow 0.6, 800^2 frames unless stated:
+//   512^3 blobs, 896 steps: uint16 983 / 891, float 943 / 786; 200 steps: uint16 390 / 406,
+//   float 472 / 429; 256^3, 448 steps: uint16 443 / 389, uint8 442 / 406
+//   128^3, 200 steps: uint16 202 / 202, uint8 198 / 211; 200^2 of 512^3, 200 steps 180 / 254
+template <typename T>
+__host__ __device__ inline bool opacity_windows(uint32_t tiles, float nmax, uint32_t n) {
+    return tiles >= 2048u && nmax >= 160.0f &&
+           (std::is_same<T, float>::value || nmax <= 2.0f * (float)n);
+}
+
+template <typename V>
+__device__ __forceinline__ float opacity_bounds(const V& vol, const Opacity& op, float px, float py,
+                                                float pz, float dx, float dy, float dz, uint32_t n,
+                                                uint32_t tiles) {
+    using T = typename V::value_type;
+    constexpr bool kShort = !std::is_same<T, float>::value;
+    const float inf = __builtin_inff();
+    const uint32_t lane = threadIdx.x & 63u, epoch = 1u << opacity_shift(n);
+    if (op.norm && !(op.den >= 0x1p-32f && op.den <= 0x1p32f)) return inf;
+    // the normalised bounds of `samples` samples with voxels in [lo, hi]: the largest (H) and
+    // the growth (G)
+    auto normalised = [&](float lo, float hi, float samples, float& H, float& G) {
+        if (op.norm) {
+            hi = (hi - op.mn) * op.rcp;
+            lo = (lo - op.mn) * op.rcp;
+        }
+        H = fmaxf(hi, 0.0f);
+        G = 1.0f;
+        if constexpr (kShort) {
+            G = __builtin_amdgcn_exp2f(samples * __builtin_amdgcn_logf(fmaxf(1.0f - op.a * lo, 1.0f))) *
+                fmaf(1e-6f, samples, 1.00001f);
+            if (op.a * H > 0.9999f) H = inf;
+        } else if (op.a > 1.0f && op.a * fminf(H, 1.0f) > 0.9999f) {
+            H = inf;
+        }
+    };
+    auto times = [](float g, float x) { return x > 0.0f ? g * x : 0.0f; };  // (not inf * 0)
+    float H = 0.0f, G = 1.0f;
+    if (!opacity_windows<T>(tiles, fmaxf(vol.fnx, fmaxf(vol.fny, vol.fnz)), n)) {
+        if (!(vol.vmin <= vol.vmax)) return inf;  // a NaN voxel, or no bounds
+        const float m = bound_margin<T>(vol.vmin, vol.vmax);
+        normalised(vol.vmin - m, vol.vmax + m, (float)(n - min(lane * epoch, n)), H, G);
+        return times(G, H) * 1.0001f;
+    }
+    const float fn = (float)n, last = (float)(n - 1u);
+    // the rays' texel coordinates at the first and the last sample: least, largest; a sample
+    // between lies between the two, but for the running sum's distance from the straight
+    // line, half an ulp of the position an addition
+    float lo0[3], hi0[3], lo1[3], hi1[3];
+    auto ends = [&](int k, float p, float d, float f) {
+        const float q = fmaf(last, d, p), a = texel<V::kPow2>(p, f), b = texel<V::kPow2>(q, f);
+        const float m = fmaf(6.1e-8f * fn * fmaxf(fabsf(p), fabsf(q)), f, 0.02f);
+        lo0[k] = a - m;
+        hi0[k] = a + m;
+        lo1[k] = b - m;
+        hi1[k] = b + m;
+    };
+    ends(0, px, dx, vol.fnx);
+    ends(1, py, dy, vol.fny);
+    ends(2, pz, dz, vol.fnz);
+    for (int o = 1; o < 64; o <<= 1) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            lo0[k] = fminf(lo0[k], __shfl_xor(lo0[k], o));
+            hi0[k] = fmaxf(hi0[k], __shfl_xor(hi0[k], o));
+            lo1[k] = fminf(lo1[k], __shfl_xor(lo1[k], o));
+            hi1[k] = fmaxf(hi1[k], __shfl_xor(hi1[k], o));
+        }
+    }
+    const uint32_t s0 = lane * epoch, s1 = min(s0 + epoch, n) - 1u;
+    const bool mine = s0 < n;
+    const float t0 = (float)s0 / last, t1 = (float)s1 / last;
+    uint32_t first[3], count[3];  // windows: every second one from the first, in blocks
+    const uint32_t size[3] = {(uint32_t)vol.nx, (uint32_t)vol.ny, (uint32_t)vol.nz};
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const float l = fminf(fmaf(t0, lo1[k] - lo0[k], lo0[k]), fmaf(t1, lo1[k] - lo0[k], lo0[k])),
+                    h = fmaxf(fmaf(t0, hi1[k] - hi0[k], hi0[k]), fmaf(t1, hi1[k] - hi0[k], hi0[k]));
+        // padded voxels floor(l) + 1 .. floor(h) + 2, kept inside the copy
+        const float end = (float)(size[k] + 1u);
+        first[k] = (uint32_t)__builtin_amdgcn_fmed3f(floorf(l) + 1.0f, 0.0f, (float)size[k]) >> kWinShift;
+        const uint32_t to = (uint32_t)__builtin_amdgcn_fmed3f(floorf(h) + 2.0f, 0.0f, end);
+        count[k] = to < 4u * first[k] + 8u ? 1u : (to - 4u * first[k]) / 8u + 1u;
+    }
+    // H: the largest normalised window, G: the growth over the epoch
+    const uint32_t gx = vol.win_gx, gy = vol.win_gy;
+    if (mine && count[0] * count[1] * count[2] > 512u) {
+        H = inf;
+    } else if (mine) {
+        float vhi = -inf, vlo = inf;
+        for (uint32_t z = 0; z < count[2]; ++z)
+            for (uint32_t y = 0; y < count[1]; y += 3u)
+                for (uint32_t x = 0; x < count[0]; x += 3u) {
+                    T hi[9], lo[9];
+#pragma unroll
+                    for (uint32_t j = 0; j < 9u; ++j) {
+                        const uint32_t xx = first[0] + 2u * min(x + j % 3u, count[0] - 1u),
+                                       yy = first[1] + 2u * min(y + j / 3u, count[1] - 1u),
+                                       w = __umul24(__umul24(first[2] + 2u * z, gy) + yy, gx) + xx;
+                        hi[j] = vol.win_max[w];
+                        if constexpr (kShort) lo[j] = vol.win_min[w];
+                    }
+#pragma unroll
+                    for (uint32_t j = 0; j < 9u; ++j) {
+                        vhi = fmaxf(vhi, (float)hi[j]);
+                        if constexpr (kShort) vlo = fminf(vlo, (float)lo[j]);
+                    }
+                }
+        normalised(vlo, vhi, (float)epoch, H, G);
+    }
+    // bound(e) = G_e max(H_e, bound(e + 1)): a suffix scan of the maps x -> max(A, G x)
+    float A = times(G, H);
+    for (uint32_t o = 1; o < 64u; o <<= 1) {
+        const float A2 = __shfl_down(A, o), G2 = __shfl_down(G, o);
+        if (lane + o < 64u) {
+            A = fmaxf(A, times(G, A2));
+            G = G * G2;
+        }
+    }
+    return A * 1.0001f;
 }
 
 template <bool kShort, typename OP>
@@ -720,7 +836,7 @@ __device__ __forceinline__ void shadow_first_active(uint64_t act, bool active, f
 // projection skips a box whose bricks' maximum cannot exceed any active ray's running
 // maximum (its samples cannot change col; only the positions advance, by the same
 // additions) and stops once every ray holds the volume's maximum; the opacity mode stops
-// once no later sample can raise any ray's colour (opacity_spent).
+// once no later sample can raise any ray's colour (opacity_bounds).
 template <typename T, bool POW2, int SLAB_BYTES, int CH, bool SHARED, bool WIDE, bool OPAC,
           bool HALVES = true, bool SKIP = false, int FILT = 0, bool FASTDIV = false>
 __device__ __forceinline__ void mip_staged_march(const PaddedVolume<T, POW2, WIDE>& vol,
@@ -881,22 +997,28 @@ __device__ __forceinline__ void mip_staged_march(const PaddedVolume<T, POW2, WID
     op.den = p.max_val - p.min_val;
     op.rcp = 1.0f / op.den;
     op.a = kShort ? 0.1f * p.alpha_pow * p.alpha_pow : p.alpha_pow * p.alpha_pow;
+    bool lag = false;  // opacity mode: the ray once broke out of a group
     int done = 0;  // samples of the current ray position sequence taken so far (uniform)
     // before n samples: a new reference 16-sample group starts the break state afresh
     auto group = [&](int n) {
         if constexpr (OPAC) {
-            if ((done & 15) == 0) op.brk = false;
+            if ((done & 15) == 0) {
+                lag = lag || op.brk;
+                op.brk = false;
+            }
         }
         done += n;
     };
     static_assert(!SKIP || !SHARED, "skipping runs with per-wave slabs");
-    // SKIP, opacity mode: whether the volume's bounds let a ray stop early, and the largest
-    // normalised sample (uniform)
-    float vmax_n = 0.0f;
-    bool can_stop = false;
-    if constexpr (SKIP && OPAC) {
-        can_stop = opacity_can_stop<T>(op, vol.vmin, vol.vmax, vmax_n);
-    }
+    // SKIP, opacity mode: what each epoch of samples and those after it can add to the rays
+    float bound = 0.0f;
+    const uint32_t shift = opacity_shift((uint32_t)(g_end - g_begin) * CH);
+    auto bound_of = [&](uint32_t e) {
+        return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(bound), e));
+    };
+    if constexpr (SKIP && OPAC)
+        bound = opacity_bounds(vol, op, px, py, pz, dx, dy, dz, (uint32_t)(g_end - g_begin) * CH,
+                               4u * p.ntiles);
     // per-wave slabs: the next box's rows are loaded into registers while this box is
     // sampled (when the next box fits and needs at most kPrefetchRows rows per lane); SKIP:
     // with its brick bounds
@@ -908,7 +1030,10 @@ __device__ __forceinline__ void mip_staged_march(const PaddedVolume<T, POW2, WID
     for (int i = g_begin; i < g_end; i += G) {
         const int ng = min(G, g_end - i);
         if constexpr (SKIP && OPAC) {
-            if (can_stop && __ballot(active && !opacity_spent(op, col, vmax_n)) == 0) break;
+            lag = lag || op.brk;
+            const float most = lag ? bound_of(0u) : bound_of((uint32_t)done >> shift);
+            const bool spent = op.cumsum >= 0.0f && op.cumsum * most <= col;
+            if (__ballot(active && !spent) == 0) break;
         }
         Box b;
         bool fits;
@@ -1585,13 +1710,16 @@ __device__ __forceinline__ PaddedVolume<T, POW2> job_volume(const BatchJob& j) {
     v.mz = (float)(j.nz - 1);
     v.bricks.keys = nullptr;  // batched frames sample every box
     v.bricks.nbx = v.bricks.nby = 0;
-    v.vmin = v.vmax = 0.0f;
+    v.vmin = 1.0f;  // none
+    v.vmax = 0.0f;
     // the window grid follows the padded copy in its allocation (VolSlot)
     v.win_max = reinterpret_cast<const T*>(static_cast<const uint8_t*>(j.base) +
                                            (((size_t)j.nbytes + 255u) & ~(size_t)255u));
-    v.win_min = nullptr;
     v.win_gx = win_entries((uint32_t)j.nx + 2u);
     v.win_gy = win_entries((uint32_t)j.ny + 2u);
+    const size_t plane = (size_t)v.win_gx * v.win_gy * win_entries((uint32_t)j.nz + 2u) * sizeof(T);
+    v.win_min = reinterpret_cast<const T*>(reinterpret_cast<const uint8_t*>(v.win_max) +
+                                           ((plane + 255u) & ~(size_t)255u));
     v.wnx = 0.25f * v.fnx;
     v.wny = 0.25f * v.fny;
     v.wnz = 0.25f * v.fnz;
@@ -1685,7 +1813,7 @@ __global__ __launch_bounds__(256) void k_max_project_batch(const BatchJob* __res
         const PaddedVolume<T, POW2> vol = job_volume<T, POW2>(j);
         if constexpr (MODE == 0 || MODE == 3)
             // (no half-wave boxes: 1.4% slower here, where the queues leave no frame tail)
-            mip_staged_rays<T, POW2, SLAB_BYTES, CH, SHARED, false, MODE == 3, false>(
+            mip_staged_rays<T, POW2, SLAB_BYTES, CH, SHARED, false, MODE == 3, false, MODE == 3>(
                 vol, p, x, y, inside, slab, s_box, j.out, j.alpha);
         else
             mip_rays<PaddedVolume<T, POW2>, MODE == 2 ? 1 : 0>(vol, p, x, y, inside, j.out,
