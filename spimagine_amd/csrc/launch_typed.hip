@@ -605,6 +605,13 @@ hipError_t launch_pair(const LaunchTuning& t, const VolSlot& vs, RayParams p, fl
     const dim3 grid(tile_grid(p.tile_map, p.ntx, p.nty));
     const int nmax = std::max(vs.nx, std::max(vs.ny, vs.nz));
     const int ch = chunk_for(t, p.nouter, nmax);
+    const float step = (float)nmax / (16.0f * (float)p.nouter);
+    if (t.skip != 0 && vs.win_bytes != 0 && windows_tuning(t) &&
+        windows_pay(false, vs.need, nmax, step, 4u * p.ntiles) &&
+        4u * tile_grid(kTileMapInterleaved, p.ntx, p.nty) <= kWinMaxGroups) {
+        launch_windows<0>(windows_group(step), padded_volume<U16Pair, P2>(vs), p, out, alpha, s);
+        return hipGetLastError();
+    }
     // (the one-wave kernel deals tiles interleaved; a cost-ordered map falls back to four)
     const bool one_wave = one_wave_for(t, p) && p.tile_map != kTileMapCostXcd;
     if (ch == 16)

@@ -735,25 +735,32 @@ __device__ __forceinline__ void staged_sample_slab_pair(const V& vol, const uint
     }
 }
 
+template <typename V>
+__device__ __forceinline__ void linear_pair(const V& vol, float px, float py, float pz, float& v0,
+                                            float& v1) {
+    float cx, cy, cz, ax, ay, az;
+    vol.locate_f(px, py, pz, &cx, &cy, &cz, &ax, &ay, &az);
+    const uint32_t off = vol.byte_offset_f(cx, cy, cz);
+    const __amdgpu_buffer_rsrc_t r = vol.rsrc();
+    float l00[2], h00[2], l10[2], h10[2], l01[2], h01[2], l11[2], h11[2];
+    PairBits<U16Pair>::load2(r, off, 0, l00, h00);
+    PairBits<U16Pair>::load2(r, off, vol.soff_y, l10, h10);
+    PairBits<U16Pair>::load2(r, off, vol.soff_z, l01, h01);
+    PairBits<U16Pair>::load2(r, off, vol.soff_yz, l11, h11);
+    v0 = trilerp(l00[0], h00[0], l10[0], h10[0], l01[0], h01[0], l11[0], h11[0], ax, ay, az);
+    v1 = trilerp(l00[1], h00[1], l10[1], h10[1], l01[1], h01[1], l11[1], h11[1], ax, ay, az);
+}
+
 template <typename V, int CH>
 __device__ __forceinline__ void staged_sample_global_pair(const V& vol, float& px, float& py,
                                                           float& pz, float dx, float dy, float dz,
                                                           float& col, float& col2) {
 #pragma unroll
     for (int j = 0; j < CH; ++j) {
-        float cx, cy, cz, ax, ay, az;
-        vol.locate_f(px, py, pz, &cx, &cy, &cz, &ax, &ay, &az);
-        const uint32_t off = vol.byte_offset_f(cx, cy, cz);
-        const __amdgpu_buffer_rsrc_t r = vol.rsrc();
-        float l00[2], h00[2], l10[2], h10[2], l01[2], h01[2], l11[2], h11[2];
-        PairBits<U16Pair>::load2(r, off, 0, l00, h00);
-        PairBits<U16Pair>::load2(r, off, vol.soff_y, l10, h10);
-        PairBits<U16Pair>::load2(r, off, vol.soff_z, l01, h01);
-        PairBits<U16Pair>::load2(r, off, vol.soff_yz, l11, h11);
-        col = fmaxf(col, trilerp(l00[0], h00[0], l10[0], h10[0], l01[0], h01[0], l11[0], h11[0],
-                                 ax, ay, az));
-        col2 = fmaxf(col2, trilerp(l00[1], h00[1], l10[1], h10[1], l01[1], h01[1], l11[1], h11[1],
-                                   ax, ay, az));
+        float v0, v1;
+        linear_pair(vol, px, py, pz, v0, v1);
+        col = fmaxf(col, v0);
+        col2 = fmaxf(col2, v1);
         px = px + dx;
         py = py + dy;
         pz = pz + dz;

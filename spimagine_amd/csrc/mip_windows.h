@@ -53,6 +53,28 @@ __device__ __forceinline__ float sum_n(float p, float d, uint32_t n) {
 
 constexpr int kWinGroups = 8;  // groups asked for together
 
+// A window's largest voxel, or a pair's of each channel
+__device__ __forceinline__ float win_value(float v) { return v; }
+__device__ __forceinline__ float win_value(uint16_t v) { return (float)v; }
+__device__ __forceinline__ float win_value(uint8_t v) { return (float)v; }
+__device__ __forceinline__ float win_value(U16Pair v) { return (float)(v.bits >> 16); }
+__device__ __forceinline__ float win_value2(U16Pair v) { return (float)(v.bits & 0xFFFFu); }
+
+// One sample, or a pair's two
+struct PairValue {
+    float v1, v0;  // channels 1 and 0
+};
+template <int FILT, typename PV>
+__device__ __forceinline__ auto window_sample(const PV& vol, float px, float py, float pz) {
+    if constexpr (std::is_same<typename PV::value_type, U16Pair>::value) {
+        PairValue r;
+        linear_pair(vol, px, py, pz, r.v0, r.v1);
+        return r;
+    } else {
+        return vol.template sample<FILT>(px, py, pz);
+    }
+}
+
 // One ray's window lookups: the block coordinates of the least corner of group j's samples
 // are (wx + j gx, ...), in windows.
 template <typename V, int GS>
@@ -114,7 +136,7 @@ struct WindowRay {
             }
 #pragma unroll
             for (int k = 0; k < 16; ++k) {
-                const float u = (float)v[k];
+                const float u = win_value(v[k]);
                 at = u > top_u ? min(i + k, probes - 1) : at;
                 top_u = fmaxf(top_u, u);
             }
@@ -141,7 +163,10 @@ constexpr int kWinSegments = 4;
 // (2 a group) 197 / 178, 512^3 float 896 steps (4) 568 / 616, 200 steps (1) 251 / 257.
 template <typename T, int GS, int FILT>
 constexpr int kWinWaves =
-    FILT == 1 || GS == 2 || (GS == 1 && !std::is_same<T, float>::value) ? 5 : 4;
+    !std::is_same<T, U16Pair>::value &&
+            (FILT == 1 || GS == 2 || (GS == 1 && !std::is_same<T, float>::value))
+        ? 5
+        : 4;
 // workgroups of one grid dimension: a launch has fewer than 2^32 threads along it
 constexpr uint64_t kWinMaxGroups = (1ull << 32) / (64 * kWinSegments) - 1;
 
@@ -207,7 +232,8 @@ struct SharedRays {
 struct WindowShared {
     float4 item[kWinSegments][128];  // each wave's waiting groups: position, ray (w's bits)
     SharedRays rays;
-    uint32_t top[64];                // the rays' running maxima (bits of floats >= 0)
+    uint32_t top[64];                // the rays' running maxima (bits of floats >= 0); a pair's
+    uint32_t top2[64];               // channel 1 in top, channel 0 in top2
 };
 
 // Samples of n >= 1 waiting groups, GS neighbouring lanes a group: batch b's lane takes sample
@@ -235,10 +261,10 @@ __device__ __forceinline__ void gather_groups(const PV& vol, const float4* item,
             qy = fmaf(ey, on[k], qy);
             qz = fmaf(ez, on[k], qz);
         }
-        return vol.template sample<FILT>(qx, qy, qz);
+        return window_sample<FILT>(vol, qx, qy, qz);
     };
     if (n == 64u) {
-        float v[GS];
+        decltype(window_sample<FILT>(vol, 0.0f, 0.0f, 0.0f)) v[GS];
         uint32_t w[GS];
 #pragma unroll
         for (int b = 0; b < GS; ++b) v[b] = value((uint32_t)b, w[b]);
@@ -248,7 +274,7 @@ __device__ __forceinline__ void gather_groups(const PV& vol, const float4* item,
 #pragma unroll 1
         for (uint32_t b = 0; b * IPB < n; ++b) {
             uint32_t w;
-            const float v = value(b, w);
+            const auto v = value(b, w);
             post(b, v, w);
         }
     }
@@ -268,6 +294,8 @@ __device__ __forceinline__ void mip_windows_rays(const PaddedVolume<T, POW2, WID
                                                  float* __restrict__ alpha, WindowShared& sh) {
     using PV = PaddedVolume<T, POW2, WIDE>;
     constexpr bool kShort = !std::is_same<T, float>::value;
+    constexpr bool kPair = std::is_same<T, U16Pair>::value;  // out: two planes of W x H
+    static_assert(!kPair || (FILT == 0 && !WIDE), "pairs: linear filter, volumes below 4 GiB");
     constexpr int BS = kWinGroups * GS;
     const uint32_t lane = threadIdx.x & 63u, seg = threadIdx.x >> 6;
     // one wave sets the rays up (~300 instructions, most of them divisions)
@@ -277,11 +305,13 @@ __device__ __forceinline__ void mip_windows_rays(const PaddedVolume<T, POW2, WID
         if (inside && !hits) {
             out[x + p.W * y] = 0.0f;
             alpha[x + p.W * y] = kShort ? 0.0f : -1.0f;
+            if constexpr (kPair) out[x + p.W * y + p.W * p.H] = 0.0f;
         }
         const uint64_t act = __ballot(hits);
         if (act != 0) shadow_first_active(act, hits, px, py, pz, dx, dy, dz);
         sh.rays.put(lane, act, px, py, pz, dx, dy, dz);
         sh.top[lane] = 0u;
+        sh.top2[lane] = 0u;
     }
     __syncthreads();
     const bool active = (sh.rays.act >> lane & 1u) != 0;
@@ -306,7 +336,13 @@ __device__ __forceinline__ void mip_windows_rays(const PaddedVolume<T, POW2, WID
         const int first = win.best(vol, px, py, pz, count);
         float qx = sum_n(px, dx, (uint32_t)first), qy = sum_n(py, dy, (uint32_t)first),
               qz = sum_n(pz, dz, (uint32_t)first), c = 0.0f;
-        staged_sample_global<PV, 2 * GS, false, FILT>(vol, qx, qy, qz, dx, dy, dz, c, op);
+        if constexpr (kPair) {
+            float c2 = 0.0f;
+            staged_sample_global_pair<PV, 2 * GS>(vol, qx, qy, qz, dx, dy, dz, c2, c);
+            if (c2 > 0.0f) atomicMax(&sh.top2[lane], __float_as_uint(c2));
+        } else {
+            staged_sample_global<PV, 2 * GS, false, FILT>(vol, qx, qy, qz, dx, dy, dz, c, op);
+        }
         if (c > 0.0f) atomicMax(&sh.top[lane], __float_as_uint(c));
     }
     __syncthreads();
@@ -316,14 +352,21 @@ __device__ __forceinline__ void mip_windows_rays(const PaddedVolume<T, POW2, WID
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         waiting -= n;
+        auto raise = [&](uint32_t* word, float v) {
+            float c = fmaxf(v, 0.0f);
+            if constexpr (GS >= 2) c = max_quad<1>(c);
+            if constexpr (GS >= 4) c = max_quad<2>(c);
+            if (lane % GS == 0 && c > 0.0f) atomicMax(word, __float_as_uint(c));
+        };
         gather_groups<FILT, GS>(vol, item + waiting, n, lane, sh.rays,
-                                [&](uint32_t, float v, uint32_t ray) {
-                                 float c = fmaxf(v, 0.0f);
-                                 if constexpr (GS >= 2) c = max_quad<1>(c);
-                                 if constexpr (GS >= 4) c = max_quad<2>(c);
-                                 if (lane % GS == 0 && c > 0.0f)
-                                     atomicMax(&sh.top[ray], __float_as_uint(c));
-                             });
+                                [&](uint32_t, auto v, uint32_t ray) {
+                                    if constexpr (kPair) {
+                                        raise(&sh.top[ray], v.v1);
+                                        raise(&sh.top2[ray], v.v0);
+                                    } else {
+                                        raise(&sh.top[ray], v);
+                                    }
+                                });
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         __builtin_amdgcn_wave_barrier();
     };
@@ -331,11 +374,16 @@ __device__ __forceinline__ void mip_windows_rays(const PaddedVolume<T, POW2, WID
         if (s + BS < count)
             win.ask(vol, px, py, pz, mgx, mgy, mgz, (float)kWinGroups, vol.win_max, nxt);
         // (other waves may raise it meanwhile: a stale value only asks for more groups)
-        const float col = __uint_as_float(__hip_atomic_load(&sh.top[lane], __ATOMIC_RELAXED,
-                                                            __HIP_MEMORY_SCOPE_WORKGROUP));
+        auto now = [](const uint32_t* word) {
+            return __uint_as_float(
+                __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
+        };
+        const float col = now(&sh.top[lane]), col2 = kPair ? now(&sh.top2[lane]) : 0.0f;
 #pragma unroll
         for (int j = 0; j < kWinGroups; ++j) {
-            const bool need = active && s + j * GS < count && (!win.ok || (float)cur[j] > col);
+            bool rises = win_value(cur[j]) > col;
+            if constexpr (kPair) rises = rises || win_value2(cur[j]) > col2;
+            const bool need = active && s + j * GS < count && (!win.ok || rises);
             const uint64_t m = __ballot(need);
             if (need)
                 item[waiting + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] =
@@ -353,8 +401,15 @@ __device__ __forceinline__ void mip_windows_rays(const PaddedVolume<T, POW2, WID
     }
     if (waiting) take(waiting);
     __syncthreads();
-    if (active && seg == 0)
-        staged_ray_end<kShort>(p, x + p.W * y, __uint_as_float(sh.top[lane]), tnear, out, alpha);
+    if (active && seg == 0) {
+        const float col = __uint_as_float(sh.top[lane]);
+        if constexpr (kPair) {
+            staged_ray_end<kShort>(p, x + p.W * y, __uint_as_float(sh.top2[lane]), tnear, out, alpha);
+            staged_plane_end(p, x + p.W * y + p.W * p.H, col, out);
+        } else {
+            staged_ray_end<kShort>(p, x + p.W * y, col, tnear, out, alpha);
+        }
+    }
 }
 
 template <typename T, bool POW2, int GS, bool WIDE, int FILT>

@@ -539,6 +539,33 @@ hipError_t pad_volume(spr_ctx* c, const VolSlot& vs, const void* src, bool from_
     return e;
 }
 
+// A channel pair's window grid and need
+hipError_t pair_windows(spr_ctx* c, VolSlot& vs) {
+    const uint32_t gx = vs.win[0], gy = vs.win[1], gz = vs.win[2];
+    uint32_t *count = nullptr, needed = 0;
+    hipError_t e = hipMallocAsync((void**)&count, sizeof(*count), c->stream);
+    if (e != hipSuccess) return e;
+    e = hipMemsetAsync(count, 0, sizeof(*count), c->stream);
+    if (e == hipSuccess) {
+        const dim3 grid((gx * gy + 255u) / 256u, gz), block(256);
+        uint32_t *blocks = (uint32_t*)vs.win_min(), *wmax = (uint32_t*)vs.win_max();
+        hipLaunchKernelGGL(k_pair_blocks, grid, block, 0, c->stream, (const U16Pair*)vs.d_pad, vs.nx,
+                           vs.ny, vs.nz, gx, gy, blocks);
+        hipLaunchKernelGGL(k_pair_windows, grid, block, 0, c->stream, (const uint32_t*)blocks, gx, gy,
+                           gz, wmax);
+        const uint32_t cols = std::max(gx * gy, std::max(gy * gz, gx * gz));
+        hipLaunchKernelGGL(k_pair_need, dim3(std::min((cols + 255u) / 256u, 256u), 3), block, 0,
+                           c->stream, (const uint32_t*)wmax, gx, gy, gz, count);
+        e = hipGetLastError();
+    }
+    if (e == hipSuccess)
+        e = hipMemcpyAsync(&needed, count, sizeof(needed), hipMemcpyDeviceToHost, c->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+    (void)hipFreeAsync(count, c->stream);
+    vs.need = (float)needed / (3.0f * (float)gx * (float)gy * (float)gz);
+    return e;
+}
+
 // fill one slot from host or device memory in the requested layout
 int fill_slot(spr_ctx* c, VolSlot& vs, const void* src, bool src_on_device, int dtype, int nx,
               int ny, int nz) {
@@ -577,12 +604,12 @@ int fill_slot(spr_ctx* c, VolSlot& vs, const void* src, bool src_on_device, int 
     // upload to the padded layout always starts a new one)
     const VolSlot before = vs;
     bool realloc = !src_on_device && layout == SPR_LAYOUT_PADDED;
-    // bounds of the padded copy (one-channel volumes): the window grid behind it in its
-    // allocation, the brick keys in their own
+    // bounds of the padded copy: the window grid behind it in its allocation (a pair's second
+    // plane holds the blocks it is made of), one-channel volumes' brick keys in their own
     const bool want_bounds = want_pad && dtype != SPR_DTYPE_U16X2;
     const uint32_t px = (uint32_t)nx + 2u, py = (uint32_t)ny + 2u, pz = (uint32_t)nz + 2u;
-    const uint32_t win[3] = {want_bounds ? win_entries(px) : 0u, want_bounds ? win_entries(py) : 0u,
-                             want_bounds ? win_entries(pz) : 0u};
+    const uint32_t win[3] = {want_pad ? win_entries(px) : 0u, want_pad ? win_entries(py) : 0u,
+                             want_pad ? win_entries(pz) : 0u};
     const size_t wbytes = (size_t)win[0] * win[1] * win[2] * es;
     // linear copy: kept as the resident volume (LINEAR layout)
     const bool need_linear = layout == SPR_LAYOUT_LINEAR;
@@ -667,6 +694,8 @@ int fill_slot(spr_ctx* c, VolSlot& vs, const void* src, bool src_on_device, int 
             vs.vmin = dtype == SPR_DTYPE_F32 ? key_value<float>(k.kmin) : (float)k.kmin;
             vs.vmax = dtype == SPR_DTYPE_F32 ? key_value<float>(~k.nkmax) : (float)~k.nkmax;
             vs.need = (float)t.needed / (3.0f * (float)win[0] * (float)win[1] * (float)win[2]);
+        } else if (e == hipSuccess) {
+            e = pair_windows(c, vs);
         }
         HIPCALL(c, e);
     }

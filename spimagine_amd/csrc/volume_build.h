@@ -156,6 +156,61 @@ __global__ __launch_bounds__(256) void k_block_windows(const BlockBounds<T>* __r
     }
 }
 
+// The window grid of a channel pair's padded copy: the maximum of each channel.  First every
+// 4x4x4 block (a thread a block, 16-byte rows), then windows of 2x2x2 of them.
+__device__ __forceinline__ uint32_t pair_max(uint32_t a, uint32_t b) {
+    return max(a & 0xFFFFu, b & 0xFFFFu) | max(a >> 16, b >> 16) << 16;
+}
+static __global__ __launch_bounds__(256) void k_pair_blocks(const U16Pair* __restrict__ pad,
+                                                            int nx, int ny, int nz, uint32_t gx,
+                                                            uint32_t gy, uint32_t* __restrict__ blocks) {
+    const uint32_t pitch = padded_pitch<U16Pair>(nx), PY = (uint32_t)ny + 2u, PZ = (uint32_t)nz + 2u;
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x, by = i / gx, bx = i - by * gx, bz = blockIdx.y;
+    if (by >= gy) return;
+    uint32_t m = 0;
+    for (uint32_t z = 4u * bz; z < min(4u * bz + 4u, PZ); ++z)
+#pragma unroll
+        for (uint32_t r = 0; r < 4u; ++r) {  // (rows past the last repeat it, voxels past a
+            const uint32_t y = min(4u * by + r, PY - 1u);  // row's end the edge voxel)
+            const uint4 v = *reinterpret_cast<const uint4*>(pad + ((size_t)z * PY + y) * pitch + 4u * bx);
+            m = pair_max(m, pair_max(pair_max(v.x, v.y), pair_max(v.z, v.w)));
+        }
+    blocks[((size_t)bz * gy + by) * gx + bx] = m;
+}
+static __global__ __launch_bounds__(256) void k_pair_windows(const uint32_t* __restrict__ blocks,
+                                                             uint32_t gx, uint32_t gy, uint32_t gz,
+                                                             uint32_t* __restrict__ wmax) {
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x, y = i / gx, x = i - y * gx, z = blockIdx.y;
+    if (y >= gy) return;
+    uint32_t m = 0;
+#pragma unroll
+    for (uint32_t c = 0; c < 8u; ++c)
+        m = pair_max(m, blocks[((size_t)min(z + (c >> 2), gz - 1u) * gy + min(y + (c >> 1 & 1u), gy - 1u)) * gx +
+                               min(x + (c & 1u), gx - 1u)]);
+    wmax[((size_t)z * gy + y) * gx + x] = m;
+}
+
+// k_window_need of a pair: a window that either channel needs, levels at three quarters of
+// the column's maximum (a pair keeps no minima)
+static __global__ __launch_bounds__(256) void k_pair_need(const uint32_t* __restrict__ wmax,
+                                                          uint32_t gx, uint32_t gy, uint32_t gz,
+                                                          uint32_t* __restrict__ count) {
+    const uint32_t n[3] = {gx, gy, gz}, stride[3] = {1u, gx, gx * gy};
+    const uint32_t a = blockIdx.y, b = a == 0 ? 1u : 0u, c = a == 2 ? 1u : 2u;
+    uint32_t need = 0;
+    for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < n[b] * n[c]; i += gridDim.x * 256u) {
+        const uint32_t ic = i / n[b], first = (i - ic * n[b]) * stride[b] + ic * stride[c];
+        uint32_t top = 0;
+        for (uint32_t k = 0; k < n[a]; ++k) top = pair_max(top, wmax[first + k * stride[a]]);
+        for (uint32_t k = 0; k < n[a]; ++k) {
+            const uint32_t v = wmax[first + k * stride[a]];
+            need += 4u * (v & 0xFFFFu) > 3u * (top & 0xFFFFu) || 4u * (v >> 16) > 3u * (top >> 16) ? 1u : 0u;
+        }
+    }
+    for (int off = 32; off > 0; off >>= 1) need += (uint32_t)__shfl_xor((int)need, off);
+    if ((threadIdx.x & 63u) == 0u) atomicAdd(count, need);
+}
+
 // Share of the windows that a max projection along the volume's axes would have to sample:
 // *count windows, over the columns of each axis (grid.y: axis), whose maximum exceeds three
 // quarters of the way from the minimum to the maximum of the column's best window.  1 for

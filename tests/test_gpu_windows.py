@@ -234,3 +234,33 @@ def test_nearest_windows_equal_every_sample(dtype, shape, steps):
         assert (outs[0][:, 1] > 0).sum() > 300
         np.testing.assert_array_equal(outs[0][0], outs[0][1])
         np.testing.assert_array_equal(outs[0][0], outs[0][2])
+
+
+# the pooled volume's rays take 4, 2 and 1 samples a group, in one box or two passes
+@pytest.mark.parametrize("shape,steps,parts", [((128, 64, 256), 224, 1), ((60, 117, 230), 96, 1),
+                                               ((66, 41, 231), 18, 1), ((61, 50, 241), 640, 2)])
+def test_pair_windows_equal_staged(shape, steps, parts):
+    """Both channels of a pooled pair by the window grid against the staged boxes
+    (SPR_TUNE_CHUNK 16): from outside and inside the volume, boxes past it."""
+    import torch
+    ctx = _lib.Context(0)
+    pair = ctx.volume_add_pooled_pair(ctx.volume_add(volume(np.uint16, shape, 9)))
+    nz, ny, nx = ctx.volume_info(pair)["shape"]
+    W, H = 119, 86
+    P = mat4_perspective(45, W / float(H), .1, 10)
+    s = torch.cuda.Stream()
+    for k, (M, box) in enumerate(zip(POSES, BOXES)):
+        iP, iM = render_matrices(M, P, (nx, ny, nz), (1., 1., 1.5))
+        p = _lib.make_params(iP, iM, box, 100., 2500., max_steps=steps)
+        outs = []
+        for chunk in (0, 16):
+            ctx.set_tuning("chunk", chunk)
+            o = torch.full((3, H, W), -7., device="cuda")
+            torch.cuda.synchronize()
+            for part in range(parts):
+                ctx.render_pair(pair, p, W, H, o[0].data_ptr(), o[2].data_ptr(), num_parts=parts,
+                                current_part=part, stream=s.cuda_stream)
+            s.synchronize()
+            outs.append(o.cpu().numpy())
+        np.testing.assert_array_equal(outs[0], outs[1], err_msg=str(k))
+        assert (outs[0][1] > 0).sum() > 300
