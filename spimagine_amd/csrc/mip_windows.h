@@ -183,7 +183,8 @@ __host__ inline int windows_group(float step) {
 // holds few samples of many voxels, and a frame of few rays leaves most of the GPU idle
 // unless their segments are marched side by side.  A nearest sample is one load, cheaper
 // than its share of a staged box unless rays are short and leave little to skip.  In volumes
-// of few voxels (nmax, the largest dimension) most of a march is its set-up and first samples.
+// of few voxels (nmax, the largest dimension) most of a march is its set-up and first samples,
+// which side by side pay only while they leave the GPU idle.
 // us staged / gathered, 800^2 frames, linear:
 //   512^3 blobs, uint16 (need 0.044): 896 steps 760 / 530, 200 steps 386 / 202
 //   256^3 blobs, uint16 (0.078): 448 steps 357 / 303, 200 steps 226 / 178
@@ -197,9 +198,10 @@ __host__ inline int windows_group(float step) {
 //   512^3 blobs, uint16: 896 steps 502 / 265, 200 steps 325 / 111
 //   256^3 white noise, uint16: 448 steps 247 / 234, 200 steps 176 / 145
 //   128^3 blobs, float (0.42): 224 steps 134 / 131, 200 steps 124 / 132
-//   48^3 .. 80^3 blobs, 130^2 .. 600^2 frames: 17-92 / 18-95, 12% slower at the median
+//   48^3 .. 80^3 blobs: 200^2 .. 600^2 frames 17-92 / 18-95, 12% slower at the median; 130^2
+//   frames 18-50 / 17-29
 __host__ inline bool windows_pay(bool nearest, float need, int nmax, float step, uint64_t tiles) {
-    if (nmax < 112) return false;
+    if (nmax < 112 && tiles >= 512u) return false;
     if (nearest) return need < 0.2f || step >= 1.25f || tiles < 2048u;
     if (step >= 1.5f || tiles < 2048u) return need < 0.6f;
     return need < 0.11f;

@@ -179,12 +179,15 @@ struct PaddedVolume {
     int nx, ny, nz;
     float fnx, fny, fnz;           // N
     float mx, my, mz;              // N - 1
-    BrickGrid bricks;              // per-brick bounds (bricks.keys == nullptr: none)
-    float vmin, vmax;              // the volume's minimum and maximum voxel
+    // (the window grid's fields stand here because the staged kernels, which don't read them,
+    // then spill no more scalar registers than without them; at the struct's end or before nx
+    // ~30 more spill slots made 600^2 frames of small volumes 3% slower)
     const T* win_max;              // window grid (brick_bounds.h): largest voxel per window,
     const T* win_min;              // smallest (nullptr: none)
     uint32_t win_gx, win_gy;       // windows per row, rows per plane
     float wnx, wny, wnz;           // N / 4: the last window that a sample's corner starts
+    BrickGrid bricks;              // per-brick bounds (bricks.keys == nullptr: none)
+    float vmin, vmax;              // the volume's minimum and maximum voxel
 
     // entry of the window at block coordinates (wx, wy, wz), kept inside the grid
     __device__ __forceinline__ uint32_t window(float wx, float wy, float wz) const {
