@@ -103,18 +103,18 @@ extern "C" {
                       bounds (default), 0 = off.  Every padded one-channel volume keeps the
                       minimum and maximum of each 8x8x8 brick and of overlapping 8x8x8
                       windows every 4 voxels (built on upload, 1/64 and 1/32 of its bytes
-                      for uint16 voxels).  With the other keys at their defaults, max
-                      projections (linear filter) of volumes whose windows leave enough to
-                      skip are gathered group by group, a group of 4, 2 or 1 samples only
+                      for uint16 voxels; a channel pair the maxima of its windows).  With the
+                      other keys at their defaults, max projections of volumes whose windows
+                      leave enough to skip are gathered group by group, a group of 4, 2 or 1 samples only
                       when its window exceeds the ray's running maximum, and the iso march
                       samples a group only when its window reaches the other side of the
                       iso value.  Otherwise, with the default per-wave slabs (slab_kb 19),
                       the max projection skips a box whose bricks' maximum cannot exceed any
                       of the wave's running maxima and the iso march a box whose bricks lie
-                      wholly on each marching ray's starting side; the opacity mode stops a
-                      wave once no later sample can raise a ray's colour (cumsum x the
-                      volume's normalised maximum <= colour, with a transparency factor
-                      provably in [0, 1]).  Results are bit-identical either way. */
+                      wholly on each marching ray's starting side.  The opacity mode (its
+                      batches always) stops a wave once transparency times the most that the
+                      windows ahead can hold, growth of the transparency included, is at most
+                      each ray's colour.  Results are bit-identical either way. */
 #define SPR_TUNE_TILE_MAP 0
 #define SPR_TUNE_SLAB_KB 1
 #define SPR_TUNE_STAGING 2
