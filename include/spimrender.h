@@ -111,8 +111,7 @@ extern "C" {
                       iso value.  Otherwise, with the default per-wave slabs (slab_kb 19),
                       the max projection skips a box whose bricks' maximum cannot exceed any
                       of the wave's running maxima and the iso march a box whose bricks lie
-                      wholly on each marching ray's starting side.  The opacity mode (its
-                      batches always) stops a wave once transparency times the most that the
+                      wholly on each marching ray's starting side.  The opacity mode stops a wave once transparency times the most that the
                       windows ahead can hold, growth of the transparency included, is at most
                       each ray's colour.  Results are bit-identical either way. */
 #define SPR_TUNE_TILE_MAP 0

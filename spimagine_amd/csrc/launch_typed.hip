@@ -354,8 +354,14 @@ hipError_t TypedLaunch<T, P2>::max_project(const LaunchTuning& t, const VolSlot&
     const bool staged_opac = !nearest && opac && t.slab_kb > 0 && t.staging == 0;
     const int nmax = std::max(vs.nx, std::max(vs.ny, vs.nz));
     // skipping by brick bounds: per-wave slabs of the default size, a volume with bounds
-    const bool skip = t.skip != 0 && vs.d_bricks != nullptr && t.staging == 0 &&
-                      (t.slab_kb == 19 || vs.pad_wide);
+    bool skip = t.skip != 0 && vs.d_bricks != nullptr && t.staging == 0 &&
+                (t.slab_kb == 19 || vs.pad_wide);
+    // the opacity mode's stop test costs 1-3% where it can't stop a ray: integer volumes that
+    // reach below min_val, in frames that don't ask the windows
+    const uint32_t samples = (uint32_t)(p.nouter + 1) * kLoopUnroll;
+    const bool stops = !std::is_integral<T>::value || p.max_val == 0.0f || p.min_val <= vs.vmin ||
+                       opacity_windows<T>(4u * p.ntiles, (float)nmax, samples);
+    if (opac && !stops) skip = false;
     // the plain max projection's box lengths (chunk 0: from the ray step)
     if (t.chunk == 0 && !opac) p.box16 = staged_groups_mip(p.nouter, nmax);
     // with the default tuning, frames that gain by it are gathered group by group
@@ -382,7 +388,7 @@ hipError_t TypedLaunch<T, P2>::max_project(const LaunchTuning& t, const VolSlot&
         void* obuf = nullptr;
         hipError_t e = order_tiles(t.tile_map, true, v, kWaveSlab19, p, s, &obuf, &g);
         if (e == hipSuccess) {
-            launch_wave_nearest<T, P2>(opac, t.skip != 0 && vs.d_bricks != nullptr, ch, g, s, v,
+            launch_wave_nearest<T, P2>(opac, t.skip != 0 && vs.d_bricks != nullptr && (!opac || stops), ch, g, s, v,
                                        p, out, alpha);
             e = hipGetLastError();
         }
@@ -541,6 +547,11 @@ hipError_t TypedLaunch<T, P2>::batch(const LaunchTuning& t, int mode, int ch, co
         if (ch == 16) return launch_batch_kernel<T, P2, kQuadSlab19, 3, 16, false>(cus, d_jobs, p, q, counters, s);
         if (ch == 8) return launch_batch_kernel<T, P2, kQuadSlab19, 3, 8, false>(cus, d_jobs, p, q, counters, s);
         return launch_batch_kernel<T, P2, kQuadSlab19, 3, 4, false>(cus, d_jobs, p, q, counters, s);
+    }
+    if (mode == 4) {
+        if (ch == 16) return launch_batch_kernel<T, P2, kQuadSlab19, 4, 16, false>(cus, d_jobs, p, q, counters, s);
+        if (ch == 8) return launch_batch_kernel<T, P2, kQuadSlab19, 4, 8, false>(cus, d_jobs, p, q, counters, s);
+        return launch_batch_kernel<T, P2, kQuadSlab19, 4, 4, false>(cus, d_jobs, p, q, counters, s);
     }
     const bool sh = t.staging == 1;
     if (t.slab_kb == 8) return launch_batch_slab<T, P2, 8192>(sh, ch, cus, d_jobs, p, q, counters, s);

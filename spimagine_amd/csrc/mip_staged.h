@@ -1779,6 +1779,8 @@ static __global__ void k_reset_counters(uint32_t* __restrict__ counters) {
 // after one failed claim on each queue.
 // MODE 0: staged plain max projection (linear filter, alpha_pow == 0; CH samples per
 // staged box); MODE 3: staged opacity mode (linear filter, alpha_pow > 0, per-wave slabs);
+// MODE 4: the same, waves stopped by the window grid (batches with a frame that asks it: the
+// others would pay 2-3% for tests that stop nothing);
 // MODE 1 / 2: every sample from global memory with the linear / nearest filter (any
 // alpha_pow; CH and SHARED unused)
 template <typename T, bool POW2, int SLAB_BYTES, int MODE, int CH, bool SHARED>
@@ -1818,9 +1820,9 @@ __global__ __launch_bounds__(256) void k_max_project_batch(const BatchJob* __res
         tile_thread_pixel(tx, ty, &x, &y);
         const bool inside = x < p.W && y < p.H;
         const PaddedVolume<T, POW2> vol = job_volume<T, POW2>(j);
-        if constexpr (MODE == 0 || MODE == 3)
+        if constexpr (MODE == 0 || MODE == 3 || MODE == 4)
             // (no half-wave boxes: 1.4% slower here, where the queues leave no frame tail)
-            mip_staged_rays<T, POW2, SLAB_BYTES, CH, SHARED, false, MODE == 3, false, MODE == 3>(
+            mip_staged_rays<T, POW2, SLAB_BYTES, CH, SHARED, false, MODE != 0, false, MODE == 4>(
                 vol, p, x, y, inside, slab, s_box, j.out, j.alpha);
         else
             mip_rays<PaddedVolume<T, POW2>, MODE == 2 ? 1 : 0>(vol, p, x, y, inside, j.out,

@@ -798,11 +798,19 @@ bool batch_windows(const spr_ctx* c, const spr_params& prm, const BatchKind& kin
                        gx * gy);
 }
 
+bool opacity_asks(int dtype, uint32_t tiles, int nmax, int nouter) {
+    const uint32_t n = (uint32_t)(nouter + 1) * kLoopUnroll;
+    return dtype == SPR_DTYPE_F32 ? opacity_windows<float>(tiles, (float)nmax, n)
+                                  : opacity_windows<uint16_t>(tiles, (float)nmax, n);
+}
+
 // A batch's launch: gathered by the window grid (windows: its grid, mixed: one row of every
-// frame's workgroups) or from the persistent queues (ch: samples per staged box)
+// frame's workgroups) or from the persistent queues (ch: samples per staged box; stops: an
+// opacity frame asks the windows)
 hipError_t dispatch_batch(const spr_ctx* c, const spr_params& prm, const BatchKind& kind, int ch,
                           const BatchJob* d_jobs, const RayParams& p, const BatchQueues& q,
-                          bool windows, dim3 g, float step, uint32_t* counters, hipStream_t s) {
+                          bool windows, bool stops, dim3 g, float step, uint32_t* counters,
+                          hipStream_t s) {
     const LaunchTuning& t = c->tune;
     const bool nearest = prm.filter == SPR_FILTER_NEAREST;
     if (windows)
@@ -810,12 +818,13 @@ hipError_t dispatch_batch(const spr_ctx* c, const spr_params& prm, const BatchKi
             return L.windows_batch(windows_group(step), nearest, d_jobs, q.njobs, g, q.mixed != 0u, p,
                                    nullptr, s);
         });
-    // 0: staged max projection, 3: staged opacity mode (per-wave 19 KiB slabs), 1 / 2: every
+    // 0: staged max projection, 3 / 4: staged opacity mode (per-wave 19 KiB slabs), 1 / 2: every
     // sample from global memory (linear / nearest)
     const int mode = nearest ? 2
                      : t.slab_kb <= 0 ? 1
                      : prm.alpha_pow == 0.0f ? 0
-                     : t.staging == 0 ? 3 : 1;
+                     : t.staging != 0 ? 1
+                     : stops && t.skip != 0 ? 4 : 3;
     return visit_launch(kind.dtype, kind.pow2, [&](auto L) {
         return L.batch(t, mode, ch, d_jobs, p, q, counters, s);
     });
@@ -828,8 +837,9 @@ hipError_t dispatch_batch(const spr_ctx* c, const spr_params& prm, const BatchKi
     const uint32_t per = 4u * tile_grid(kTileMapInterleaved, p.ntx, p.nty);
     const float step = (float)kind.nmax / (16.0f * (float)p.nouter);
     return dispatch_batch(c, prm, kind, chunk_for(c->tune, p.nouter, kind.nmax), d_jobs, p, q,
-                          batch_windows(c, prm, kind, per, q.njobs, step), dim3(per, q.njobs), step,
-                          counters, s);
+                          batch_windows(c, prm, kind, per, q.njobs, step),
+                          opacity_asks(kind.dtype, 4u * p.ntiles, kind.nmax, p.nouter),
+                          dim3(per, q.njobs), step, counters, s);
 }
 
 // Enqueues the copy of a batch's job table to d_jobs on stream s from pinned host memory
@@ -1428,6 +1438,7 @@ int spr_render_frames(spr_ctx* c, const spr_frame* frames, int n, float alpha_po
     int ch = kLoopUnroll;
     uint64_t groups = 0;
     float step = 0.0f;
+    bool stops = false;
     for (int i = 0; i < n; ++i) {
         BatchJob& b = host[i];
         const uint32_t ntx = (b.W + 15u) / 16u, nty = (b.H + 15u) / 16u;
@@ -1439,6 +1450,7 @@ int spr_render_frames(spr_ctx* c, const spr_frame* frames, int n, float alpha_po
         ch = std::min(ch, chunk_for(c->tune, b.nouter, nmax));
         groups += 4u * tile_grid(kTileMapInterleaved, ntx, nty);
         step = std::max(step, (float)nmax / (16.0f * (float)b.nouter));
+        stops = stops || opacity_asks(kind.dtype, 4u * ntx * nty, nmax, b.nouter);
     }
     q.mixed = 1;
     q.njobs = (uint32_t)n;
@@ -1467,8 +1479,8 @@ int spr_render_frames(spr_ctx* c, const spr_frame* frames, int n, float alpha_po
     uint32_t* d_counters = (uint32_t*)((char*)buf + jbytes);
     hipError_t e = stage_jobs(c, host.data(), jbytes, d_jobs, s);
     if (e == hipSuccess)
-        e = dispatch_batch(c, prm, kind, ch, d_jobs, p, q, windows, dim3((uint32_t)groups), step,
-                           d_counters, s);
+        e = dispatch_batch(c, prm, kind, ch, d_jobs, p, q, windows, stops, dim3((uint32_t)groups),
+                           step, d_counters, s);
     (void)hipFreeAsync(buf, s);
     HIPCALL(c, e);
     return SPR_OK;
