@@ -559,7 +559,7 @@ def bench_iso(args):
         "skipping_ms": table,
         "max_steps_200_ms": default_steps,
         "roofline": dict(roofline(b_alg, kernel_ms, None),
-                         kernel="iso pipeline per frame (march k_iso_staged + 6 post-pass "
+                         kernel="iso pipeline per frame (march k_iso_windows + 6 post-pass "
                                 "kernels; the march dominates, see profiles/)",
                          frac_skipping_off=round(
                              float(np.mean([b / (t * 1e-3) for b, t in zip(
