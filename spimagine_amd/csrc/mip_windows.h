@@ -53,6 +53,19 @@ __device__ __forceinline__ float sum_n(float p, float d, uint32_t n) {
 
 constexpr int kWinGroups = 8;  // groups asked for together
 
+// What a window lookup allows for, as a share of the volume, between a position estimated
+// with one fma and the running sum: each addition since the exact position is off by half an
+// ulp of the position, 3.0e-8 inside the volume (2e-6 over the at most 64 samples that the max
+// projection asks ahead, 2.7e-5 over kIsoAnchor), and 6.0e-8 times how far the box reaches
+// where that is past it.
+constexpr float kMipMargin = 1e-5f, kIsoMargin = 3e-5f;
+__device__ __forceinline__ float window_margin(const RayParams& p, float inside) {
+    float reach = 0.0f;  // (uniform)
+#pragma unroll
+    for (int k = 0; k < 6; ++k) reach = fmaxf(reach, 0.5f + 0.5f * fabsf(p.box[k]));
+    return reach <= 1.0f ? inside : 2.0f * reach * inside;
+}
+
 // A window's largest voxel, or a pair's of each channel
 __device__ __forceinline__ float win_value(float v) { return v; }
 __device__ __forceinline__ float win_value(uint16_t v) { return (float)v; }
@@ -327,8 +340,8 @@ __device__ __forceinline__ void mip_windows_rays(const PaddedVolume<T, POW2, WID
     px = sum_n(px, dx, (uint32_t)s0);
     py = sum_n(py, dy, (uint32_t)s0);
     pz = sum_n(pz, dz, (uint32_t)s0);
-    const float mgx = 1e-5f * vol.fnx + 0.01f, mgy = 1e-5f * vol.fny + 0.01f,
-                mgz = 1e-5f * vol.fnz + 0.01f;
+    const float mg = window_margin(p, kMipMargin);
+    const float mgx = mg * vol.fnx + 0.01f, mgy = mg * vol.fny + 0.01f, mgz = mg * vol.fnz + 0.01f;
     Opacity op;  // (unused)
     WindowRay<PV, GS> win;
     win.begin(vol, dx, dy, dz, mgx, mgy, mgz);
@@ -468,12 +481,7 @@ struct IsoWindowShared {
     uint64_t above;    // the rays that start above the iso value
     uint32_t hit[64];  // the rays' least crossing sample (~0: none)
 };
-// Voxels that a window lookup allows for between a position estimated with one fma and the
-// running sum, kIsoAnchor samples from the last exact position: each addition is off by half
-// an ulp of the position, 3.0e-8 N voxels inside the volume, twice as much for each doubling
-// of how far the box reaches past it.
-constexpr float kIsoMargin = 3e-5f;
-constexpr uint32_t kIsoAnchor = 900;
+constexpr uint32_t kIsoAnchor = 900;  // samples that a lookup may lie past an exact position
 constexpr int kIsoWindowMaxSteps = 1 << 24;
 
 template <typename T, bool POW2, int GS, bool WIDE, int FILT>
@@ -527,10 +535,7 @@ __global__ __launch_bounds__(64 * kWinSegments) void k_iso_windows(
     const bool active = (sh.rays.act >> lane & 1u) != 0;
     const bool gt = (sh.above >> lane & 1u) != 0;  // the ray's side
     if (seg != 0) sh.rays.get(lane, px, py, pz, dx, dy, dz);
-    float reach = 0.0f;  // uniform
-#pragma unroll
-    for (int k = 0; k < 6; ++k) reach = fmaxf(reach, 0.5f + 0.5f * fabsf(p.box[k]));
-    const float mg = reach <= 1.0f ? kIsoMargin : 2.0f * reach * kIsoMargin;
+    const float mg = window_margin(p, kIsoMargin);
     const float mgx = mg * vol.fnx + 0.01f, mgy = mg * vol.fny + 0.01f, mgz = mg * vol.fnz + 0.01f;
     WindowRay<PV, GS> win;
     win.begin(vol, dx, dy, dz, mgx, mgy, mgz);
