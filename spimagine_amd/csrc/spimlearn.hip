@@ -480,11 +480,17 @@ constexpr int kGW = 32, kGH = 8;                  // tile
 constexpr int kGLW = kGW + 2, kGLH = kGH + 2;     // with its halo
 constexpr int kXStride = 36;                      // bf16 elements per halo pixel (32 + padding)
 
-// three bf16 pieces of two floats, packed (low half: a)
+// three bf16 pieces of two floats, packed (low half: a).  ODD: an infinity or NaN is its first
+// piece alone (the others would be inf - inf).
+template <bool ODD = false>
 __device__ __forceinline__ void split3(float a, float b, uint32_t& p0, uint32_t& p1, uint32_t& p2) {
     const uint32_t ua = __float_as_uint(a), ub = __float_as_uint(b);
     p0 = __builtin_amdgcn_perm(ub, ua, 0x07060302u);
-    const float ra = a - __uint_as_float(ua & 0xFFFF0000u), rb = b - __uint_as_float(ub & 0xFFFF0000u);
+    float ra = a - __uint_as_float(ua & 0xFFFF0000u), rb = b - __uint_as_float(ub & 0xFFFF0000u);
+    if constexpr (ODD) {
+        ra = ra == ra ? ra : 0.0f;
+        rb = rb == rb ? rb : 0.0f;
+    }
     const uint32_t va = __float_as_uint(ra), vb = __float_as_uint(rb);
     p1 = __builtin_amdgcn_perm(vb, va, 0x07060302u);
     const float sa = ra - __uint_as_float(va & 0xFFFF0000u), sb = rb - __uint_as_float(vb & 0xFFFF0000u);
@@ -530,6 +536,11 @@ __device__ __forceinline__ void load_grad_tile(const float* __restrict__ g,
     }
 }
 
+// all bits of each half that holds an infinity or NaN
+__device__ __forceinline__ uint32_t not_finite(uint32_t pair) {
+    return ((((pair & 0x7F807F80u) + 0x00800080u) & 0x80008000u) >> 15) * 0xFFFFu;
+}
+
 // the three pieces of this lane's B fragment: channel lane % 32 of pixels 8 (lane / 32) + 0..7
 // of the 16 from pix on; their sum added to bsum
 template <int COUT>
@@ -544,7 +555,7 @@ __device__ __forceinline__ void grad_fragment(const float* gs, int pix, uint32_t
         bsum += v[j];
     }
 #pragma unroll
-    for (int j = 0; j < 4; ++j) split3(v[2 * j], v[2 * j + 1], b[0][j], b[1][j], b[2][j]);
+    for (int j = 0; j < 4; ++j) split3<true>(v[2 * j], v[2 * j + 1], b[0][j], b[1][j], b[2][j]);
 }
 
 // One wave after the other adds its accumulators (N per lane, lane-major) into buf
@@ -691,10 +702,15 @@ __global__ __launch_bounds__(256) void k_wgrad_in(const float* __restrict__ x,
             for (int j = 0; j < 8; ++j) v[j] = row < 18 ? src[j] : 0.0f;
 #pragma unroll
             for (int j = 0; j < 4; ++j) split3(v[2 * j], v[2 * j + 1], a[0][j], a[1][j], a[2][j]);
+            acc[0] = mfma16(a[0], b[0], acc[0]);
+            // an infinite gradient meets x's first piece only: the others may be 0, and 0 x inf is NaN
+#pragma unroll
+            for (int j = 0; j < 4; ++j) b[0][j] &= ~not_finite(b[0][j]);
 #pragma unroll
             for (int k = 0; k < 3; ++k)
 #pragma unroll
-                for (int m = 0; m < 3; ++m) acc[0] = mfma16(a[m], b[k], acc[0]);
+                for (int m = 0; m < 3; ++m)
+                    if (k + m > 0) acc[0] = mfma16(a[m], b[k], acc[0]);
         }
     }
     add_waves<1>(gs, acc, bsum);
