@@ -231,7 +231,9 @@ int spr_volume_add_pooled_pair(spr_ctx *ctx, int src_slot, int *slot);
 int spr_volume_read(spr_ctx *ctx, int slot, void *host, size_t bytes);
 /* Free a slot >= 1 (waits for the device to finish work that may read it). */
 int spr_volume_release(spr_ctx *ctx, int slot);
-/* Voxel type, size and device bytes of a slot (0 = the renderer's volume). */
+/* Voxel type, size and device bytes of a slot (0 = the renderer's volume): its voxels, their
+   window grid and brick bounds.  A context also keeps up to 64 MiB (four planes where that is
+   more) that uploads from host memory go through. */
 int spr_volume_info(spr_ctx *ctx, int slot, int *dtype, int *nx, int *ny, int *nz,
                     size_t *device_bytes);
 

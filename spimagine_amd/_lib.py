@@ -50,6 +50,15 @@ EXPORTS = (
 )
 
 
+def padded_bytes(shape, dtype):
+    """Device bytes of a (nz, ny, nx) volume in the padded layout: one voxel of apron on
+    every side, rows padded to 16 bytes (the layout spr_volume_add picks when it fits)."""
+    nz, ny, nx = shape
+    es = np.dtype(dtype).itemsize
+    per16 = 16 // es
+    return (nz + 2) * (ny + 2) * ((nx + 2 + per16 - 1) // per16) * 16
+
+
 class SprParams(ctypes.Structure):
     """struct spr_params (include/spimrender.h)."""
     _fields_ = [
@@ -440,6 +449,18 @@ class Context:
         self._check(self.lib.spr_volume_info(self.handle, int(slot), ctypes.byref(d), ctypes.byref(x),
                                              ctypes.byref(y), ctypes.byref(z), ctypes.byref(b)))
         return {"dtype": d.value, "shape": (z.value, y.value, x.value), "bytes": b.value}
+
+    @staticmethod
+    def volume_bytes(shape, dtype):
+        """The bytes that volume_info will report of a volume added with the AUTO layout: its
+        voxels (padded, and linear too above 4 GiB padded), the two planes of its window grid
+        and its brick keys."""
+        es = np.dtype(dtype).itemsize
+        pb = padded_bytes(shape, dtype)
+        windows = int(np.prod([(n + 5) // 4 for n in shape])) * es  # every 4 of n + 2 voxels
+        bricks = int(np.prod([(n + 9) // 8 for n in shape])) + 2
+        linear = 0 if pb <= 0xFFFFFFFF else int(np.prod(shape)) * es
+        return linear + -(-pb // 256) * 256 + 2 * (-(-windows // 256) * 256) + 8 * bricks
 
     @staticmethod
     def make_jobs(jobs):

@@ -654,15 +654,15 @@ int fill_slot(spr_ctx* c, VolSlot& vs, const void* src, bool src_on_device, int 
     if (want_pad) {
         if (!vs.d_pad) {
             realloc = true;
-            HIPCALL(c, hipMalloc(&vs.d_pad, VolSlot::align256(pbytes) + 2 * VolSlot::align256(wbytes)));
             vs.pad_bytes = pbytes;
             vs.win_bytes = wbytes;
+            HIPCALL(c, hipMalloc(&vs.d_pad, vs.pad_alloc()));
         }
         const size_t nbricks = (size_t)nbx * nby * nbz;
         if (want_bounds && !vs.d_bricks) {
             realloc = true;
             // two more entries: the volume's bounds, the count of k_window_need
-            HIPCALL(c, hipMalloc(&vs.d_bricks, (nbricks + 2) * sizeof(BrickKey)));
+            HIPCALL(c, hipMalloc(&vs.d_bricks, vs.brick_alloc()));
         }
         // the 4x4x4 block bounds live from the padding pass to the windows' only
         void* blocks = nullptr;
@@ -1218,7 +1218,9 @@ int spr_volume_info(spr_ctx* c, int slot, int* dtype, int* nx, int* ny, int* nz,
     if (nx) *nx = vs->nx;
     if (ny) *ny = vs->ny;
     if (nz) *nz = vs->nz;
-    if (device_bytes) *device_bytes = vs->vol_bytes + vs->pad_bytes;
+    if (device_bytes)
+        *device_bytes = vs->vol_bytes + (vs->d_pad ? vs->pad_alloc() : 0) +
+                        (vs->d_bricks ? vs->brick_alloc() : 0);
     return SPR_OK;
 }
 

@@ -44,6 +44,8 @@ struct VolSlot {
     static size_t align256(size_t n) { return (n + 255) / 256 * 256; }
     void* win_max() const { return (char*)d_pad + align256(pad_bytes); }
     void* win_min() const { return (char*)win_max() + align256(win_bytes); }
+    size_t pad_alloc() const { return align256(pad_bytes) + 2 * align256(win_bytes); }
+    size_t brick_alloc() const { return ((size_t)nbx * nby * nbz + 2) * sizeof(BrickKey); }
 };
 
 // spr_set_tuning state (include/spimrender.h SPR_TUNE_*) plus the device's CU count

@@ -93,6 +93,8 @@ class RenderServer(object):
             free, _ = _lib.device_memory(device)
             hbm_budget = int(.6 * free)
         self.hbm_budget = int(hbm_budget)
+        # what a volume will take, as volume_info reports it once resident
+        self._volume_bytes = getattr(self.ctx, "volume_bytes", device_bytes)
         self.max_batch = int(max_batch)
         self.volumes = {}
         self.resident_bytes = 0
@@ -163,7 +165,7 @@ class RenderServer(object):
             return "ready"
         if vol.loading:
             return "wait"
-        need = device_bytes(vol.data.shape, vol.data.dtype)
+        need = self._volume_bytes(vol.data.shape, vol.data.dtype)
         if need > self.hbm_budget:
             raise MemoryError("volume %r larger than the HBM budget" % vol.name)
         idle = sorted((v for v in self.volumes.values() if v.slot is not None and v.users == 0
@@ -187,7 +189,7 @@ class RenderServer(object):
 
     def _load(self, vol, victims):
         """Releases the evicted slots and uploads `vol` (no scheduler lock held)."""
-        need = device_bytes(vol.data.shape, vol.data.dtype)
+        need = self._volume_bytes(vol.data.shape, vol.data.dtype)
         try:
             with self.table_lock:
                 for slot, _ in victims:
@@ -393,18 +395,12 @@ class RenderServer(object):
             fut.set_result(res)
 
 
-def padded_bytes(shape, dtype):
-    """Device bytes of a (nz, ny, nx) volume in the padded layout: one voxel of apron on
-    every side, rows padded to 16 bytes (the layout spr_volume_add picks when it fits)."""
-    nz, ny, nx = shape
-    es = np.dtype(dtype).itemsize
-    per16 = 16 // es
-    return (nz + 2) * (ny + 2) * ((nx + 2 + per16 - 1) // per16) * 16
+padded_bytes = _lib.padded_bytes
 
 
 def device_bytes(shape, dtype):
-    """Device bytes spr_volume_add takes for a volume: the padded copy, plus the linear
-    volume when the padded copy exceeds 4 GiB."""
+    """Device bytes of a volume's voxels in a slot: the padded copy, plus the linear volume when
+    the padded copy exceeds 4 GiB (the bounds beside them: Context.volume_bytes)."""
     pb = padded_bytes(shape, dtype)
     if pb <= 0xFFFFFFFF:
         return pb
