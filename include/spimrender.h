@@ -352,7 +352,9 @@ int spr_render_batch_noalloc(spr_ctx *ctx, const spr_params *params, const spr_j
    releasing or refilling one of them (spr_volume_release, a spr_volume_add that reuses the
    slot, a spr_set_volume* that reallocates slot 0 or changes its shape, type or layout)
    makes spr_batch_graph_launch fail with SPR_ERR_INVALID_ARG until spr_batch_graph_update
-   names live slots again.  An update must keep the voxel type and whether every volume's
+   names live slots again.  How the frames are marched follows the volumes' voxels at each
+   launch, as spr_render_batch's does: a create or an update captures the launch for either
+   case.  An update must keep the voxel type and whether every volume's
    dimensions are powers of two (the captured kernel's texel rule). */
 typedef struct spr_batch_graph spr_batch_graph;
 int spr_batch_graph_create(spr_ctx *ctx, const spr_job *jobs, int n, int w, int h,

@@ -45,12 +45,30 @@ static void* g_scratch_ptr[kMaxDevices] = {};
 static std::mutex g_noalloc_mu;
 static BatchJob g_noalloc_jobs[SPR_NOALLOC_MAX_JOBS];
 
+// How a batch is marched: gathered by the window grid, gs samples a group, or from the
+// persistent queues, ch samples a staged box (stops: an opacity frame asks the windows).
+struct BatchPlan {
+    bool windows, stops;
+    int gs, ch;
+    bool operator==(const BatchPlan& o) const {
+        return windows == o.windows && (windows ? gs == o.gs : stops == o.stops && ch == o.ch);
+    }
+};
+
+// The captured launch of each plan that the jobs' volumes may ask for: which of them pays
+// depends on the voxels, and a volume refilled in place keeps its graphs.
 struct spr_batch_graph {
     int n = 0, w = 0, h = 0;
     BatchJob* d_jobs = nullptr;
     uint32_t* d_counters = nullptr;
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t exec = nullptr;
+    struct Captured {
+        BatchPlan plan;
+        hipGraph_t graph;
+        hipGraphExec_t exec;
+    };
+    std::vector<Captured> captured;
+    spr_params prm{};
+    LaunchTuning tune;
     hipStream_t last_stream = nullptr;
     int dtype = -1;
     bool pow2 = false;  // the captured kernel's texel rule (every volume a power of two)
@@ -790,9 +808,9 @@ BatchQueues make_queues(const RayParams& p, int n) {
 // Whether a batch is gathered by the window grid: plain max projections with the default
 // tuning whose volumes gain by it (g: the launch, workgroups x frames; step: the longest ray
 // step in voxels)
-bool batch_windows(const spr_ctx* c, const spr_params& prm, const BatchKind& kind, uint64_t gx,
+bool batch_windows(const LaunchTuning& t, const spr_params& prm, const BatchKind& kind, uint64_t gx,
                    uint64_t gy, float step) {
-    return prm.alpha_pow == 0.0f && windows_tuning(c->tune) && gx <= kWinMaxGroups &&
+    return prm.alpha_pow == 0.0f && windows_tuning(t) && gx <= kWinMaxGroups &&
            gy <= 65535u &&
            windows_pay(prm.filter == SPR_FILTER_NEAREST, kind.need, kind.nmax, step,
                        gx * gy);
@@ -804,19 +822,14 @@ bool opacity_asks(int dtype, uint32_t tiles, int nmax, int nouter) {
                                   : opacity_windows<uint16_t>(tiles, (float)nmax, n);
 }
 
-// A batch's launch: gathered by the window grid (windows: its grid, mixed: one row of every
-// frame's workgroups) or from the persistent queues (ch: samples per staged box; stops: an
-// opacity frame asks the windows)
-hipError_t dispatch_batch(const spr_ctx* c, const spr_params& prm, const BatchKind& kind, int ch,
-                          const BatchJob* d_jobs, const RayParams& p, const BatchQueues& q,
-                          bool windows, bool stops, dim3 g, float step, uint32_t* counters,
-                          hipStream_t s) {
-    const LaunchTuning& t = c->tune;
+// A batch's launch (g: the window grid's, mixed: one row of every frame's workgroups)
+hipError_t dispatch_batch(const LaunchTuning& t, const spr_params& prm, int dtype, bool pow2,
+                          const BatchPlan& plan, const BatchJob* d_jobs, const RayParams& p,
+                          const BatchQueues& q, dim3 g, uint32_t* counters, hipStream_t s) {
     const bool nearest = prm.filter == SPR_FILTER_NEAREST;
-    if (windows)
-        return visit_launch(kind.dtype, kind.pow2, [&](auto L) {
-            return L.windows_batch(windows_group(step), nearest, d_jobs, q.njobs, g, q.mixed != 0u, p,
-                                   nullptr, s);
+    if (plan.windows)
+        return visit_launch(dtype, pow2, [&](auto L) {
+            return L.windows_batch(plan.gs, nearest, d_jobs, q.njobs, g, q.mixed != 0u, p, nullptr, s);
         });
     // 0: staged max projection, 3 / 4: staged opacity mode (per-wave 19 KiB slabs), 1 / 2: every
     // sample from global memory (linear / nearest)
@@ -824,22 +837,78 @@ hipError_t dispatch_batch(const spr_ctx* c, const spr_params& prm, const BatchKi
                      : t.slab_kb <= 0 ? 1
                      : prm.alpha_pow == 0.0f ? 0
                      : t.staging != 0 ? 1
-                     : stops && t.skip != 0 ? 4 : 3;
-    return visit_launch(kind.dtype, kind.pow2, [&](auto L) {
-        return L.batch(t, mode, ch, d_jobs, p, q, counters, s);
+                     : plan.stops && t.skip != 0 ? 4 : 3;
+    return visit_launch(dtype, pow2, [&](auto L) {
+        return L.batch(t, mode, plan.ch, d_jobs, p, q, counters, s);
     });
 }
 
-// The same for a uniform batch (make_queues): frames of p.W x p.H with p.nouter blocks
-hipError_t dispatch_batch(const spr_ctx* c, const spr_params& prm, const BatchKind& kind,
+// A uniform batch (make_queues), frames of p.W x p.H with p.nouter blocks: its plan
+uint32_t frame_groups(const RayParams& p) { return 4u * tile_grid(kTileMapInterleaved, p.ntx, p.nty); }
+
+BatchPlan uniform_plan(const LaunchTuning& t, const spr_params& prm, const BatchKind& kind,
+                       const RayParams& p, uint32_t njobs) {
+    const float step = (float)kind.nmax / (16.0f * (float)p.nouter);
+    return BatchPlan{batch_windows(t, prm, kind, frame_groups(p), njobs, step),
+                     opacity_asks(kind.dtype, 4u * p.ntiles, kind.nmax, p.nouter), windows_group(step),
+                     chunk_for(t, p.nouter, kind.nmax)};
+}
+
+// ... and its launch
+hipError_t dispatch_batch(const LaunchTuning& t, const spr_params& prm, const BatchKind& kind,
                           const BatchJob* d_jobs, const RayParams& p, const BatchQueues& q,
                           uint32_t* counters, hipStream_t s) {
-    const uint32_t per = 4u * tile_grid(kTileMapInterleaved, p.ntx, p.nty);
-    const float step = (float)kind.nmax / (16.0f * (float)p.nouter);
-    return dispatch_batch(c, prm, kind, chunk_for(c->tune, p.nouter, kind.nmax), d_jobs, p, q,
-                          batch_windows(c, prm, kind, per, q.njobs, step),
-                          opacity_asks(kind.dtype, 4u * p.ntiles, kind.nmax, p.nouter),
-                          dim3(per, q.njobs), step, counters, s);
+    return dispatch_batch(t, prm, kind.dtype, kind.pow2, uniform_plan(t, prm, kind, p, q.njobs), d_jobs,
+                          p, q, dim3(frame_groups(p), q.njobs), counters, s);
+}
+
+// A graph's ray parameters (num_parts 1)
+RayParams graph_params(const spr_batch_graph* bg) {
+    RayParams p = make_params(bg->prm, bg->tune.tile_map, bg->w, bg->h);
+    staged_tuning(bg->tune, p);
+    p.nouter = bg->prm.max_steps / kLoopUnroll;
+    p.current_part = 0;
+    return p;
+}
+
+// The graph's launch of a plan, captured if it was not yet
+int graph_capture(spr_ctx* c, spr_batch_graph* bg, const BatchPlan& plan) {
+    for (const auto& k : bg->captured)
+        if (k.plan == plan) return SPR_OK;
+    const RayParams p = graph_params(bg);
+    const BatchQueues q = make_queues(p, bg->n);
+    spr_batch_graph::Captured k{plan, nullptr, nullptr};
+    hipStream_t cs;
+    if (hipStreamCreateWithFlags(&cs, hipStreamNonBlocking) != hipSuccess)
+        return fail(c, SPR_ERR_HIP, "capture stream");
+    hipError_t e = hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal);
+    hipError_t e2 = hipSuccess;
+    if (e == hipSuccess) {
+        e2 = dispatch_batch(bg->tune, bg->prm, bg->dtype, bg->pow2, plan, bg->d_jobs, p, q,
+                            dim3(frame_groups(p), q.njobs), bg->d_counters, cs);
+        e = hipStreamEndCapture(cs, &k.graph);
+    }
+    (void)hipStreamDestroy(cs);
+    if (e == hipSuccess) e = e2;
+    if (e == hipSuccess) e = hipGraphInstantiate(&k.exec, k.graph, nullptr, nullptr, 0);
+    if (e != hipSuccess) {
+        if (k.graph) (void)hipGraphDestroy(k.graph);
+        return fail(c, SPR_ERR_HIP, "graph capture failed: %s", hipGetErrorString(e));
+    }
+    bg->captured.push_back(k);
+    return SPR_OK;
+}
+
+// Captures the plans that volumes of this kind may ask for, whatever voxels they hold
+int graph_capture(spr_ctx* c, spr_batch_graph* bg, BatchKind kind) {
+    const RayParams p = graph_params(bg);
+    int rc = SPR_OK;
+    for (const float need : {0.0f, 1.0f}) {  // (windows_pay is monotonic in need)
+        kind.need = need;
+        if (rc == SPR_OK)
+            rc = graph_capture(c, bg, uniform_plan(bg->tune, bg->prm, kind, p, (uint32_t)bg->n));
+    }
+    return rc;
 }
 
 // Enqueues the copy of a batch's job table to d_jobs on stream s from pinned host memory
@@ -1377,7 +1446,7 @@ int spr_render_batch(spr_ctx* c, const spr_params* params, const spr_job* jobs, 
     p.current_part = current_part;
     const BatchQueues q = make_queues(p, n);
     if (e == hipSuccess)
-        e = dispatch_batch(c, prm, kind, d_jobs, p, q, d_counters, s);
+        e = dispatch_batch(c->tune, prm, kind, d_jobs, p, q, d_counters, s);
     (void)hipFreeAsync(buf, s);
     HIPCALL(c, e);
     return SPR_OK;
@@ -1466,8 +1535,8 @@ int spr_render_frames(spr_ctx* c, const spr_frame* frames, int n, float alpha_po
     staged_tuning(c->tune, p);
     p.nouter = host[0].nouter;
     p.current_part = 0;
-    const bool windows = batch_windows(c, prm, kind, groups, 1, step);
-    if (windows) {  // each frame's first workgroup
+    const BatchPlan plan{batch_windows(c->tune, prm, kind, groups, 1, step), stops, windows_group(step), ch};
+    if (plan.windows) {  // each frame's first workgroup
         uint32_t first = 0;
         for (BatchJob& b : host) {
             b.first[0] = first;
@@ -1481,8 +1550,8 @@ int spr_render_frames(spr_ctx* c, const spr_frame* frames, int n, float alpha_po
     uint32_t* d_counters = (uint32_t*)((char*)buf + jbytes);
     hipError_t e = stage_jobs(c, host.data(), jbytes, d_jobs, s);
     if (e == hipSuccess)
-        e = dispatch_batch(c, prm, kind, ch, d_jobs, p, q, windows, stops, dim3((uint32_t)groups),
-                           step, d_counters, s);
+        e = dispatch_batch(c->tune, prm, kind.dtype, kind.pow2, plan, d_jobs, p, q,
+                           dim3((uint32_t)groups), d_counters, s);
     (void)hipFreeAsync(buf, s);
     HIPCALL(c, e);
     return SPR_OK;
@@ -1585,7 +1654,7 @@ int spr_render_batch_noalloc(spr_ctx* c, const spr_params* params, const spr_job
     p.nouter = (prm.max_steps / num_parts) / kLoopUnroll;
     p.current_part = current_part;
     const BatchQueues q = make_queues(p, n);
-    HIPCALL(c, dispatch_batch(c, prm, kind, d_jobs, p, q, d_counters, s));
+    HIPCALL(c, dispatch_batch(c->tune, prm, kind, d_jobs, p, q, d_counters, s));
     // blocking: the next call may overwrite the staging table and the scratch
     HIPCALL(c, hipStreamSynchronize(s));
     return SPR_OK;
@@ -1681,6 +1750,8 @@ int spr_batch_graph_create(spr_ctx* c, const spr_job* jobs, int n, int w, int h,
     bg->n = n;
     bg->w = w;
     bg->h = h;
+    bg->prm = c->params;
+    bg->tune = c->tune;
     bg->dtype = kind.dtype;
     bg->pow2 = kind.pow2;
     record_refs(c, jobs, n, bg->refs);
@@ -1695,28 +1766,8 @@ int spr_batch_graph_create(spr_ctx* c, const spr_job* jobs, int n, int w, int h,
         hipSuccess)
         return cleanup(fail(c, SPR_ERR_HIP, "job upload failed"));
     rc = check_parts(c, c->params, 1);
+    if (rc == SPR_OK) rc = graph_capture(c, bg, kind);
     if (rc) return cleanup(rc);
-    RayParams p = make_params(c, w, h);
-    staged_tuning(c->tune, p);
-    p.nouter = c->params.max_steps / kLoopUnroll;
-    p.current_part = 0;
-    const BatchQueues q = make_queues(p, n);
-    hipStream_t cs;
-    if (hipStreamCreateWithFlags(&cs, hipStreamNonBlocking) != hipSuccess)
-        return cleanup(fail(c, SPR_ERR_HIP, "capture stream"));
-    hipError_t e = hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal);
-    hipError_t e2 = hipSuccess;
-    if (e == hipSuccess) {
-        // the box length follows the captured jobs' volumes (speed only, never results)
-        e2 = dispatch_batch(c, c->params, kind, bg->d_jobs, p, q, bg->d_counters, cs);
-        e = hipStreamEndCapture(cs, &bg->graph);
-    }
-    (void)hipStreamDestroy(cs);
-    if (e != hipSuccess || e2 != hipSuccess)
-        return cleanup(fail(c, SPR_ERR_HIP, "graph capture failed: %s",
-                            hipGetErrorString(e != hipSuccess ? e : e2)));
-    if (hipGraphInstantiate(&bg->exec, bg->graph, nullptr, nullptr, 0) != hipSuccess)
-        return cleanup(fail(c, SPR_ERR_HIP, "graph instantiation failed"));
     *out = bg;
     return SPR_OK;
 }
@@ -1739,6 +1790,8 @@ int spr_batch_graph_update(spr_ctx* c, spr_batch_graph* bg, const spr_job* jobs,
                     "(capture a new graph)", bg->pow2 ? "all have" : "do not all have",
                     kind.pow2 ? "do" : "do not");
     DeviceGuard g(c->device);
+    rc = graph_capture(c, bg, kind);
+    if (rc) return rc;
     if (bg->last_stream) HIPCALL(c, hipStreamSynchronize(bg->last_stream));
     HIPCALL(c, hipMemcpy(bg->d_jobs, host.data(), (size_t)n * sizeof(BatchJob),
                          hipMemcpyHostToDevice));
@@ -1748,17 +1801,25 @@ int spr_batch_graph_update(spr_ctx* c, spr_batch_graph* bg, const spr_job* jobs,
 
 int spr_batch_graph_launch(spr_ctx* c, spr_batch_graph* bg, void* stream) {
     if (!c) return fail(nullptr, SPR_ERR_INVALID_ARG, "NULL context");
-    if (!bg || !bg->exec) return fail(c, SPR_ERR_INVALID_ARG, "NULL graph");
+    if (!bg) return fail(c, SPR_ERR_INVALID_ARG, "NULL graph");
+    BatchKind kind;  // of the volumes as they are now
+    kind.dtype = bg->dtype;
     for (const auto& r : bg->refs) {
         const VolSlot* vs = slot_of(c, r.first);
         if (!vs || vs->generation != r.second)
             return fail(c, SPR_ERR_INVALID_ARG,
                         "slot %d was released or refilled since the graph's jobs were set "
                         "(spr_batch_graph_update or a new graph)", r.first);
+        kind.nmax = std::max(kind.nmax, std::max(vs->nx, std::max(vs->ny, vs->nz)));
+        kind.need = std::max(kind.need, vs->need);
     }
     DeviceGuard g(c->device);
     hipStream_t s = stream ? (hipStream_t)stream : c->stream;
-    HIPCALL(c, hipGraphLaunch(bg->exec, s));
+    const BatchPlan plan = uniform_plan(bg->tune, bg->prm, kind, graph_params(bg), (uint32_t)bg->n);
+    hipGraphExec_t exec = bg->captured[0].exec;
+    for (const auto& k : bg->captured)
+        if (k.plan == plan) exec = k.exec;
+    HIPCALL(c, hipGraphLaunch(exec, s));
     bg->last_stream = s;
     return SPR_OK;
 }
@@ -1769,8 +1830,10 @@ int spr_batch_graph_destroy(spr_ctx* c, spr_batch_graph* bg) {
         DeviceGuard g(c->device);
         if (bg->last_stream) (void)hipStreamSynchronize(bg->last_stream);
     }
-    if (bg->exec) (void)hipGraphExecDestroy(bg->exec);
-    if (bg->graph) (void)hipGraphDestroy(bg->graph);
+    for (const auto& k : bg->captured) {
+        (void)hipGraphExecDestroy(k.exec);
+        (void)hipGraphDestroy(k.graph);
+    }
     if (bg->d_jobs) (void)hipFree(bg->d_jobs);
     if (bg->d_counters) (void)hipFree(bg->d_counters);
     delete bg;
