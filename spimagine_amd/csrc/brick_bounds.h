@@ -21,7 +21,10 @@
 // lies between its two endpoints exactly and the sample lies in [min, max] of its corners.
 // For float voxels each lerp can leave that interval by a few ulps of the corners'
 // magnitude; float bounds are widened by 2^-16 of the magnitude (plus 1e-30 for
-// denormals), far above the at most ~9 ulps three lerps can add.
+// denormals), far above the at most ~9 ulps three lerps can add.  Where all voxels are equal
+// the lerps are exact and the bounds stay as they are: rays through empty parts of a volume
+// (all 0) then have nothing to sample (256^3 float, one voxel in 2,000 set, 800^2 frame, 448
+// steps: 685 us with those widened too, 434 staged, 295 now).
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -67,10 +70,13 @@ __host__ __device__ inline float key_value(uint32_t k) {
 // widening of a float bound (see the file comment); integer voxels need none
 template <typename T>
 __device__ __forceinline__ float bound_margin(float lo, float hi) {
-    if constexpr (std::is_same<T, float>::value)
+    if constexpr (std::is_same<T, float>::value) {
+        // a lerp of equal values is exact (and infinite ones make NaN)
+        if (lo == hi && fabsf(hi) < __builtin_inff()) return 0.0f;
         return fmaxf(fabsf(lo), fabsf(hi)) * 0x1p-16f + 1e-30f;
-    else
+    } else {
         return 0.0f;
+    }
 }
 
 // Windows of a padded volume (see the file comment): g* = entries per axis

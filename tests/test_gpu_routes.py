@@ -1,0 +1,117 @@
+"""GPU: the march that the default tuning picks for a frame or a batch is not slower than the
+staged one (a chunk length picks that, SPR_TUNE_CHUNK), on volumes that leave little to skip or
+whose bounds promise more than they keep; and the frames are the same, bit for bit."""
+import numpy as np
+import pytest
+
+from spimagine_amd import _lib
+from spimagine_amd.utils import mat4_perspective, mat4_rotation, mat4_translate
+from spimagine_amd.volumerender.volumerender import render_matrices
+
+pytestmark = pytest.mark.gpu
+
+TOP = {np.uint16: 3000., np.uint8: 200., np.float32: 1.}
+
+
+def volume(torch, kind, dtype, shape):
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(3)
+
+    def uniform(*s):
+        return torch.rand(s, generator=gen, device="cuda")
+
+    def normal(*s):
+        return torch.randn(s, generator=gen, device="cuda")
+
+    if kind == "noise":
+        v = uniform(*shape)
+    elif kind == "points":  # one voxel in 2,000 over nothing
+        v = (uniform(*shape) > .9995) * uniform(*shape)
+    elif kind == "grain":  # coarse noise over fine
+        small = normal(1, 1, *[max(2, n // 8) for n in shape])
+        v = torch.nn.functional.interpolate(small, size=shape, mode="trilinear")[0, 0]
+        v = .5 + .15 * v + .02 * normal(*shape)
+    elif kind == "noisy spots":
+        v = torch.zeros(shape, device="cuda")
+        rng = np.random.default_rng(4)
+        for c in rng.integers(8, [n - 8 for n in shape], (int(np.prod(shape) / 50000.), 3)):
+            z, y, x = [int(n) for n in c]
+            v[z - 4:z + 5, y - 4:y + 5, x - 4:x + 5] += float(rng.uniform(.2, 1.))
+        v = v + .1 + .3 * normal(*shape)
+    v = (v * TOP[dtype]).clamp(0, 255 if dtype == np.uint8 else 32767)
+    kinds = {np.uint16: torch.int16, np.uint8: torch.uint8, np.float32: torch.float32}
+    return (v if dtype == np.float32 else v.round()).to(kinds[dtype]).contiguous()
+
+
+def times(torch, s, ctx, go, chunks):
+    """The least time of each chunk setting (0: the default), taken in turn."""
+    best = {k: 1e9 for k in chunks}
+    for _ in range(7):
+        for k in chunks:
+            ctx.set_tuning("chunk", k)
+            go()
+            e = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+            e[0].record(s)
+            for _ in range(4):
+                go()
+            e[1].record(s)
+            e[1].synchronize()
+            best[k] = min(best[k], e[0].elapsed_time(e[1]) * 250.)
+    return best
+
+
+# (how, voxel type, volume, shape, frame size, steps, frames); slower by half or more before
+ROUTES = [
+    # bounds of empty float windows were widened above the ray's zero, and each was sampled
+    ("frame", np.float32, "points", (256, 256, 256), 800, 448, 1),
+]
+
+
+@pytest.mark.parametrize("how,dtype,kind,shape,size,steps,n", ROUTES)
+def test_default_march_is_not_slower(how, dtype, kind, shape, size, steps, n):
+    import torch
+    ctx = _lib.Context(0)
+    vol = volume(torch, kind, dtype, shape)
+    torch.cuda.synchronize()
+    slot = ctx.volume_add(dev_ptr=vol.data_ptr(), dtype=dtype, shape=shape)
+    s = torch.cuda.Stream()
+    o = torch.zeros((n, 7, size, size), device="cuda")
+    ps = []
+    for k in range(n):
+        M = np.dot(mat4_translate(0, 0, -3.2), mat4_rotation(.6 + .5 * k, .3, 1, -.2))
+        iP, iM = render_matrices(M, mat4_perspective(45, 1., .1, 10), shape[::-1])
+        ps.append(_lib.make_params(iP, iM, min_val=0., max_val=TOP[dtype], max_steps=steps,
+                                   filter=_lib.FILTER_NEAREST if how.endswith("nearest") else
+                                   _lib.FILTER_LINEAR))
+    at = [[o[k, j].data_ptr() for j in range(5)] for k in range(n)]
+    jobs = ctx.make_jobs([(slot, list(p.inv_p), list(p.inv_m), a[0], a[1]) for p, a in zip(ps, at)])
+    frames = [_lib.make_frame(slot, p, size, size, a[0], a[1]) for p, a in zip(ps, at)]
+
+    def go():
+        st = s.cuda_stream
+        if how.startswith("frame"):
+            ctx.render_slot(slot, ps[0], _lib.METHOD_MAX_PROJECT, size, size, at[0][0], at[0][1], stream=st)
+        elif how == "iso":
+            ctx.render_slot(slot, ps[0], _lib.METHOD_ISO_SURFACE, size, size, at[0][0], at[0][1], at[0][2],
+                            at[0][4], at[0][3], stream=st)
+        elif how.startswith("batch"):
+            ctx.render_batch(jobs, size, size, params=ps[0], stream=st)
+        else:
+            ctx.render_frames_split(frames, stream=st)
+
+    torch.cuda.synchronize()
+    outs = []
+    for chunk in (0, 16):
+        ctx.set_tuning("chunk", chunk)
+        o.fill_(-1.)
+        torch.cuda.synchronize()
+        go()
+        s.synchronize()
+        outs.append(o.clone())
+    assert torch.equal(outs[0], outs[1])
+    best = times(torch, s, ctx, go, (0, 8, 16, 32))
+    staged = min(v for k, v in best.items() if k)
+    print("%s %s %s %s %d^2 %d steps: default %.0f us, staged %.0f us" % (
+        how, np.dtype(dtype).name, kind, shape, size, steps, best[0], staged), flush=True)
+    ctx.close()
+    assert best[0] <= 1.2 * staged
