@@ -155,35 +155,48 @@ __host__ inline int windows_group(float step) {
     return 3.0f * step <= 2.9f ? 4 : step <= 2.9f ? 2 : 1;
 }
 
-// Whether the frame is gathered group by group (k_mip_windows) instead of staged box by box.
-// need: the volume's share of windows to sample (k_window_need); step: voxels a sample;
-// tiles: 8x8 pixel quarters.  Trilinear samples gathered cost ~1.5 times staged ones at a
-// fine step, so most groups have to fall away there; from 1.5 voxels a step on a staged box
-// holds few samples of many voxels, and a frame of few rays leaves most of the GPU idle
-// unless their segments are marched side by side.  A nearest sample is one load, cheaper
-// than its share of a staged box unless rays are short and leave little to skip.  In volumes
-// of few voxels (nmax, the largest dimension) most of a march is its set-up and first samples,
-// which side by side pay only while they leave the GPU idle.
-// us staged / gathered, 800^2 frames, linear:
-//   512^3 blobs, uint16 (need 0.044): 896 steps 760 / 530, 200 steps 386 / 202
-//   256^3 blobs, uint16 (0.078): 448 steps 357 / 303, 200 steps 226 / 178
-//   256^3 blobs, float (0.097): 448 steps 316 / 303, 200 steps 215 / 185
-//   256x256x128 blobs, uint16 (0.107): 384 steps 259 / 254, 200 steps 188 / 172
-//   256x256x128 blobs, float (0.141): 384 steps 225 / 250
-//   128^3 blobs, uint16 (0.28): 200 steps 189 / 212
-//   256^3 white noise, uint16 (1.0): 448 steps 401 / 534, 200 steps 248 / 300
-//   200^2 frames: 128^3 float blobs (0.42), 200 steps 79 / 43; 96^3 uint16 (0.32) 47 / 48
-// nearest:
-//   512^3 blobs, uint16: 896 steps 502 / 265, 200 steps 325 / 111
-//   256^3 white noise, uint16: 448 steps 247 / 234, 200 steps 176 / 145
-//   128^3 blobs, float (0.42): 224 steps 134 / 131, 200 steps 124 / 132
-//   48^3 .. 80^3 blobs: 200^2 .. 600^2 frames 17-92 / 18-95, 12% slower at the median; 130^2
-//   frames 18-50 / 17-29
-__host__ inline bool windows_pay(bool nearest, float need, int nmax, float step, uint64_t tiles) {
+// Whether frames are gathered group by group (k_mip_windows) instead of staged box by box, or
+// read sample by sample from the persistent queues (batches with the nearest filter).
+// need: the volume's share of windows to sample (k_ray_need); step: voxels a sample;
+// tiles: 8x8 pixel quarters of all frames.
+//
+// A gathered trilinear sample costs ~1.5 times a staged one at a fine step, so most groups have
+// to fall away there.  From 1.5 voxels a step on a staged box holds few samples of many voxels,
+// and a frame of fewer quarters than waves fit the GPU (2,048) leaves it idle unless its rays'
+// segments are marched side by side, all of it below a third of that.  A nearest sample is one
+// load, cheaper than its share of a staged box unless rays are short and leave little to skip;
+// the queues' are as cheap as a lookup while neighbouring rays share the lines of a volume that
+// the caches hold, and few tiles leave the queues' workgroups idle.  In volumes of few voxels
+// (nmax, the largest dimension) most of a march is its set-up and first samples.
+//
+// Each line lies below the smallest need at which one of 15 kinds of volume (blobs in noise of
+// 0.5 to 30% of their height, spots in noise, textures, white noise, sparse voxels, labels, a
+// shell; 112 to 512 voxels, uint16 and float) ran more than 3-6% slower gathered.  us staged /
+// gathered there:
+//   linear, from 224 voxels: 0.55 at coarse steps: shell (need 0.57), 384^3, 1000^2, 200 steps 281 / 340;
+//     0.35 and 0.23 (from 320) at fine ones: float texture (0.39) 256^3, 1000^2, 448 steps 366 / 425,
+//     512^3 (0.26), 768 steps 571 / 617, gained below: blobs (0.13) 571 / 520, batches of it 0.65
+//   192^3: 0.4 and 0.27: texture (0.43), 24 x 500^2, 112 steps 1447 / 1620; float blobs (0.29), 1000^2,
+//     336 steps 282 / 330; 112^3 and 128^3: 0.3: texture (0.34), 6 x 800^2, 200 steps 950 / 1130
+//   fewer than 2,048 quarters: texture (0.43), 192^3, 340^2, 200 steps 77 / 85; fewer than 700: every
+//     volume gained, 128^3 blobs 57 / 31, white noise 78 / 47, but for steps of 3 voxels (shell, 0.57)
+//   nearest, from 224 voxels: 0.55: float shell (0.57) 384^3, 260^2, 200 steps 65 / 70; 192^3: 0.4:
+//     texture (0.43), 1000^2, 200 steps 124 / 141; smaller: labels (0.10), 1000^2, 112 steps 86 / 95
+//   nearest batches, fewer than 20,000 quarters: 0.55: 112^3 shell (0.65), 24 x 200^2 320 / 346; above:
+//     shell (0.57) 384^3, 6 x 800^2 911 / 966; texture (0.39) 256^3, 448 steps 1010 / 1050; labels
+//     (0.10) 128^3, 24 x 500^2, 112 steps 22% slower, blobs (0.15) 256^3, 200 steps 604 / 713
+__host__ inline bool windows_pay(bool nearest, bool batch, float need, int nmax, float step,
+                                 uint64_t tiles) {
     if (nmax < 112 && tiles >= 512u) return false;
-    if (nearest) return need < 0.2f || step >= 1.25f || tiles < 2048u;
-    if (step >= 1.5f || tiles < 2048u) return need < 0.6f;
-    return need < 0.11f;
+    if (tiles < 700u) return step < 3.0f || need < 0.55f;
+    const bool coarse = step >= 1.5f || tiles < 2048u;
+    if (nearest && batch && tiles >= 20000u)
+        return nmax >= 320 ? need < 0.5f : nmax >= 224 && step < 1.0f && need < 0.35f;
+    if (nearest && nmax < 160 && !batch && tiles >= 4000u) return false;
+    if (nearest) return need < (nmax >= 160 && nmax < 224 && !batch ? 0.4f : 0.55f);
+    if (nmax < 160) return need < 0.3f;
+    if (nmax < 224) return need < (coarse ? 0.4f : 0.27f);
+    return need < (coarse ? 0.55f : nmax < 320 ? 0.35f : 0.23f);
 }
 
 // the rays of a workgroup: which lanes have one, sample 0 and step

@@ -408,6 +408,14 @@ hipError_t launch_pad(const VolSlot& vs, const void* src, int sz0, uint32_t bz0,
     return hipGetLastError();
 }
 
+// The share of the windows that a max projection has to sample: *sum is its rays', from 0
+template <typename T>
+void launch_need(const VolSlot& vs, uint32_t* sum, hipStream_t s) {
+    hipLaunchKernelGGL(k_ray_need<T>, dim3(kNeedRays * kNeedRays, 3), dim3(64), 0, s, (const T*)vs.d_pad,
+                       vs.nx, vs.ny, vs.nz, (const T*)vs.win_max(), vs.win[0], vs.win[1], vs.win[2], sum);
+}
+float need_of(uint32_t sum) { return (float)sum / (65536.0f * 3.0f * kNeedRays * kNeedRays); }
+
 // The window grid and the brick keys from the block bounds; *total: the volume's keys
 template <typename T>
 void launch_windows(const VolSlot& vs, const void* blocks, BrickKey* total, hipStream_t s) {
@@ -416,10 +424,7 @@ void launch_windows(const VolSlot& vs, const void* blocks, BrickKey* total, hipS
     hipLaunchKernelGGL(k_block_windows<T>, grid, dim3(256), 0, s, (const BlockBounds<T>*)blocks,
                        padded_pitch<T>(vs.nx) / 4u, gx, gy, gz, (T*)vs.win_max(), (T*)vs.win_min(),
                        vs.nbx, vs.nby, vs.d_bricks, total);
-    const uint32_t cols = std::max(gx * gy, std::max(gy * gz, gx * gz));
-    hipLaunchKernelGGL(k_window_need<T>, dim3(std::min((cols + 255u) / 256u, 256u), 3), dim3(256), 0,
-                       s, (const T*)vs.win_max(), (const T*)vs.win_min(), gx, gy, gz,
-                       (uint32_t*)(total + 1));
+    launch_need<T>(vs, (uint32_t*)(total + 1), s);
 }
 
 // out(x, y, z) = max of in over [c - r, c + r] along AXIS (0 x, 1 y, 2 z), coordinates
@@ -571,16 +576,14 @@ hipError_t pair_windows(spr_ctx* c, VolSlot& vs) {
                            vs.ny, vs.nz, gx, gy, blocks);
         hipLaunchKernelGGL(k_pair_windows, grid, block, 0, c->stream, (const uint32_t*)blocks, gx, gy,
                            gz, wmax);
-        const uint32_t cols = std::max(gx * gy, std::max(gy * gz, gx * gz));
-        hipLaunchKernelGGL(k_pair_need, dim3(std::min((cols + 255u) / 256u, 256u), 3), block, 0,
-                           c->stream, (const uint32_t*)wmax, gx, gy, gz, count);
+        launch_need<U16Pair>(vs, count, c->stream);
         e = hipGetLastError();
     }
     if (e == hipSuccess)
         e = hipMemcpyAsync(&needed, count, sizeof(needed), hipMemcpyDeviceToHost, c->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     (void)hipFreeAsync(count, c->stream);
-    vs.need = (float)needed / (3.0f * (float)gx * (float)gy * (float)gz);
+    vs.need = need_of(needed);
     return e;
 }
 
@@ -679,7 +682,7 @@ int fill_slot(spr_ctx* c, VolSlot& vs, const void* src, bool src_on_device, int 
         const size_t nbricks = (size_t)nbx * nby * nbz;
         if (want_bounds && !vs.d_bricks) {
             realloc = true;
-            // two more entries: the volume's bounds, the count of k_window_need
+            // two more entries: the volume's bounds, the sum of k_ray_need
             HIPCALL(c, hipMalloc(&vs.d_bricks, vs.brick_alloc()));
         }
         // the 4x4x4 block bounds live from the padding pass to the windows' only
@@ -711,7 +714,7 @@ int fill_slot(spr_ctx* c, VolSlot& vs, const void* src, bool src_on_device, int 
             const BrickKey k = t.keys;
             vs.vmin = dtype == SPR_DTYPE_F32 ? key_value<float>(k.kmin) : (float)k.kmin;
             vs.vmax = dtype == SPR_DTYPE_F32 ? key_value<float>(~k.nkmax) : (float)~k.nkmax;
-            vs.need = (float)t.needed / (3.0f * (float)win[0] * (float)win[1] * (float)win[2]);
+            vs.need = need_of(t.needed);
         } else if (e == hipSuccess) {
             e = pair_windows(c, vs);
         }
@@ -812,8 +815,7 @@ bool batch_windows(const LaunchTuning& t, const spr_params& prm, const BatchKind
                    uint64_t gy, float step) {
     return prm.alpha_pow == 0.0f && windows_tuning(t) && gx <= kWinMaxGroups &&
            gy <= 65535u &&
-           windows_pay(prm.filter == SPR_FILTER_NEAREST, kind.need, kind.nmax, step,
-                       gx * gy);
+           windows_pay(prm.filter == SPR_FILTER_NEAREST, true, kind.need, kind.nmax, step, gx * gy);
 }
 
 bool opacity_asks(int dtype, uint32_t tiles, int nmax, int nouter) {
@@ -1567,8 +1569,10 @@ int spr_render_frames_split(spr_ctx* c, const spr_frame* frames, int n, int seg,
     BatchKind kind;
     int rc = frames_to_jobs(c, frames, n, host, &kind);
     if (rc) return rc;
-    // rays far apart share no voxels, so a volume whose windows leave enough to skip is
-    // gathered by them (8 frames of 64 x 64 rays of a 512^3 volume, 896 steps: staged 1.03 ms)
+    // rays far apart share no voxels, so volumes whose windows leave enough to skip are gathered
+    // by them.  us staged / gathered: 6 frames of 200^2 of 512^3 blobs (need 0.10), 768 steps
+    // 999 / 350, shell (0.57) 384^3, 200 steps 793 / 896, texture (0.34) 128^3 149 / 158; 8 of 64^2 of
+    // textures (0.16) 384^3, 112 steps 140 / 157, (0.26) 512^3, 768 steps 272 / 310
     uint64_t groups = 0;
     float step = 0.0f;
     int ch = kLoopUnroll;
@@ -1580,7 +1584,8 @@ int spr_render_frames_split(spr_ctx* c, const spr_frame* frames, int n, int seg,
         b.first[0] = (uint32_t)groups;
         groups += 4u * tile_grid(kTileMapInterleaved, (b.W + 15u) / 16u, (b.H + 15u) / 16u);
     }
-    const bool windows = windows_tuning(c->tune) && groups <= kWinMaxGroups && kind.need < 0.6f;
+    const bool windows = windows_tuning(c->tune) && groups <= kWinMaxGroups &&
+                         kind.need < (groups < 1500u ? 0.15f : kind.nmax < 160 ? 0.3f : 0.5f);
     // else job k's first work item (8 x 8 rays x one segment) and first pixel; staged in LDS
     // slabs (tuning slab_kb > 0) when every frame's ray step allows 16-sample boxes
     uint64_t items = 0, pix = 0;

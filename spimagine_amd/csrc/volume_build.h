@@ -190,51 +190,59 @@ static __global__ __launch_bounds__(256) void k_pair_windows(const uint32_t* __r
     wmax[((size_t)z * gy + y) * gx + x] = m;
 }
 
-// k_window_need of a pair: a window that either channel needs, levels at three quarters of
-// the column's maximum (a pair keeps no minima)
-static __global__ __launch_bounds__(256) void k_pair_need(const uint32_t* __restrict__ wmax,
-                                                          uint32_t gx, uint32_t gy, uint32_t gz,
-                                                          uint32_t* __restrict__ count) {
-    const uint32_t n[3] = {gx, gy, gz}, stride[3] = {1u, gx, gx * gy};
-    const uint32_t a = blockIdx.y, b = a == 0 ? 1u : 0u, c = a == 2 ? 1u : 2u;
-    uint32_t need = 0;
-    for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < n[b] * n[c]; i += gridDim.x * 256u) {
-        const uint32_t ic = i / n[b], first = (i - ic * n[b]) * stride[b] + ic * stride[c];
-        uint32_t top = 0;
-        for (uint32_t k = 0; k < n[a]; ++k) top = pair_max(top, wmax[first + k * stride[a]]);
-        for (uint32_t k = 0; k < n[a]; ++k) {
-            const uint32_t v = wmax[first + k * stride[a]];
-            need += 4u * (v & 0xFFFFu) > 3u * (top & 0xFFFFu) || 4u * (v >> 16) > 3u * (top >> 16) ? 1u : 0u;
-        }
-    }
-    for (int off = 32; off > 0; off >>= 1) need += (uint32_t)__shfl_xor((int)need, off);
-    if ((threadIdx.x & 63u) == 0u) atomicAdd(count, need);
+// Share of the windows that a max projection has to sample, measured along kNeedRays x kNeedRays
+// rays parallel to each axis, between the voxels: the windows of a ray whose maximum exceeds the
+// ray's own (a pair's: in either channel).  One wave a ray; *sum: the rays' shares, 16 bits each.
+//
+// Windows alone do not tell: where few voxels are bright or noise is strong a ray seldom meets a
+// window's maximum.  Against three quarters of the best window of a column, which was counted
+// before, this misjudged half as often by how much the better march would have gained (0.8% of
+// the time of frames on average instead of 1.1, batches 1.4 instead of 2.6).
+constexpr uint32_t kNeedRays = 16;
+
+__device__ __forceinline__ float2 need_value(float v) { return make_float2(v, 0.0f); }
+__device__ __forceinline__ float2 need_value(uint16_t v) { return make_float2((float)v, 0.0f); }
+__device__ __forceinline__ float2 need_value(uint8_t v) { return make_float2((float)v, 0.0f); }
+__device__ __forceinline__ float2 need_value(U16Pair v) {
+    return make_float2((float)(v.bits & 0xFFFFu), (float)(v.bits >> 16));
 }
 
-// Share of the windows that a max projection along the volume's axes would have to sample:
-// *count windows, over the columns of each axis (grid.y: axis), whose maximum exceeds three
-// quarters of the way from the minimum to the maximum of the column's best window.  1 for
-// white noise, 0.04-0.35 for blobs over camera noise.
 template <typename T>
-__global__ __launch_bounds__(256) void k_window_need(const T* __restrict__ wmax,
-                                                     const T* __restrict__ wmin, uint32_t gx,
-                                                     uint32_t gy, uint32_t gz,
-                                                     uint32_t* __restrict__ count) {
-    const uint32_t n[3] = {gx, gy, gz}, stride[3] = {1u, gx, gx * gy};
-    const uint32_t a = blockIdx.y, b = a == 0 ? 1u : 0u, c = a == 2 ? 1u : 2u;
-    uint32_t need = 0;
-    for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < n[b] * n[c]; i += gridDim.x * 256u) {
-        const uint32_t ic = i / n[b], first = (i - ic * n[b]) * stride[b] + ic * stride[c];
-        float level = 0.0f;
-        for (uint32_t k = 0; k < n[a]; ++k) {
-            const uint32_t o = first + k * stride[a];
-            level = fmaxf(level, 0.25f * (float)wmin[o] + 0.75f * (float)wmax[o]);
+__global__ __launch_bounds__(64) void k_ray_need(const T* __restrict__ pad, int nx, int ny, int nz,
+                                                 const T* __restrict__ wmax, uint32_t gx, uint32_t gy,
+                                                 uint32_t gz, uint32_t* __restrict__ sum) {
+    const uint32_t n[3] = {(uint32_t)nx, (uint32_t)ny, (uint32_t)nz}, g[3] = {gx, gy, gz};
+    const size_t pitch = padded_pitch<T>(nx), stride[3] = {1, pitch, pitch * (n[1] + 2u)};
+    const size_t wstride[3] = {1, gx, (size_t)gx * gy};
+    const uint32_t a = blockIdx.y, b = a == 0 ? 1u : 0u, c = a == 2 ? 1u : 2u, lane = threadIdx.x;
+    const uint32_t rb = blockIdx.x % kNeedRays, rc = blockIdx.x / kNeedRays;
+    const uint32_t ib = min(1u + (rb * n[b] + n[b] / 2u) / kNeedRays, n[b]),
+                   ic = min(1u + (rc * n[c] + n[c] / 2u) / kNeedRays, n[c]);
+    const T* at = pad + ib * stride[b] + ic * stride[c];
+    float top = 0.0f, top2 = 0.0f;
+    for (uint32_t k = lane; k <= n[a]; k += 64u) {
+        float s = 0.0f, s2 = 0.0f;
+#pragma unroll
+        for (uint32_t j = 0; j < 8u; ++j) {
+            const float2 v = need_value(at[(k + (j & 1u)) * stride[a] + (j >> 1 & 1u) * stride[b] + (j >> 2) * stride[c]]);
+            s += v.x;
+            s2 += v.y;
         }
-        for (uint32_t k = 0; k < n[a]; ++k)
-            need += (float)wmax[first + k * stride[a]] > level ? 1u : 0u;
+        top = fmaxf(top, 0.125f * s);
+        top2 = fmaxf(top2, 0.125f * s2);
     }
-    for (int off = 32; off > 0; off >>= 1) need += (uint32_t)__shfl_xor((int)need, off);
-    if ((threadIdx.x & 63u) == 0u) atomicAdd(count, need);
+    for (int o = 32; o > 0; o >>= 1) {
+        top = fmaxf(top, __shfl_xor(top, o));
+        top2 = fmaxf(top2, __shfl_xor(top2, o));
+    }
+    const T* w = wmax + (ib >> kWinShift) * wstride[b] + (ic >> kWinShift) * wstride[c];
+    uint32_t need = 0;
+    for (uint32_t k = lane; k < g[a]; k += 64u) {
+        const float2 v = need_value(w[k * wstride[a]]);
+        need += v.x > top || v.y > top2 ? 1u : 0u;
+    }
+    for (int o = 32; o > 0; o >>= 1) need += (uint32_t)__shfl_xor((int)need, o);
+    if (lane == 0u) atomicAdd(sum, (need << 16) / g[a]);
 }
 
 }  // namespace spr

@@ -60,10 +60,18 @@ def times(torch, s, ctx, go, chunks):
     return best
 
 
-# (how, voxel type, volume, shape, frame size, steps, frames); slower by half or more before
+# (how, voxel type, volume, shape, frame size, steps, frames)
 ROUTES = [
     # bounds of empty float windows were widened above the ray's zero, and each was sampled
     ("frame", np.float32, "points", (256, 256, 256), 800, 448, 1),
+    # more windows to sample than their gain paid for
+    ("batch nearest", np.uint16, "noise", (256, 256, 256), 800, 200, 6),
+    ("batch nearest", np.float32, "points", (128, 128, 128), 800, 200, 6),
+    ("batch nearest", np.uint8, "grain", (192, 192, 192), 800, 200, 6),
+    ("batch", np.uint16, "noisy spots", (256, 512, 512), 800, 200, 6),
+    ("frame", np.uint16, "noisy spots", (384, 384, 384), 520, 200, 1),
+    ("split", np.uint16, "noisy spots", (256, 512, 512), 200, 200, 6),
+    ("split", np.uint8, "grain", (128, 128, 128), 200, 224, 6),
 ]
 
 
