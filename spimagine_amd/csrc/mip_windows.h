@@ -81,7 +81,8 @@ struct WindowRay {
         wy = fmaf(0.25f, texel<V::kPow2>(py, vol.fny) + (1.0f - mgy), fminf(kBack * gy, 0.0f));
         wz = fmaf(0.25f, texel<V::kPow2>(pz, vol.fnz) + (1.0f - mgz), fminf(kBack * gz, 0.0f));
     }
-    // entries of the kWinGroups groups that start `ahead` groups past (px, py, pz)
+    // entries of kWinGroups groups, every APART-th from the one `ahead` groups past (px, py, pz)
+    template <int APART = 1>
     __device__ __forceinline__ void ask(const V& vol, float px, float py, float pz, float mgx,
                                         float mgy, float mgz, float ahead, const T* plane,
                                         T (&u)[kWinGroups]) const {
@@ -89,7 +90,7 @@ struct WindowRay {
         at(vol, px, py, pz, mgx, mgy, mgz, wx, wy, wz);
 #pragma unroll
         for (int j = 0; j < kWinGroups; ++j) {
-            const float f = ahead + (float)j;
+            const float f = ahead + (float)(APART * j);
             u[j] = plane[vol.window(fmaf(f, gx, wx), fmaf(f, gy, wy), fmaf(f, gz, wz))];
         }
     }
@@ -445,31 +446,43 @@ __global__ __launch_bounds__(64 * kWinSegments, (kWinWaves<T, GS, FILT>)) void k
 // Iso-surface march by the window grid (iso_kernel.cl:83-131, k_iso_surface): sample 0 sets a
 // ray's side, the first later sample on the other side is the crossing.  A group is sampled
 // only when its window reaches the other side of the iso value.  The four waves of an 8x8
-// quarter take every fourth run of kWinGroups groups, so they move front to back together
-// and stop together; waiting groups are queued and gathered 64 at a time as above, and a
-// crossing is posted as the least sample index.  The refinement, the gradient and the
-// shading then run per ray (iso_finish).
+// quarter take every fourth group each, so they move front to back together and stop together;
+// waiting groups are queued and gathered 64 at a time as above, a crossing is posted as the
+// least sample index, and no group past a posted one is queued: rays that cross at once (white
+// noise, 256^3 float, 800^2, 200 steps) take 259 us, 284 with every fourth run of eight groups
+// a wave and crossings looked up once a run, 250 staged.  Noise that reaches the iso value now and then
+// all along the rays stays 5-20% slower than staged: no window falls away.  The refinement, the
+// gradient and the shading then run per ray (iso_finish).
 //
 // Bound by VALU (65% busy; address units 40%): ~5 instructions a sample in windows on one
 // side, the rest in groups near surfaces, their exact positions and the finish.  512^3
-// uint16 -> 1024^2, 896 steps: frame 477 us (511 us with a lane taking a whole group); march
-// of the frame 412 us before that, 828 us staged with 8^3 brick tests of a wave's box.
+// uint16 -> 1024^2, 896 steps: frame 446 us (487 with runs of groups a wave and four waves a SIMD,
+// 511 with a lane taking a whole group; march of the frame 412 us before that, 828 us staged
+// with 8^3 brick tests of a wave's box).
 struct IsoWindowShared {
     float4 item[kWinSegments][128];  // position; w's bits: ray | side << 6 | first sample << 7
     SharedRays rays;
     uint64_t above;    // the rays that start above the iso value
     uint32_t hit[64];  // the rays' least crossing sample (~0: none)
 };
+// Waves per SIMD that the registers are held to: five (96), but for groups of four float samples,
+// which would spill 16.  The finish of a ray is one wave's work, so the workgroups resident count:
+// left alone uint8 frames took 139 registers.  us left alone / four / five, 1200^2 frames: 128^3
+// white noise, 112 steps, uint8 550 / 451 / 450, uint16 475 / 483 / 470; 512x512x256 blobs, 768 steps, uint8
+// 561 / 545 / 520, uint16 535 / 524 / 513.
+template <typename T, int GS>
+constexpr int kIsoWaves = std::is_same<T, float>::value && GS == 4 ? 4 : 5;
 constexpr uint32_t kIsoAnchor = 900;  // samples that a lookup may lie past an exact position
 constexpr int kIsoWindowMaxSteps = 1 << 24;
 
 template <typename T, bool POW2, int GS, bool WIDE, int FILT>
-__global__ __launch_bounds__(64 * kWinSegments) void k_iso_windows(
+__global__ __launch_bounds__(64 * kWinSegments, (kIsoWaves<T, GS>)) void k_iso_windows(
     PaddedVolume<T, POW2, WIDE> vol, RayParams p, float* __restrict__ out, float* __restrict__ alpha,
     float* __restrict__ depth, float* __restrict__ normals) {
     using PV = PaddedVolume<T, POW2, WIDE>;
     static_assert(FILT == 0 || !WIDE, "nearest: volumes below 4 GiB");
-    constexpr int BS = kWinGroups * GS, RS = kWinSegments * BS;
+    constexpr uint32_t NS = kWinSegments * GS, RS = kWinGroups * NS;  // samples from one of a wave's
+                                                                     // groups, runs to the next
     __shared__ IsoWindowShared sh;
     const uint32_t lane = threadIdx.x & 63u, seg = threadIdx.x >> 6;
     uint32_t x = 0, y = 0;
@@ -539,9 +552,9 @@ __global__ __launch_bounds__(64 * kWinSegments) void k_iso_windows(
     // (px, py, pz): the exact position of sample ka, a whole number of groups from k0 and at
     // most kIsoAnchor samples before the last one asked for; a run without waiting groups
     // moves only k0
-    uint32_t k0 = seg * (uint32_t)BS, ka = 0;
+    uint32_t k0 = seg * (uint32_t)GS, ka = 0;
     auto ask = [&](uint32_t k, T (&u)[kWinGroups]) {
-        win.ask(vol, px, py, pz, mgx, mgy, mgz, (float)((int)(k - ka) / GS), plane, u);
+        win.template ask<kWinSegments>(vol, px, py, pz, mgx, mgy, mgz, (float)((int)(k - ka) / GS), plane, u);
     };
     auto anchor = [&](uint32_t k) {
         px = sum_n(px, dx, k - ka);
@@ -551,16 +564,16 @@ __global__ __launch_bounds__(64 * kWinSegments) void k_iso_windows(
     };
     T cur[kWinGroups], nxt[kWinGroups];
     ask(k0, cur);
-    for (; k0 < nsteps; k0 += (uint32_t)RS) {
+    for (; k0 < nsteps; k0 += RS) {
         const uint32_t hit = min(nsteps, __hip_atomic_load(&sh.hit[lane], __ATOMIC_RELAXED,
                                                            __HIP_MEMORY_SCOPE_WORKGROUP));
         if (__ballot(active && k0 < hit) == 0) break;  // every ray has crossed before
-        if (k0 + (uint32_t)(RS + BS) > ka + kIsoAnchor) anchor(k0);
-        ask(k0 + (uint32_t)RS, nxt);
+        if (k0 + 2u * RS > ka + kIsoAnchor) anchor(k0);
+        ask(k0 + RS, nxt);
         uint32_t mask = 0, any = 0;  // groups that may cross: this ray's, some ray's (uniform)
 #pragma unroll
         for (int j = 0; j < kWinGroups; ++j) {
-            const uint32_t k = k0 + (uint32_t)(j * GS);
+            const uint32_t k = k0 + (uint32_t)(j * NS);
             const bool need = active && k < hit && (!win.ok || ((float)cur[j] > p.iso_val) != gt);
             mask |= need ? 1u << j : 0u;
             any |= __ballot(need) != 0 ? 1u << j : 0u;
@@ -568,21 +581,25 @@ __global__ __launch_bounds__(64 * kWinSegments) void k_iso_windows(
         }
         if (any == 0) continue;
         const uint32_t first = (uint32_t)__builtin_ctz(any);
-        anchor(k0 + first * (uint32_t)GS);
+        anchor(k0 + first * NS);
         float qx = px, qy = py, qz = pz;
         for (uint32_t j = first; any >> j != 0u; ++j) {
             if (any >> j & 1u) {
-                const bool need = (mask >> j & 1u) != 0;
+                // (not past a crossing that the groups before have shown)
+                const bool need = (mask >> j & 1u) != 0 &&
+                                  k0 + j * NS <
+                                      __hip_atomic_load(&sh.hit[lane], __ATOMIC_RELAXED,
+                                                        __HIP_MEMORY_SCOPE_WORKGROUP);
                 const uint64_t m = __ballot(need);
                 if (need)
                     item[waiting + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] =
                         float4{qx, qy, qz,
-                               __uint_as_float(lane | (gt ? 64u : 0u) | (k0 + j * (uint32_t)GS) << 7)};
+                               __uint_as_float(lane | (gt ? 64u : 0u) | (k0 + j * NS) << 7)};
                 waiting += (uint32_t)__popcll(m);
                 if (waiting >= 64u) take(64u);
             }
 #pragma unroll
-            for (int k = 0; k < GS; ++k) {
+            for (uint32_t k = 0; k < NS; ++k) {
                 qx = qx + dx;
                 qy = qy + dy;
                 qz = qz + dz;

@@ -72,6 +72,9 @@ ROUTES = [
     ("frame", np.uint16, "noisy spots", (384, 384, 384), 520, 200, 1),
     ("split", np.uint16, "noisy spots", (256, 512, 512), 200, 200, 6),
     ("split", np.uint8, "grain", (128, 128, 128), 200, 224, 6),
+    # rays that cross the iso value at once, with look-ahead for many groups
+    ("iso", np.uint8, "noise", (128, 128, 128), 1200, 112, 1),
+    ("iso", np.float32, "noise", (128, 128, 128), 800, 200, 1),
 ]
 
 
