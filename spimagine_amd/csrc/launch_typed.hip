@@ -357,10 +357,14 @@ hipError_t TypedLaunch<T, P2>::max_project(const LaunchTuning& t, const VolSlot&
     bool skip = t.skip != 0 && vs.d_bricks != nullptr && t.staging == 0 &&
                 (t.slab_kb == 19 || vs.pad_wide);
     // the opacity mode's stop test costs 1-3% where it can't stop a ray: integer volumes that
-    // reach below min_val, in frames that don't ask the windows
+    // reach far below min_val, where transparency may grow e-fold or more on the way
+    constexpr bool kInt = std::is_integral<T>::value;
     const uint32_t samples = (uint32_t)(p.nouter + 1) * kLoopUnroll;
-    const bool stops = !std::is_integral<T>::value || p.max_val == 0.0f || p.min_val <= vs.vmin ||
-                       opacity_windows<T>(4u * p.ntiles, (float)nmax, samples);
+    const float grow = opacity_exponent(kInt, p, vs.vmin, samples);
+    if (opac)
+        p.asks = opacity_windows(kInt, 4u * p.ntiles, nmax, samples, vs.need,
+                                 -opacity_exponent(kInt, p, vs.mean, samples), grow);
+    const bool stops = p.asks != 0u || !(grow > 1.0f);
     if (opac && !stops) skip = false;
     // the plain max projection's box lengths (chunk 0: from the ray step)
     if (t.chunk == 0 && !opac) p.box16 = staged_groups_mip(p.nouter, nmax);

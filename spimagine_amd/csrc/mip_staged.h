@@ -466,29 +466,50 @@ __host__ inline bool fast_norm_ok(float min_val, float max_val) {
 //
 // A lane asks for its epoch's windows over the box of all 64 rays, ~27 of them: 1-2% of the
 // march.  Asked by each ray for itself along its length the windows stop rays ~3% sooner but
-// cost 9% of the march.  Where opacity_windows says no, the volume's own bounds take the
-// windows' place (they stop few rays where noise reaches below min_val).
+// cost 9% of the march.  Where a frame does not ask (opacity_windows) the volume's own bounds take
+// the windows' place (they stop few rays where noise reaches far below min_val).
 __device__ __forceinline__ uint32_t opacity_shift(uint32_t n) {  // n > 0
     return n <= 64u ? 0u : 32u - (uint32_t)__builtin_clz((n - 1u) >> 6);
 }
 
-// Whether a frame's rays ask the windows: enough waves that ending some early ends the frame
-// early, rays close together (tiles: 8x8 pixel quarters; a frame of few has them far apart),
-// and a march long enough in voxels (nmax, the largest dimension) and samples.  us volume's
-// bounds / windows, alpha_pow 0.6, 800^2 frames unless stated:
-//   512^3 blobs, 896 steps: uint16 983 / 891, float 943 / 786; 200 steps: uint16 390 / 406,
-//   float 472 / 429; 256^3, 448 steps: uint16 443 / 389, uint8 442 / 406
-//   128^3, 200 steps: uint16 202 / 202, uint8 198 / 211; 200^2 of 512^3, 200 steps 180 / 254
-template <typename T>
-__host__ __device__ inline bool opacity_windows(uint32_t tiles, float nmax, uint32_t n) {
-    return tiles >= 2048u && nmax >= 160.0f &&
-           (std::is_same<T, float>::value || nmax <= 2.0f * (float)n);
+// The change of a ray's transparency, as an exponent, over n samples of voxel v (integral:
+// integer voxels): < 0 falls, > 0 grows
+__host__ inline float opacity_exponent(bool integral, const RayParams& p, float v, uint32_t n) {
+    const float a = (integral ? 0.1f : 1.0f) * p.alpha_pow * p.alpha_pow;
+    const float x = p.max_val != 0.0f ? (v - p.min_val) / (p.max_val - p.min_val) : v;
+    return a * (float)n * fminf(fmaxf(-x, -1.0f), integral ? 1.0f : 0.0f);
+}
+
+// Whether a frame's rays ask the windows, a few us a wave: enough waves that ending some early
+// ends the frame early, rays close together (tiles: 8x8 pixel quarters; a frame of few has them
+// far apart), a march long enough in voxels (nmax, the largest dimension) and samples, and
+// windows that can end rays which the volume's own bounds don't: below a ray's colour while it
+// is still transparent (need: k_ray_need's share), or where it turns opaque (fall: the exponent
+// over n samples of the mean voxel) among integer voxels far enough below min_val (grow: of the
+// least voxel) that the volume's bounds can't say so.  us volume's bounds / windows, alpha_pow
+// 0.6, 256^3, 200 steps, 800^2 frames unless stated:
+//   need .2, uint16 229 / 188; 512^3, 896 steps: uint16 983 / 891, float 943 / 786
+//   need .6, fall 0: 600^2 frames 149 / 157; 400^2 (2,500 quarters): need .6 126 / 137, .3 77 / 77
+//   alpha_pow 1, 448 steps, fall 22: grow 0, 600^2 33 / 40; grow 3, 175 / 57
+//   float, need .4, fall 59, 320 steps, 600^2 38 / 44; noise (need 1), alpha_pow 0.2, 109 / 121
+__host__ inline bool opacity_windows(bool integral, uint32_t tiles, int nmax, uint32_t n, float need,
+                                     float fall, float grow) {
+    if (tiles < 4096u || nmax < 160 || (integral && (uint32_t)nmax > 2u * n)) return false;
+    if (!(need < 0.5f || fall >= 2.0f)) return false;
+    return integral ? fall < 8.0f || grow > 1.0f : need < 0.9f && fall < 18.0f;
+}
+
+// The same for a batch, whose frames have no other stop test: wherever rays lose most of their
+// transparency.  us without / windows, six 400^2 frames of 256^3, 448 steps: uint16 textures 850 / 336
+// (fall 9), blobs 955 / 1014 (0.5), float blobs 1411 / 936 (6), sparse voxels 1040 / 1051 (0)
+__host__ inline bool opacity_windows_batch(bool integral, uint32_t tiles, int nmax, uint32_t n, float fall) {
+    return tiles >= 2048u && nmax >= 160 && (!integral || (uint32_t)nmax <= 2u * n) && fall >= 1.5f;
 }
 
 template <typename V>
 __device__ __forceinline__ float opacity_bounds(const V& vol, const Opacity& op, float px, float py,
                                                 float pz, float dx, float dy, float dz, uint32_t n,
-                                                uint32_t tiles) {
+                                                bool asks) {
     using T = typename V::value_type;
     constexpr bool kShort = !std::is_same<T, float>::value;
     const float inf = __builtin_inff();
@@ -513,7 +534,7 @@ __device__ __forceinline__ float opacity_bounds(const V& vol, const Opacity& op,
     };
     auto times = [](float g, float x) { return x > 0.0f ? g * x : 0.0f; };  // (not inf * 0)
     float H = 0.0f, G = 1.0f;
-    if (!opacity_windows<T>(tiles, fmaxf(vol.fnx, fmaxf(vol.fny, vol.fnz)), n)) {
+    if (!asks) {  // (uniform)
         if (!(vol.vmin <= vol.vmax)) return inf;  // a NaN voxel, or no bounds
         const float m = bound_margin<T>(vol.vmin, vol.vmax);
         normalised(vol.vmin - m, vol.vmax + m, (float)(n - min(lane * epoch, n)), H, G);
@@ -1025,7 +1046,7 @@ __device__ __forceinline__ void mip_staged_march(const PaddedVolume<T, POW2, WID
     };
     if constexpr (SKIP && OPAC)
         bound = opacity_bounds(vol, op, px, py, pz, dx, dy, dz, (uint32_t)(g_end - g_begin) * CH,
-                               4u * p.ntiles);
+                               p.asks != 0u);
     // per-wave slabs: the next box's rows are loaded into registers while this box is
     // sampled (when the next box fits and needs at most kPrefetchRows rows per lane); SKIP:
     // with its brick bounds

@@ -253,6 +253,7 @@ RayParams make_params(const spr_params& prm, int tile_map, int w, int h) {
     p.tile_map = tile_map == (int)kTileMapCostXcd ? kTileMapInterleaved : (uint32_t)tile_map;
     p.row_pad = 0;
     p.box16 = 1;
+    p.asks = 0;
     p.order = nullptr;
     p.gate = nullptr;
     return p;
@@ -408,7 +409,8 @@ hipError_t launch_pad(const VolSlot& vs, const void* src, int sz0, uint32_t bz0,
     return hipGetLastError();
 }
 
-// The share of the windows that a max projection has to sample: *sum is its rays', from 0
+// The share of the windows that a max projection has to sample and the mean voxel: sum[0] and (as a
+// float) sum[1] are its rays', from 0
 template <typename T>
 void launch_need(const VolSlot& vs, uint32_t* sum, hipStream_t s) {
     hipLaunchKernelGGL(k_ray_need<T>, dim3(kNeedRays * kNeedRays, 3), dim3(64), 0, s, (const T*)vs.d_pad,
@@ -566,9 +568,9 @@ hipError_t pad_volume(spr_ctx* c, const VolSlot& vs, const void* src, bool from_
 hipError_t pair_windows(spr_ctx* c, VolSlot& vs) {
     const uint32_t gx = vs.win[0], gy = vs.win[1], gz = vs.win[2];
     uint32_t *count = nullptr, needed = 0;
-    hipError_t e = hipMallocAsync((void**)&count, sizeof(*count), c->stream);
+    hipError_t e = hipMallocAsync((void**)&count, 2 * sizeof(*count), c->stream);
     if (e != hipSuccess) return e;
-    e = hipMemsetAsync(count, 0, sizeof(*count), c->stream);
+    e = hipMemsetAsync(count, 0, 2 * sizeof(*count), c->stream);
     if (e == hipSuccess) {
         const dim3 grid((gx * gy + 255u) / 256u, gz), block(256);
         uint32_t *blocks = (uint32_t*)vs.win_min(), *wmax = (uint32_t*)vs.win_max();
@@ -695,7 +697,8 @@ int fill_slot(spr_ctx* c, VolSlot& vs, const void* src, bool src_on_device, int 
             BrickKey* total = vs.d_bricks + nbricks;
             struct {
                 BrickKey keys;
-                uint32_t needed, pad;
+                uint32_t needed;
+                float means;
             } t{};
             if (e == hipSuccess) e = hipMemsetAsync(total, 0xFF, sizeof(BrickKey), c->stream);
             if (e == hipSuccess) e = hipMemsetAsync(total + 1, 0, sizeof(BrickKey), c->stream);
@@ -715,6 +718,7 @@ int fill_slot(spr_ctx* c, VolSlot& vs, const void* src, bool src_on_device, int 
             vs.vmin = dtype == SPR_DTYPE_F32 ? key_value<float>(k.kmin) : (float)k.kmin;
             vs.vmax = dtype == SPR_DTYPE_F32 ? key_value<float>(~k.nkmax) : (float)~k.nkmax;
             vs.need = need_of(t.needed);
+            vs.mean = t.means / (3.0f * kNeedRays * kNeedRays);
         } else if (e == hipSuccess) {
             e = pair_windows(c, vs);
         }
@@ -745,6 +749,7 @@ struct BatchKind {
     bool pow2 = true;
     int nmax = 1;
     float need = 0.0f;
+    float mean = 0.0f;  // largest mean voxel
 };
 
 // Converts the caller's jobs into device job records in out[0 .. n-1]; checks that every
@@ -770,6 +775,7 @@ int build_jobs_into(spr_ctx* c, const spr_job* jobs, int n, BatchJob* out, Batch
         kind->pow2 = kind->pow2 && slot_pow2(*vs);
         kind->nmax = std::max(kind->nmax, std::max(vs->nx, std::max(vs->ny, vs->nz)));
         kind->need = std::max(kind->need, vs->need);
+        kind->mean = std::max(kind->mean, vs->mean);
         BatchJob& b = out[i];
         b = BatchJob{};
         b.base = vs->d_pad;
@@ -818,16 +824,18 @@ bool batch_windows(const LaunchTuning& t, const spr_params& prm, const BatchKind
            windows_pay(prm.filter == SPR_FILTER_NEAREST, true, kind.need, kind.nmax, step, gx * gy);
 }
 
-bool opacity_asks(int dtype, uint32_t tiles, int nmax, int nouter) {
-    const uint32_t n = (uint32_t)(nouter + 1) * kLoopUnroll;
-    return dtype == SPR_DTYPE_F32 ? opacity_windows<float>(tiles, (float)nmax, n)
-                                  : opacity_windows<uint16_t>(tiles, (float)nmax, n);
+// Whether a batch's opacity frames of p's size and settings ask the windows
+bool opacity_asks(int dtype, const RayParams& p, int nmax, float mean) {
+    const bool integral = dtype != SPR_DTYPE_F32;
+    const uint32_t n = (uint32_t)(p.nouter + 1) * kLoopUnroll;
+    return opacity_windows_batch(integral, 4u * p.ntiles, nmax, n, -opacity_exponent(integral, p, mean, n));
 }
 
 // A batch's launch (g: the window grid's, mixed: one row of every frame's workgroups)
 hipError_t dispatch_batch(const LaunchTuning& t, const spr_params& prm, int dtype, bool pow2,
-                          const BatchPlan& plan, const BatchJob* d_jobs, const RayParams& p,
+                          const BatchPlan& plan, const BatchJob* d_jobs, RayParams p,
                           const BatchQueues& q, dim3 g, uint32_t* counters, hipStream_t s) {
+    p.asks = plan.stops ? 1u : 0u;
     const bool nearest = prm.filter == SPR_FILTER_NEAREST;
     if (plan.windows)
         return visit_launch(dtype, pow2, [&](auto L) {
@@ -852,7 +860,7 @@ BatchPlan uniform_plan(const LaunchTuning& t, const spr_params& prm, const Batch
                        const RayParams& p, uint32_t njobs) {
     const float step = (float)kind.nmax / (16.0f * (float)p.nouter);
     return BatchPlan{batch_windows(t, prm, kind, frame_groups(p), njobs, step),
-                     opacity_asks(kind.dtype, 4u * p.ntiles, kind.nmax, p.nouter), windows_group(step),
+                     opacity_asks(kind.dtype, p, kind.nmax, kind.mean), windows_group(step),
                      chunk_for(t, p.nouter, kind.nmax)};
 }
 
@@ -905,8 +913,9 @@ int graph_capture(spr_ctx* c, spr_batch_graph* bg, const BatchPlan& plan) {
 int graph_capture(spr_ctx* c, spr_batch_graph* bg, BatchKind kind) {
     const RayParams p = graph_params(bg);
     int rc = SPR_OK;
-    for (const float need : {0.0f, 1.0f}) {  // (windows_pay is monotonic in need)
-        kind.need = need;
+    for (const bool much : {false, true}) {  // (windows_pay and opacity_asks are monotonic in these)
+        kind.need = much ? 1.0f : 0.0f;
+        kind.mean = much ? __builtin_inff() : 0.0f;
         if (rc == SPR_OK)
             rc = graph_capture(c, bg, uniform_plan(bg->tune, bg->prm, kind, p, (uint32_t)bg->n));
     }
@@ -1523,7 +1532,13 @@ int spr_render_frames(spr_ctx* c, const spr_frame* frames, int n, float alpha_po
         ch = std::min(ch, chunk_for(c->tune, b.nouter, nmax));
         groups += 4u * tile_grid(kTileMapInterleaved, ntx, nty);
         step = std::max(step, (float)nmax / (16.0f * (float)b.nouter));
-        stops = stops || opacity_asks(kind.dtype, 4u * ntx * nty, nmax, b.nouter);
+        spr_params frame{};
+        frame.alpha_pow = alpha_pow;
+        frame.min_val = b.min_val;
+        frame.max_val = b.max_val;
+        RayParams rp = make_params(frame, c->tune.tile_map, (int)b.W, (int)b.H);
+        rp.nouter = b.nouter;
+        stops = stops || opacity_asks(kind.dtype, rp, nmax, slot_of(c, frames[i].slot)->mean);
     }
     q.mixed = 1;
     q.njobs = (uint32_t)n;
@@ -1817,6 +1832,7 @@ int spr_batch_graph_launch(spr_ctx* c, spr_batch_graph* bg, void* stream) {
                         "(spr_batch_graph_update or a new graph)", r.first);
         kind.nmax = std::max(kind.nmax, std::max(vs->nx, std::max(vs->ny, vs->nz)));
         kind.need = std::max(kind.need, vs->need);
+        kind.mean = std::max(kind.mean, vs->mean);
     }
     DeviceGuard g(c->device);
     hipStream_t s = stream ? (hipStream_t)stream : c->stream;

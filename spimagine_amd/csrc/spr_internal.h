@@ -41,6 +41,7 @@ struct VolSlot {
     uint32_t win[3] = {0, 0, 0};
     size_t win_bytes = 0;
     float need = 1.0f;  // share of the windows a max projection has to sample (k_ray_need)
+    float mean = 0.0f;  // mean voxel (of k_ray_need's rays)
     static size_t align256(size_t n) { return (n + 255) / 256 * 256; }
     void* win_max() const { return (char*)d_pad + align256(pad_bytes); }
     void* win_min() const { return (char*)win_max() + align256(win_bytes); }

@@ -192,7 +192,8 @@ static __global__ __launch_bounds__(256) void k_pair_windows(const uint32_t* __r
 
 // Share of the windows that a max projection has to sample, measured along kNeedRays x kNeedRays
 // rays parallel to each axis, between the voxels: the windows of a ray whose maximum exceeds the
-// ray's own (a pair's: in either channel).  One wave a ray; *sum: the rays' shares, 16 bits each.
+// ray's own (a pair's: in either channel).  One wave a ray; sum[0]: the rays' shares, 16 bits each;
+// sum[1], a float: the means of their samples (channel 0), which finite rays have.
 //
 // Windows alone do not tell: where few voxels are bright or noise is strong a ray seldom meets a
 // window's maximum.  Against three quarters of the best window of a column, which was counted
@@ -219,7 +220,7 @@ __global__ __launch_bounds__(64) void k_ray_need(const T* __restrict__ pad, int 
     const uint32_t ib = min(1u + (rb * n[b] + n[b] / 2u) / kNeedRays, n[b]),
                    ic = min(1u + (rc * n[c] + n[c] / 2u) / kNeedRays, n[c]);
     const T* at = pad + ib * stride[b] + ic * stride[c];
-    float top = 0.0f, top2 = 0.0f;
+    float top = 0.0f, top2 = 0.0f, mean = 0.0f;
     for (uint32_t k = lane; k <= n[a]; k += 64u) {
         float s = 0.0f, s2 = 0.0f;
 #pragma unroll
@@ -228,10 +229,12 @@ __global__ __launch_bounds__(64) void k_ray_need(const T* __restrict__ pad, int 
             s += v.x;
             s2 += v.y;
         }
+        mean += 0.125f * s;
         top = fmaxf(top, 0.125f * s);
         top2 = fmaxf(top2, 0.125f * s2);
     }
     for (int o = 32; o > 0; o >>= 1) {
+        mean += __shfl_xor(mean, o);
         top = fmaxf(top, __shfl_xor(top, o));
         top2 = fmaxf(top2, __shfl_xor(top2, o));
     }
@@ -242,7 +245,10 @@ __global__ __launch_bounds__(64) void k_ray_need(const T* __restrict__ pad, int 
         need += v.x > top || v.y > top2 ? 1u : 0u;
     }
     for (int o = 32; o > 0; o >>= 1) need += (uint32_t)__shfl_xor((int)need, o);
-    if (lane == 0u) atomicAdd(sum, (need << 16) / g[a]);
+    if (lane == 0u) {
+        atomicAdd(sum, (need << 16) / g[a]);
+        if (fabsf(mean) < __builtin_inff()) atomicAdd((float*)sum + 1, mean / (float)(n[a] + 1u));
+    }
 }
 
 }  // namespace spr

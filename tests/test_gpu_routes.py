@@ -43,12 +43,12 @@ def volume(torch, kind, dtype, shape):
     return (v if dtype == np.float32 else v.round()).to(kinds[dtype]).contiguous()
 
 
-def times(torch, s, ctx, go, chunks):
-    """The least time of each chunk setting (0: the default), taken in turn."""
+def times(torch, s, ctx, go, chunks, key="chunk"):
+    """The least time of each setting of a tuning key, taken in turn."""
     best = {k: 1e9 for k in chunks}
     for _ in range(7):
         for k in chunks:
-            ctx.set_tuning("chunk", k)
+            ctx.set_tuning(key, k)
             go()
             e = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
             e[0].record(s)
@@ -126,3 +126,61 @@ def test_default_march_is_not_slower(how, dtype, kind, shape, size, steps, n):
         how, np.dtype(dtype).name, kind, shape, size, steps, best[0], staged), flush=True)
     ctx.close()
     assert best[0] <= 1.2 * staged
+
+
+# (voxel type, volume, shape, frame size, steps, frames, alpha_pow, bound of the time against no test)
+OPACITY = [
+    # windows asked where they could not end a ray: too few waves, a batch's still transparent rays
+    (np.uint16, "noisy spots", (256, 256, 256), 400, 448, 1, .6, 1.07),
+    (np.uint16, "noisy spots", (256, 256, 256), 400, 200, 1, .6, 1.07),
+    (np.uint8, "noisy spots", (256, 256, 256), 400, 448, 6, .6, 1.07),
+    (np.uint16, "noisy spots", (192, 192, 192), 400, 200, 6, .2, 1.07),
+    # not asked, and the volume's own bounds end rays though voxels lie below min_val
+    (np.uint16, "noise", (160, 160, 160), 200, 200, 1, .6, 1.),
+    (np.uint8, "noise", (160, 160, 160), 600, 112, 1, .7, 1.),
+    # asked: rays turn opaque, and voxels lie too far below min_val for the volume's bounds
+    (np.uint16, "noise", (256, 256, 256), 800, 448, 1, .7, 1.),
+    (np.uint16, "grain", (176, 176, 176), 400, 320, 6, .6, 1.),
+    (np.float32, "grain", (176, 176, 176), 400, 320, 6, .6, 1.),
+]
+
+
+@pytest.mark.parametrize("dtype,kind,shape,size,steps,n,alpha_pow,bound", OPACITY)
+def test_opacity_rays_end_early_where_that_pays(dtype, kind, shape, size, steps, n, alpha_pow, bound):
+    import torch
+    ctx = _lib.Context(0)
+    vol = volume(torch, kind, dtype, shape)
+    torch.cuda.synchronize()
+    slot = ctx.volume_add(dev_ptr=vol.data_ptr(), dtype=dtype, shape=shape)
+    s = torch.cuda.Stream()
+    o = torch.zeros((n, 2, size, size), device="cuda")
+    jobs = []
+    for k in range(n):
+        M = np.dot(mat4_translate(0, 0, -3.2), mat4_rotation(.6 + .5 * k, .3, 1, -.2))
+        iP, iM = render_matrices(M, mat4_perspective(45, 1., .1, 10), shape[::-1])
+        p = _lib.make_params(iP, iM, min_val=.08 * TOP[dtype], max_val=.9 * TOP[dtype], max_steps=steps,
+                             alpha_pow=alpha_pow)
+        jobs.append((slot, list(p.inv_p), list(p.inv_m), o[k, 0].data_ptr(), o[k, 1].data_ptr()))
+    frame = (slot, p, _lib.METHOD_MAX_PROJECT, size, size, o[0, 0].data_ptr(), o[0, 1].data_ptr())
+    jobs = ctx.make_jobs(jobs)
+
+    def go():
+        if n == 1:
+            ctx.render_slot(*frame, stream=s.cuda_stream)
+        else:
+            ctx.render_batch(jobs, size, size, params=p, stream=s.cuda_stream)
+
+    outs = []
+    for skip in (0, 1):
+        ctx.set_tuning("skip", skip)
+        o.fill_(-1.)
+        torch.cuda.synchronize()
+        go()
+        s.synchronize()
+        outs.append(o.clone())
+    assert torch.equal(outs[0], outs[1])
+    best = times(torch, s, ctx, go, (0, 1), "skip")
+    print("opacity %s %s %s %d^2 %d steps, %d: %.0f us, without the test %.0f us" % (
+        np.dtype(dtype).name, kind, shape, size, steps, n, best[1], best[0]), flush=True)
+    ctx.close()
+    assert best[1] <= bound * best[0]
