@@ -72,7 +72,8 @@ def roofline(b_alg, kernel_ms, traffic):
     out = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
            "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
            "kernel_ms": round(kernel_ms, 4), "algorithmic_bytes": int(b_alg),
-           "achieved_is": "effective gather bandwidth (reference samples x 8 corners)"}
+           "achieved_is": "effective gather bandwidth (reference samples x 8 corners; most are "
+                          "shown not to matter and not taken, so it can pass the peak)"}
     if traffic:
         measured = traffic / (kernel_ms * 1e-3) / 1e9
         out["measured_hbm_GBps"] = round(measured, 1)
@@ -321,15 +322,15 @@ def skip_table(ctx, stream, frame, set_pose, samples, reps):
 
 
 def filter_table(ctx, stream, frame, set_pose, samples, reps):
-    """Per-pose frame times of the nearest filter (set_pose(k) selects it) staged in LDS
-    slabs (the context's slab_kb) and with every sample gathered from global memory
-    (slab_kb 0).  Restores slab_kb.  reps 0: no table (None)."""
+    """Per-pose frame times of the nearest filter (set_pose(k) selects it) by the march that
+    the context's tuning picks and with every sample gathered from global memory (slab_kb 0).
+    Restores slab_kb.  reps 0: no table (None)."""
     import torch
     if reps <= 0:
         return None
     keep = ctx.get_tuning("slab_kb")
     out = {}
-    for name, slab in (("staged", keep), ("global", 0)):
+    for name, slab in (("default", keep), ("global", 0)):
         ctx.set_tuning("slab_kb", slab)
         ms = []
         for k in range(len(samples)):

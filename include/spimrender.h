@@ -101,19 +101,22 @@ extern "C" {
                       4 (a 16x16 tile), 0 = default (1: faster at 1024^2 and 2048^2)
    SPR_TUNE_SKIP      1 = empty-space skipping and early ray termination by the volume's
                       bounds (default), 0 = off.  Every padded one-channel volume keeps the
-                      minimum and maximum of each 8x8x8 brick and of overlapping 8x8x8
-                      windows every 4 voxels (built on upload, 1/64 and 1/32 of its bytes
-                      for uint16 voxels; a channel pair the maxima of its windows).  With the
-                      other keys at their defaults, max projections of volumes whose windows
-                      leave enough to skip are gathered group by group, a group of 4, 2 or 1 samples only
-                      when its window exceeds the ray's running maximum, and the iso march
-                      samples a group only when its window reaches the other side of the
-                      iso value.  Otherwise, with the default per-wave slabs (slab_kb 19),
-                      the max projection skips a box whose bricks' maximum cannot exceed any
-                      of the wave's running maxima and the iso march a box whose bricks lie
-                      wholly on each marching ray's starting side.  The opacity mode stops a wave once transparency times the most that the
-                      windows ahead can hold, growth of the transparency included, is at most
-                      each ray's colour.  Results are bit-identical either way. */
+                      minimum and maximum of each 8x8x8 brick (8 bytes: 1/128 of a uint16
+                      volume) and of overlapping 8x8x8 windows every 4 voxels (1/32 of the
+                      volume), built on upload; a channel pair the maxima of its windows.
+                      With the other keys at their defaults, max projections of volumes whose
+                      windows leave enough to skip are gathered group by group, a group of 4,
+                      2 or 1 samples only when its window exceeds the ray's running maximum,
+                      and the iso march samples a group only when its window reaches the
+                      other side of the iso value.  Otherwise, with the default per-wave
+                      slabs (slab_kb 19), the max projection skips a box whose bricks'
+                      maximum cannot exceed any of the wave's running maxima and the iso
+                      march a box whose bricks lie wholly on each marching ray's starting
+                      side.  The opacity mode stops a wave once transparency times the most
+                      that is still to come is at most each ray's colour, growth of the
+                      transparency included: by the windows ahead where those end rays
+                      sooner, else by the volume's minimum and maximum.  Results are
+                      bit-identical either way. */
 #define SPR_TUNE_TILE_MAP 0
 #define SPR_TUNE_SLAB_KB 1
 #define SPR_TUNE_STAGING 2

@@ -421,7 +421,7 @@ __global__ __launch_bounds__(64 * kWinSegments, (kWinWaves<T, GS, FILT>)) void k
 // The frames of a batch (many volumes x poses, or frames of their own sizes and settings)
 // the same way, one launch.  Uniform batches: grid.y = job.  Mixed ones: job k's first
 // workgroup in jobs[k].first[0].  A workgroup per quarter instead of persistent ones
-// claiming tiles: the workgroups are short and hold 12 KB of LDS, so the next ones fill in.
+// claiming tiles: the workgroups are short and hold 10 KB of LDS, so the next ones fill in.
 // gates: nullptr, or one device word per frame (0: the frame is left untouched).
 template <typename T, bool POW2, int GS, int FILT>
 __global__ __launch_bounds__(64 * kWinSegments, (kWinWaves<T, GS, FILT>)) void k_mip_windows_batch(
