@@ -120,7 +120,7 @@ def test_volume_above_4_gib_staged_and_by_windows():
     sw, sl = [c.volume_add(dev_ptr=v16.data_ptr(), dtype=np.uint16, shape=shape) for c in (wide, lin)]
     del v16
     s = torch.cuda.Stream()
-    W, H = 416, 400  # 2,600 quarters: opacity frames ask the windows
+    W, H = 528, 512  # 4,224 quarters: opacity frames ask the windows
 
     def mip(ctx, slot, p):
         o = torch.full((2, H, W), -7., device="cuda")
