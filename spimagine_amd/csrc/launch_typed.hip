@@ -371,9 +371,9 @@ hipError_t TypedLaunch<T, P2>::max_project(const LaunchTuning& t, const VolSlot&
     // with the default tuning, frames that gain by it are gathered group by group
     const float step = (float)nmax / (16.0f * (float)p.nouter);
     if (!opac && skip && windows_tuning(t) &&
-        windows_pay(nearest, false, vs.need, nmax, step, 4u * p.ntiles) &&
         4u * tile_grid(kTileMapInterleaved, p.ntx, p.nty) <= kWinMaxGroups &&
-        (vs.layout == SPR_LAYOUT_PADDED || (vs.pad_wide && !nearest))) {
+        (vs.layout == SPR_LAYOUT_PADDED || (vs.pad_wide && !nearest)) &&
+        windows_pay(nearest, vs.need, nmax, step, p)) {
         const int gs = windows_group(step);
         if (vs.pad_wide && !nearest)
             launch_windows<0>(gs, padded_volume<T, P2, true>(vs), p, out, alpha, s);
@@ -622,7 +622,7 @@ hipError_t launch_pair(const LaunchTuning& t, const VolSlot& vs, RayParams p, fl
     const int ch = chunk_for(t, p.nouter, nmax);
     const float step = (float)nmax / (16.0f * (float)p.nouter);
     if (t.skip != 0 && vs.win_bytes != 0 && windows_tuning(t) &&
-        windows_pay(false, false, vs.need, nmax, step, 4u * p.ntiles) &&
+        windows_pay(false, vs.need, nmax, step, p) &&
         4u * tile_grid(kTileMapInterleaved, p.ntx, p.nty) <= kWinMaxGroups) {
         launch_windows<0>(windows_group(step), padded_volume<U16Pair, P2>(vs), p, out, alpha, s);
         return hipGetLastError();

@@ -72,6 +72,7 @@ struct spr_batch_graph {
     hipStream_t last_stream = nullptr;
     int dtype = -1;
     bool pow2 = false;  // the captured kernel's texel rule (every volume a power of two)
+    float hits = 1.0f;  // share of the jobs' rays that hit (hit_share)
     // (slot, generation) of every job: a launch after any of these slots was refilled or
     // released is refused
     std::vector<std::pair<int, uint32_t>> refs;
@@ -750,6 +751,30 @@ struct BatchKind {
     int nmax = 1;
     float need = 0.0f;
     float mean = 0.0f;  // largest mean voxel
+    // share of the rays that hit (hit_share): of the jobs if given, else as stated; box: all
+    // jobs' (nullptr: each has its own)
+    float hits = 1.0f;
+    const BatchJob* jobs = nullptr;
+    int njobs = 0;
+    const float* box = nullptr;
+    void hits_of(const std::vector<BatchJob>& j, const float* b) {
+        jobs = j.data();
+        njobs = (int)j.size();
+        box = b;
+    }
+    // (of up to 8 of the jobs, by their pixels)
+    float share() const {
+        if (!jobs) return hits;
+        const int every = (njobs + 7) / 8;
+        float hit = 0.0f, all = 0.0f;
+        for (int i = 0; i < njobs; i += every) {
+            const BatchJob& j = jobs[i];
+            const float pixels = box ? 1.0f : (float)j.W * (float)j.H;
+            hit += pixels * hit_share(j.invP, j.invM, box ? box : j.box);
+            all += pixels;
+        }
+        return hit / all;
+    }
 };
 
 // Converts the caller's jobs into device job records in out[0 .. n-1]; checks that every
@@ -819,9 +844,11 @@ BatchQueues make_queues(const RayParams& p, int n) {
 // step in voxels)
 bool batch_windows(const LaunchTuning& t, const spr_params& prm, const BatchKind& kind, uint64_t gx,
                    uint64_t gy, float step) {
-    return prm.alpha_pow == 0.0f && windows_tuning(t) && gx <= kWinMaxGroups &&
-           gy <= 65535u &&
-           windows_pay(prm.filter == SPR_FILTER_NEAREST, true, kind.need, kind.nmax, step, gx * gy);
+    if (prm.alpha_pow != 0.0f || !windows_tuning(t) || gx > kWinMaxGroups || gy > 65535u) return false;
+    const bool nearest = prm.filter == SPR_FILTER_NEAREST;
+    const float groups = (float)(gx * gy);
+    return windows_pay(nearest, true, kind.need, kind.nmax, step, groups) ||
+           windows_pay(nearest, true, kind.need, kind.nmax, step, groups * kind.share());
 }
 
 // Whether a batch's opacity frames of p's size and settings ask the windows
@@ -913,8 +940,10 @@ int graph_capture(spr_ctx* c, spr_batch_graph* bg, const BatchPlan& plan) {
 int graph_capture(spr_ctx* c, spr_batch_graph* bg, BatchKind kind) {
     const RayParams p = graph_params(bg);
     int rc = SPR_OK;
+    bg->hits = kind.share();
+    kind.jobs = nullptr;
     for (const bool much : {false, true}) {  // (windows_pay and opacity_asks are monotonic in these)
-        kind.need = much ? 1.0f : 0.0f;
+        kind.need = kind.hits = much ? 1.0f : 0.0f;
         kind.mean = much ? __builtin_inff() : 0.0f;
         if (rc == SPR_OK)
             rc = graph_capture(c, bg, uniform_plan(bg->tune, bg->prm, kind, p, (uint32_t)bg->n));
@@ -1441,6 +1470,7 @@ int spr_render_batch(spr_ctx* c, const spr_params* params, const spr_job* jobs, 
     BatchKind kind;
     rc = build_jobs(c, jobs, n, host, &kind);
     if (rc) return rc;
+    kind.hits_of(host, prm.box);
     DeviceGuard g(c->device);
     hipStream_t s = stream ? (hipStream_t)stream : c->stream;
     // per-call job table and queue counters from the stream-ordered allocator, so batches
@@ -1514,6 +1544,7 @@ int spr_render_frames(spr_ctx* c, const spr_frame* frames, int n, float alpha_po
     BatchKind kind;
     int rc = frames_to_jobs(c, frames, n, host, &kind);
     if (rc) return rc;
+    kind.hits_of(host, nullptr);
     // each frame's first item in each queue; the box length follows the frame with the
     // longest ray step
     BatchQueues q{};
@@ -1663,6 +1694,9 @@ int spr_render_batch_noalloc(spr_ctx* c, const spr_params* params, const spr_job
     BatchKind kind;
     rc = build_jobs_into(c, jobs, n, g_noalloc_jobs, &kind);
     if (rc) return rc;
+    kind.jobs = g_noalloc_jobs;
+    kind.njobs = n;
+    kind.box = prm.box;
     DeviceGuard g(c->device);
     hipStream_t s = stream ? (hipStream_t)stream : c->stream;
     uint32_t* d_counters = (uint32_t*)c->d_scratch;  // cleared by the launch's reset kernel
@@ -1786,6 +1820,7 @@ int spr_batch_graph_create(spr_ctx* c, const spr_job* jobs, int n, int w, int h,
         hipSuccess)
         return cleanup(fail(c, SPR_ERR_HIP, "job upload failed"));
     rc = check_parts(c, c->params, 1);
+    kind.hits_of(host, bg->prm.box);
     if (rc == SPR_OK) rc = graph_capture(c, bg, kind);
     if (rc) return cleanup(rc);
     *out = bg;
@@ -1809,6 +1844,7 @@ int spr_batch_graph_update(spr_ctx* c, spr_batch_graph* bg, const spr_job* jobs,
                     "the captured batch's volumes %s power-of-two dimensions and the new ones %s "
                     "(capture a new graph)", bg->pow2 ? "all have" : "do not all have",
                     kind.pow2 ? "do" : "do not");
+    kind.hits_of(host, bg->prm.box);
     DeviceGuard g(c->device);
     rc = graph_capture(c, bg, kind);
     if (rc) return rc;
@@ -1824,6 +1860,7 @@ int spr_batch_graph_launch(spr_ctx* c, spr_batch_graph* bg, void* stream) {
     if (!bg) return fail(c, SPR_ERR_INVALID_ARG, "NULL graph");
     BatchKind kind;  // of the volumes as they are now
     kind.dtype = bg->dtype;
+    kind.hits = bg->hits;
     for (const auto& r : bg->refs) {
         const VolSlot* vs = slot_of(c, r.first);
         if (!vs || vs->generation != r.second)
