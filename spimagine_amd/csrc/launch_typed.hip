@@ -361,9 +361,15 @@ hipError_t TypedLaunch<T, P2>::max_project(const LaunchTuning& t, const VolSlot&
     constexpr bool kInt = std::is_integral<T>::value;
     const uint32_t samples = (uint32_t)(p.nouter + 1) * kLoopUnroll;
     const float grow = opacity_exponent(kInt, p, vs.vmin, samples);
-    if (opac)
-        p.asks = opacity_windows(kInt, 4u * p.ntiles, nmax, samples, vs.need,
-                                 -opacity_exponent(kInt, p, vs.mean, samples), grow);
+    if (opac) {
+        const float fall = -opacity_exponent(kInt, p, vs.mean, samples);
+        // (also in small frames where rays turn opaque and the volume's bounds never say so: 200x536x482
+        // uint16 textures, 397x546, 752 steps, 1,518 quarters hit 627 us without, 102 with; 2-1.1 times
+        // longer with fewer than 200 hit)
+        p.asks = opacity_windows(kInt, 4u * p.ntiles, nmax, samples, vs.need, fall, grow) ||
+                 (grow > 1.0f && fall >= 4.0f &&
+                  4.0f * (float)p.ntiles * hit_share(p.invP, p.invM, p.box) >= 200.0f);
+    }
     const bool stops = p.asks != 0u || !(grow > 1.0f);
     if (opac && !stops) skip = false;
     // the plain max projection's box lengths (chunk 0: from the ray step)
