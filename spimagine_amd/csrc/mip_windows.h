@@ -195,7 +195,8 @@ __host__ inline int windows_group(float step) {
 __host__ inline bool windows_pay(bool nearest, bool batch, float need, int nmax, float step,
                                  float hits) {
     if (hits < (nearest ? (batch ? 8000.0f : nmax >= 190 ? 6000.0f : 1500.0f)
-                        : (batch ? 1500.0f : step >= 2.0f ? 3000.0f : 700.0f)))
+                : batch ? 1500.0f
+                : need < 0.9f ? (step >= 2.0f ? 3000.0f : 700.0f) : (step >= 2.0f ? 1500.0f : 500.0f)))
         return true;
     if (hits < (batch ? (nearest ? 12000.0f : 6000.0f) : 1000.0f) && need < (batch ? 0.7f : 0.6f))
         return true;
@@ -499,27 +500,27 @@ __global__ __launch_bounds__(64 * kWinSegments, (kWinWaves<T, GS, FILT>)) void k
 //
 // Bound by VALU (65% busy; address units 40%): ~5 instructions a sample in windows on one
 // side, the rest in groups near surfaces, their exact positions and the finish.  512^3
-// uint16 -> 1024^2, 896 steps: frame 446 us (487 with runs of groups a wave and four waves a SIMD,
-// 511 with a lane taking a whole group; march of the frame 412 us before that, 828 us staged
-// with 8^3 brick tests of a wave's box).
+// uint16 -> 1024^2, 896 steps: frame 467 us (487 with runs of groups a wave, 511
+// with a lane taking a whole group; march of the frame 412 us before that, 828 us staged with 8^3
+// brick tests of a wave's box).
 struct IsoWindowShared {
     float4 item[kWinSegments][128];  // position; w's bits: ray | side << 6 | first sample << 7
     SharedRays rays;
     uint64_t above;    // the rays that start above the iso value
     uint32_t hit[64];  // the rays' least crossing sample (~0: none)
 };
-// Waves per SIMD that the registers are held to: five (96), but for groups of four float samples,
-// which would spill 16.  The finish of a ray is one wave's work, so the workgroups resident count:
-// left alone uint8 frames took 139 registers.  us left alone / four / five, 1200^2 frames: 128^3
-// white noise, 112 steps, uint8 550 / 451 / 450, uint16 475 / 483 / 470; 512x512x256 blobs, 768 steps, uint8
-// 561 / 545 / 520, uint16 535 / 524 / 513.
-template <typename T, int GS>
-constexpr int kIsoWaves = std::is_same<T, float>::value && GS == 4 ? 4 : 5;
+// Waves per SIMD that the registers are held to (1: none).  The finish of a ray is one wave's work,
+// so the workgroups resident count: left alone trilinear uint8 frames take 139 registers (1200^2
+// frames of 128^3 white noise, 112 steps, 550 us, held to five 450; 512x512x256 blobs, 768 steps 561 /
+// 520).  The others take 100 to 112 and gain nothing on average (300 frames of 48 to 1,024 voxels an
+// axis drawn at random 1.7% slower held to five, those of few rays 2%).
+template <typename T, int FILT>
+constexpr int kIsoWaves = std::is_same<T, uint8_t>::value && FILT == 0 ? 5 : 1;
 constexpr uint32_t kIsoAnchor = 900;  // samples that a lookup may lie past an exact position
 constexpr int kIsoWindowMaxSteps = 1 << 24;
 
 template <typename T, bool POW2, int GS, bool WIDE, int FILT>
-__global__ __launch_bounds__(64 * kWinSegments, (kIsoWaves<T, GS>)) void k_iso_windows(
+__global__ __launch_bounds__(64 * kWinSegments, (kIsoWaves<T, FILT>)) void k_iso_windows(
     PaddedVolume<T, POW2, WIDE> vol, RayParams p, float* __restrict__ out, float* __restrict__ alpha,
     float* __restrict__ depth, float* __restrict__ normals) {
     using PV = PaddedVolume<T, POW2, WIDE>;
